@@ -475,6 +475,18 @@ int supa_amd_softmax_backward(const void* grad, const void* output, int32_t gy_d
                               void* grad_in, int32_t gin_dtype, int64_t rows, int64_t cols,
                               void* stream);
 
+/* log_softmax (log != 0) or softmax over the middle dim of a contiguous
+ * [outer, cols, inner] tensor (inner > 1: the class dim of [N, C, H, W]
+ * logits), forward and backward; dtypes, special values and the formulas as
+ * for the row forms above.  The output may be the input.  SUPA_AMD_ELAYOUT
+ * when outer * inner or cols reaches 2^31.  Replaces the same ops over a dim
+ * that is not the last (upstream SoftMax.cu's spatial kernels). */
+int supa_amd_softmax_dim_forward(int log, const void* in, int32_t in_dtype, void* out, int32_t out_dtype,
+                                 int64_t outer, int64_t cols, int64_t inner, void* stream);
+int supa_amd_softmax_dim_backward(int log, const void* grad, const void* output, int32_t gy_dtype,
+                                  void* grad_in, int32_t gin_dtype, int64_t outer, int64_t cols, int64_t inner,
+                                  void* stream);
+
 /* ------------------------------------------------------------ nll_loss */
 
 /* nll_loss over logp [n, c] (contiguous, dtype f32/bf16/f16/f64), int64

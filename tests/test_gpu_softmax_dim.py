@@ -1,0 +1,88 @@
+"""log_softmax and softmax over a dim that is not the last one (the spatial
+kernels): class counts around the edges of each split of the classes over
+class groups, planes of every remainder of the vector, special values, and
+the output written over the input."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import bf16_ulp_dist
+
+pytestmark = pytest.mark.gpu
+
+LSM_BWD = torch.ops.aten._log_softmax_backward_data
+SM_BWD = torch.ops.aten._softmax_backward_data
+
+
+def seeded(shape, seed, scale=1.0, dtype=torch.float32):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(shape, generator=g) * scale).to(dtype)
+
+
+def rows_of(t):
+    """[outer, cols, inner] -> [outer * inner, cols] float32."""
+    return np.ascontiguousarray(np.moveaxis(t.float().numpy(), 1, 2)).reshape(-1, t.shape[1])
+
+
+def planes_of(a, shape):
+    return np.moveaxis(a.reshape(shape[0], shape[2], shape[1]), 2, 1)
+
+
+def check(got, ref, dtype):
+    got = got.cpu()
+    if dtype == torch.float32:
+        np.testing.assert_allclose(got.numpy(), ref, rtol=1e-5, atol=1e-6)
+    else:  # one rounding to the storage type of a float32 value
+        r = torch.from_numpy(np.ascontiguousarray(ref)).to(dtype)
+        a, b = (v.view(torch.int16).numpy().view(np.uint16) for v in (got.contiguous(), r))
+        assert bf16_ulp_dist(a, b).max() <= 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(3, 1, 2), (2, 2, 3), (2, 7, 5), (3, 8, 64), (2, 9, 257), (5, 19, 1030), (2, 32, 33),
+                                   (2, 33, 12), (1, 128, 71), (2, 129, 9), (2, 256, 15), (2, 257, 11), (2, 300, 8201),
+                                   (70, 21, 4)])
+def test_spatial_softmax_matches_oracle(shape, dtype, no_fallback):
+    x = seeded(shape, 1, 2.0, dtype)
+    g = seeded(shape, 2, 1.0, dtype)
+    dx, dg = x.to("supa"), g.to("supa")
+    for log, fwd, bwd, ofwd, obwd in ((True, torch.log_softmax, LSM_BWD, O.log_softmax, O.log_softmax_backward),
+                                      (False, torch.softmax, SM_BWD, O.softmax, O.softmax_backward)):
+        y = fwd(dx, 1)
+        assert y.is_contiguous()
+        check(y, planes_of(ofwd(rows_of(x)), shape), dtype)
+        gi = bwd(dg, y, 1, dtype)
+        check(gi, planes_of(obwd(rows_of(g), rows_of(y.cpu())), shape), dtype)
+
+
+@pytest.mark.parametrize("shape", [(2, 19, 37), (2, 300, 4101), (2, 5, 3)])
+def test_spatial_softmax_over_its_input(shape, no_fallback):
+    x, g = seeded(shape, 3, 2.0), seeded(shape, 4)
+    want = torch.log_softmax(x.to("supa"), 1)
+    dx = x.to("supa")
+    torch.ops.aten._log_softmax.out(dx, 1, False, out=dx)
+    assert torch.equal(dx.cpu(), want.cpu())
+    gi = LSM_BWD(g.to("supa"), want, 1, torch.float32)
+    dg = g.to("supa")
+    LSM_BWD.out(dg, want, 1, torch.float32, out=dg)
+    assert torch.equal(dg.cpu(), gi.cpu())
+
+
+def test_spatial_softmax_layouts_and_special_values(no_fallback):
+    x = seeded((2, 5, 6, 7), 5, 2.0)
+    x[0, 1, 0, 0] = float("nan")
+    x[0, 2, 0, 1] = float("inf")
+    x[0, :, 0, 2] = -float("inf")
+    x[1, 3, 2, 3] = -float("inf")
+    for f in (torch.log_softmax, torch.softmax):
+        want = f(x, 1)
+        for dx in (x.to("supa"), x.to("supa").to(memory_format=torch.channels_last),
+                   x.transpose(2, 3).contiguous().to("supa").transpose(2, 3)):
+            got = f(dx, 1).cpu()
+            assert torch.equal(torch.isnan(got), torch.isnan(want))
+            np.testing.assert_allclose(got.numpy(), want.numpy(), rtol=1e-5, atol=1e-6)
+    h = torch._log_softmax(seeded((2, 5, 9), 6, 2.0, torch.bfloat16).to("supa"), 1, True)
+    assert h.dtype == torch.float32
+    np.testing.assert_allclose(h.cpu().numpy(), torch.log_softmax(seeded((2, 5, 9), 6, 2.0, torch.bfloat16).float(), 1),
+                               rtol=1e-5, atol=1e-6)
