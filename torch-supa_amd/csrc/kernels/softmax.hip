@@ -1,27 +1,28 @@
 // log_softmax and softmax, forward and backward, over the last dim of a
 // contiguous [rows, cols] tensor.
 //
-// Main path (16-byte aligned rows of up to 1024 threads x VPT vectors): one
-// 1024-thread workgroup per row holds the whole row in registers, so the
-// forward reads the row once and writes it once, and the backward reads grad
-// and output once each and writes once -- the HBM minimum for these aten ops.
-// Row statistics: per-thread partials, a 64-lane butterfly inside each
-// wavefront, then the 16 wavefront results through LDS (the forward combines
-// (max, sum) pairs in one exchange and walks rows with a persistent grid).  exp() of the row
-// statistics is the hardware base-2 exponential of (x - max) * log2 e: the
-// row maximum's term is exactly 1, as upstream's exp(x - max) makes it (a
-// pre-scaled x * log2 e - max * log2 e leaves max's term 1 +- 2^-18 at
-// |max| near 60, and a row with one dominant logit then gets a log-probability
-// of -1.7e-6 where upstream gives 0); the row results are rounded to bf16/f16
-// (or kept in f32) exactly once.
+// A row is read once and written once (the HBM minimum of these aten ops)
+// wherever it fits the registers of the threads that share it, by its length
+// in 16-byte vectors:
+//   up to 512     a sub-wavefront of 16 lanes or a wavefront (k_row_fwd,
+//                 k_row_bwd): statistics by shuffles alone;
+//   up to 2560    (backward 2048) a workgroup of 256 to 1024 threads, the
+//                 same kernels with one LDS exchange;
+//   2 to 32 parts of that: split over K workgroups of 512 threads that
+//                 exchange row partials through a small per-stream buffer, so
+//                 four parts share a CU (the section below);
+//   otherwise     (split rows switched off, under graph capture, or writing
+//                 over the input) aligned rows of up to 16384 vectors in one
+//                 1024-thread workgroup, the rest streaming twice.
+// Rows of any length and alignment move in 16-byte vectors at element
+// alignment (unaligned.h); the last cols mod V elements go one to a thread.
 //
-// Split rows (rows of 2 to 32 parts of 2048 or 2560 vectors): K workgroups
-// of 512 threads share a row, exchanging row partials through a small
-// per-stream buffer, so the same single pass runs with four parts per CU
-// (the section below).
-//
-// Fallback (any cols, any alignment): one 256-thread workgroup per row,
-// online max/sum in a first pass over memory, the output in a second pass.
+// exp() of the row statistics is the hardware base-2 exponential of
+// (x - max) * log2 e: the row maximum's term is exactly 1, as upstream's
+// exp(x - max) makes it (a pre-scaled x * log2 e - max * log2 e leaves max's
+// term 1 +- 2^-18 at |max| near 60, and a row with one dominant logit then
+// gets a log-probability of -1.7e-6 where upstream gives 0); the row results
+// are rounded to bf16/f16 (or kept in f32) exactly once.
 //
 // Replaces _log_softmax.out (NF:3752), _log_softmax_backward_data.out
 // (NF:3763), _softmax.out and _softmax_backward_data.out, upstream SoftMax.cu /
@@ -32,19 +33,11 @@
 #include <mutex>
 
 #include "softmax_common.h"
+#include "unaligned.h"
 
 namespace sa {
 
 constexpr int kRowBlock = 1024;
-// NaN-propagating max (a NaN anywhere in the row makes the row NaN, as the
-// upstream kernels' results are).
-__device__ __forceinline__ float nmax(float a, float b) { return (a != a || b != b) ? __builtin_nanf("") : fmaxf(a, b); }
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = nmax(v, __shfl_xor(v, off, 64));
-  return v;
-}
 template <typename ACC>
 __device__ __forceinline__ ACC wave_sum(ACC v) {
 #pragma unroll
@@ -54,18 +47,6 @@ __device__ __forceinline__ ACC wave_sum(ACC v) {
 
 // Block-wide reductions returning the result to every thread.  `lds` holds
 // one slot per wavefront; NW = blockDim / 64.
-template <int NW>
-__device__ __forceinline__ float block_max_all(float v, float* lds) {
-  v = wave_max(v);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) lds[wave] = v;
-  __syncthreads();
-  float r = lds[0];
-#pragma unroll
-  for (int w = 1; w < NW; ++w) r = nmax(r, lds[w]);
-  return r;
-}
 template <int NW>
 __device__ __forceinline__ float block_sum_all(float v, float* lds) {
   v = wave_sum(v);
@@ -90,14 +71,6 @@ __device__ __forceinline__ float block_sum_all(float v, float* lds) {
 // NaN, as in the upstream kernels.
 constexpr int kLsmGrid = 512;  // 2 workgroups per CU on MI355X's 256 CUs
 
-// (m, s) (+) (m2, s2); a pair with m = -inf has s = 0 and drops out.
-__device__ __forceinline__ void lse_combine(float& m, float& s, float m2, float s2) {
-  const float M = fmaxf(m, m2);
-  if (M != -__builtin_inff())
-    s = s * __builtin_amdgcn_exp2f((m - M) * kLog2e) + s2 * __builtin_amdgcn_exp2f((m2 - M) * kLog2e);
-  m = M;
-}
-
 // (max, sum of exp) pairs of `width` lanes (a power of two; lanes w apart in
 // the XOR pattern hold the other pairs) combined: a max butterfly, one
 // rescale per lane to that max, and a sum butterfly -- one exponential per
@@ -114,6 +87,215 @@ __device__ __forceinline__ void lanes_lse(float& m, float& s) {
   m = M;
 }
 
+// ------------------------------------------------- rows in registers
+// G threads share a row: 16 or 64 lanes of a wavefront (a 256-thread workgroup
+// then holds 256 / G rows) or a workgroup of G = 256 or 512.  Thread l holds
+// vectors l, l + G, ... (NV of them) and, where cols is no multiple of the
+// vector, element nvec V + l of the rest as a float.  VW = 1: rows of up to
+// G elements, one to a lane.
+//
+// A 1024-thread workgroup per row, as longer rows take, left most of its
+// threads without a vector here; rows of odd length took a 256-thread
+// workgroup of scalar loads and three passes.  Measured on MI355X, us before
+// -> after, forward / backward: bf16 [1048576, 10] 830 -> 40 / 449 -> 39,
+// [262144, 64] 1136 -> 20 / 674 -> 22, [65536, 1024] 292 -> 42 (6.3 TB/s) /
+// 201 -> 64 (6.3 TB/s), [32768, 1659] 105 -> 40 / 139 -> 60, [16384, 4096]
+// 89 -> 45 / 79 -> 68, [8192, 10000] 67 -> 56; float32 [65536, 1000] 289 ->
+// 96 / 268 -> 149.
+template <int G> constexpr int row_block() { return G <= 64 ? 256 : G; }
+
+// This thread's row and place in it; false past the last row.
+template <int G>
+__device__ __forceinline__ bool row_place(int64_t rows, int64_t& row, int& l) {
+  l = threadIdx.x & (G - 1);
+  row = G <= 64 ? (int64_t)blockIdx.x * (256 / (G <= 64 ? G : 256)) + threadIdx.x / G : (int64_t)blockIdx.x;
+  return row < rows;
+}
+
+template <typename T, int VW, int G, int NV>
+__device__ __forceinline__ void row_load(uint4 (&x)[NV], const T* src, int l, int nvec) {
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (l + j * G < nvec) {
+      if constexpr (VW == 1) x[j].x = __float_as_uint((float)to_arith(src[l + j * G]));
+      else x[j] = ld_any_stream(src + (int64_t)(l + j * G) * VW);
+    }
+}
+template <typename T, int VW>
+__device__ __forceinline__ float row_elem(const uint4& w, int k) {
+  if constexpr (VW == 1) return __uint_as_float(w.x);
+  else return elem_f<T>(w, k);
+}
+template <typename TO, int VW>
+__device__ __forceinline__ void row_store(TO* p, const float (&f)[VW]) {
+  if constexpr (VW == 1) p[0] = from_arith<TO>(f[0]);
+  else store_any<TO, VW>(p, f);
+}
+
+// Values of the G threads of a row combined; every thread ends with the total.
+template <int G>
+__device__ __forceinline__ void row_lse(float& m, float& s) {
+  lanes_lse<(G < 64 ? G : 64)>(m, s);
+  if constexpr (G > 64) {
+    __shared__ float lds_m[G / 64], lds_s[G / 64];
+    const int wave = threadIdx.x >> 6, i = threadIdx.x & 15;
+    if ((threadIdx.x & 63) == 0) {
+      lds_m[wave] = m;
+      lds_s[wave] = s;
+    }
+    __syncthreads();
+    m = i < G / 64 ? lds_m[i] : -__builtin_inff();
+    s = i < G / 64 ? lds_s[i] : 0.0f;
+    lanes_lse<16>(m, s);
+  }
+}
+template <int G>
+__device__ __forceinline__ float row_sum(float s) {
+#pragma unroll
+  for (int off = (G < 64 ? G : 64) / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if constexpr (G > 64) {
+    __shared__ float lds[G / 64];
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+    __syncthreads();
+    const int i = threadIdx.x & 15;
+    s = i < G / 64 ? lds[i] : 0.0f;
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  }
+  return s;
+}
+
+template <typename TI, typename TO, int VW, int G, int NV, bool LOG>
+__global__ void __launch_bounds__(row_block<G>())
+k_row_fwd(const TI* __restrict__ in, TO* __restrict__ out, int64_t rows, int cols) {
+  int64_t row;
+  int l;
+  if (!row_place<G>(rows, row, l)) return;
+  const TI* src = in + row * cols;
+  const int nvec = cols / VW, rest = cols - nvec * VW;
+  uint4 x[NV];
+  row_load<TI, VW, G, NV>(x, src, l, nvec);
+  float xt = -__builtin_inff();  // the identity: adds exp(-inf) = 0
+  if (VW > 1 && l < rest) xt = (float)to_arith(src[nvec * VW + l]);
+  float m = xt;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (l + j * G < nvec) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) m = fmaxf(m, row_elem<TI, VW>(x[j], k));
+    }
+  const float mb = m == -__builtin_inff() ? 0.0f : m;  // all -inf: keep exp arguments finite
+  if constexpr (VW > 1) opaque<NV>(x);
+  float s = VW > 1 ? __builtin_amdgcn_exp2f((xt - mb) * kLog2e) : 0.0f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (l + j * G < nvec) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) s += __builtin_amdgcn_exp2f((row_elem<TI, VW>(x[j], k) - mb) * kLog2e);
+    }
+  row_lse<G>(m, s);
+  // log: (x - M) - log S;  softmax: e^(x - M) / S (an all -inf row gives
+  // 0 * inf = NaN, as upstream)
+  const float a = LOG ? m : (m == -__builtin_inff() ? 0.0f : m);
+  const float b = LOG ? sa_logf(s) : 1.0f / s;
+  auto res = [&](float v) {
+    if constexpr (LOG) return (v - a) - b;
+    else return __builtin_amdgcn_exp2f((v - a) * kLog2e) * b;
+  };
+  if constexpr (VW > 1) opaque<NV>(x);
+  TO* dst = out + row * cols;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (l + j * G < nvec) {
+      float f[VW];
+#pragma unroll
+      for (int k = 0; k < VW; ++k) f[k] = res(row_elem<TI, VW>(x[j], k));
+      row_store<TO, VW>(dst + (int64_t)(l + j * G) * VW, f);
+    }
+  if (VW > 1 && l < rest) dst[nvec * VW + l] = from_arith<TO>(res(xt));
+}
+
+// LOG: gi = g - exp(y) sum(g);  softmax: gi = y (g - sum(g y)).
+template <typename TG, typename TO, int VW, int G, int NV, bool LOG>
+__global__ void __launch_bounds__(row_block<G>())
+k_row_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restrict__ gin, int64_t rows, int cols) {
+  int64_t row;
+  int l;
+  if (!row_place<G>(rows, row, l)) return;
+  const TG* gsrc = grad + row * cols;
+  const TG* ysrc = outp + row * cols;
+  const int nvec = cols / VW, rest = cols - nvec * VW;
+  uint4 g[NV], y[NV];
+  // g, then y: the sum of g runs while y is in flight
+  const bool more = VW > 1 && l < rest;
+  row_load<TG, VW, G, NV>(g, gsrc, l, nvec);
+  float gt = 0.0f, yt = 0.0f;
+  if (more) gt = (float)to_arith(gsrc[nvec * VW + l]);
+  row_load<TG, VW, G, NV>(y, ysrc, l, nvec);
+  if (more) yt = (float)to_arith(ysrc[nvec * VW + l]);
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (l + j * G < nvec) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) {
+        if constexpr (LOG) s += row_elem<TG, VW>(g[j], k);
+        else s = fmaf(row_elem<TG, VW>(g[j], k), row_elem<TG, VW>(y[j], k), s);
+      }
+    }
+  s = row_sum<G>(LOG ? s + gt : fmaf(gt, yt, s));
+  auto res = [&](float gk, float yk) {
+    if constexpr (LOG) return fmaf(-__builtin_amdgcn_exp2f(yk * kLog2e), s, gk);
+    else return yk * (gk - s);
+  };
+  if constexpr (VW > 1) {
+    opaque<NV>(g);
+    opaque<NV>(y);
+  }
+  TO* dst = gin + row * cols;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (l + j * G < nvec) {
+      float f[VW];
+#pragma unroll
+      for (int k = 0; k < VW; ++k) f[k] = res(row_elem<TG, VW>(g[j], k), row_elem<TG, VW>(y[j], k));
+      row_store<TO, VW>(dst + (int64_t)(l + j * G) * VW, f);
+    }
+  if (VW > 1 && l < rest) dst[nvec * VW + l] = from_arith<TO>(res(gt, yt));
+}
+
+// Calls launch(VW, G, NV as integral constants, workgroups) for a row of
+// `cols` elements in vectors of V; false when the row has more than MAXV
+// vectors.  Up to 16 elements one lane per element; else the fewest lanes
+// that hold the row in one vector each (16, 64), then 2, 4 and 8 vectors a
+// lane of one wavefront, then workgroups: forward 256 threads by 4 and 512 by
+// 4 or 5, backward 1024 by 1 or 2 (bf16 [8192, 8192] forward 45 us against 56
+// with 1024 threads, backward 64 us against 66 with 256).
+template <int V, int MAXV, bool BWD, typename F>
+bool row_split(int64_t rows, int64_t cols, F&& launch) {
+  using std::integral_constant;
+  const int64_t nv = (cols + V - 1) / V;
+  if (nv > MAXV) return false;
+  auto go = [&](auto vw, auto g, auto n) {
+    const int64_t per = g.value <= 64 ? 256 / g.value : 1;
+    launch(vw, g, n, (unsigned)((rows + per - 1) / per));
+  };
+  using I1 = integral_constant<int, 1>;
+  using IV = integral_constant<int, V>;
+  if (cols <= 16) go(I1{}, integral_constant<int, 16>{}, I1{});
+  else if (nv <= 16) go(IV{}, integral_constant<int, 16>{}, I1{});
+  else if (nv <= 64) go(IV{}, integral_constant<int, 64>{}, I1{});
+  else if (nv <= 128) go(IV{}, integral_constant<int, 64>{}, integral_constant<int, 2>{});
+  else if (nv <= 256) go(IV{}, integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  else if (nv <= 512) go(IV{}, integral_constant<int, 64>{}, integral_constant<int, 8>{});
+  else if constexpr (BWD) {
+    if (nv <= 1024) go(IV{}, integral_constant<int, 1024>{}, I1{});
+    else go(IV{}, integral_constant<int, 1024>{}, integral_constant<int, 2>{});
+  } else if (nv <= 1024) go(IV{}, integral_constant<int, 256>{}, integral_constant<int, 4>{});
+  else if (nv <= 2048) go(IV{}, integral_constant<int, 512>{}, integral_constant<int, 4>{});
+  else go(IV{}, integral_constant<int, 512>{}, integral_constant<int, MAXV / 512>{});
+  return true;
+}
 
 template <typename TI, typename TO, int VPT, bool LOG>
 __global__ void __launch_bounds__(kRowBlock)
@@ -183,27 +365,66 @@ k_lsm_fwd_reg(const TI* __restrict__ in, TO* __restrict__ out, int64_t rows, int
   }
 }
 
-// Streaming fallback: any cols.
+// Rows past every other kernel: an online (max, sum) pass, then the output
+// from a second read, in 16-byte vectors with kStreamU in flight.
+constexpr int kStreamU = 4;
+
 template <typename TI, typename TO, bool LOG>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kRowBlock)
 k_lsm_fwd_stream(const TI* __restrict__ in, TO* __restrict__ out, int64_t cols) {
-  __shared__ float lds[kBlock / 64];
-  const TI* x = in + (int64_t)blockIdx.x * cols;
-  float m = -__builtin_inff();
-  for (int64_t c = threadIdx.x; c < cols; c += kBlock) m = nmax(m, (float)to_arith(x[c]));
-  m = block_max_all<kBlock / 64>(m, lds);
-  const float mb = (m == -__builtin_inff()) ? 0.0f : m;
-  float s = 0.0f;
-  for (int64_t c = threadIdx.x; c < cols; c += kBlock) s += fast_exp((float)to_arith(x[c]) - mb);
-  s = block_sum_all<kBlock / 64>(s, lds);
-  TO* o = out + (int64_t)blockIdx.x * cols;
-  if constexpr (LOG) {
-    const float logsum = sa_logf(s);
-    for (int64_t c = threadIdx.x; c < cols; c += kBlock) o[c] = from_arith<TO>(((float)to_arith(x[c]) - m) - logsum);
-  } else {
-    const float inv = 1.0f / s;
-    for (int64_t c = threadIdx.x; c < cols; c += kBlock) o[c] = from_arith<TO>(fast_exp((float)to_arith(x[c]) - mb) * inv);
+  constexpr int V = VecOf<TI>::V, U = kStreamU, NW = kRowBlock / 64;
+  __shared__ float lds_m[NW], lds_s[NW];
+  const TI* src = in + (int64_t)blockIdx.x * cols;
+  TO* dst = out + (int64_t)blockIdx.x * cols;
+  const int64_t nvec = cols / V;
+  const int tid = threadIdx.x, rest = (int)(cols - nvec * V);
+  const float xt = tid < rest ? (float)to_arith(src[nvec * V + tid]) : -__builtin_inff();
+  float m = xt, s = xt == -__builtin_inff() ? 0.0f : (xt != xt ? xt : fast_exp(xt - xt));  // e^0, NaN for NaN and inf
+  for (int64_t v0 = tid; v0 < nvec; v0 += (int64_t)U * kRowBlock) {
+    uint4 w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (v0 + (int64_t)u * kRowBlock < nvec) w[u] = ld_any(src + (v0 + (int64_t)u * kRowBlock) * V);
+    float M = m;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (v0 + (int64_t)u * kRowBlock < nvec) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) M = fmaxf(M, elem_f<TI>(w[u], k));
+      }
+    const float mb = M == -__builtin_inff() ? 0.0f : M;
+    s = lse_rescale(s, m, M);
+    m = M;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (v0 + (int64_t)u * kRowBlock < nvec) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) s += __builtin_amdgcn_exp2f((elem_f<TI>(w[u], k) - mb) * kLog2e);
+      }
   }
+  lanes_lse<64>(m, s);
+  if ((tid & 63) == 0) {
+    lds_m[tid >> 6] = m;
+    lds_s[tid >> 6] = s;
+  }
+  __syncthreads();
+  m = lds_m[tid & 15];
+  s = lds_s[tid & 15];
+  lanes_lse<NW>(m, s);
+  const float a = LOG ? m : (m == -__builtin_inff() ? 0.0f : m);
+  const float b = LOG ? sa_logf(s) : 1.0f / s;
+  auto res = [&](float v) {
+    if constexpr (LOG) return (v - a) - b;
+    else return __builtin_amdgcn_exp2f((v - a) * kLog2e) * b;
+  };
+  for (int64_t v = tid; v < nvec; v += kRowBlock) {
+    const uint4 w = ld_any_stream(src + v * V);
+    float f[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) f[k] = res(elem_f<TI>(w, k));
+    store_any<TO, V>(dst + v * V, f);
+  }
+  if (tid < rest) dst[nvec * V + tid] = from_arith<TO>(res(xt));
 }
 
 // ------------------------------------------------------------ backward
@@ -270,16 +491,53 @@ k_lsm_bwd_reg(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __re
   }
 }
 
-template <typename TG, typename TO>
-__global__ void __launch_bounds__(kBlock)
-k_lsm_bwd_stream(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restrict__ gin, int64_t cols) {
-  __shared__ float lds[kBlock / 64];
-  const int64_t base = (int64_t)blockIdx.x * cols;
-  float s = 0.0f;
-  for (int64_t c = threadIdx.x; c < cols; c += kBlock) s += (float)to_arith(grad[base + c]);
-  s = block_sum_all<kBlock / 64>(s, lds);
-  for (int64_t c = threadIdx.x; c < cols; c += kBlock)
-    gin[base + c] = from_arith<TO>(fmaf(-fast_exp((float)to_arith(outp[base + c])), s, (float)to_arith(grad[base + c])));
+// Rows past every other kernel: the sum, then the output from a second read.
+template <typename TG, typename TO, bool LOG>
+__global__ void __launch_bounds__(kRowBlock)
+k_bwd_stream(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restrict__ gin, int64_t cols) {
+  constexpr int V = VecOf<TG>::V, U = kStreamU;
+  __shared__ float lds[kRowBlock / 64];
+  const int64_t base = (int64_t)blockIdx.x * cols, nvec = cols / V;
+  const TG* gs = grad + base;
+  const TG* ys = outp + base;
+  TO* dst = gin + base;
+  const int tid = threadIdx.x, rest = (int)(cols - nvec * V);
+  const float gt = tid < rest ? (float)to_arith(gs[nvec * V + tid]) : 0.0f;
+  const float yt = tid < rest ? (float)to_arith(ys[nvec * V + tid]) : 0.0f;
+  float s = LOG ? gt : gt * yt;
+  for (int64_t v0 = tid; v0 < nvec; v0 += (int64_t)U * kRowBlock) {
+    uint4 g[U], y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t v = v0 + (int64_t)u * kRowBlock;
+      if (v < nvec) {
+        g[u] = ld_any(gs + v * V);
+        if constexpr (!LOG) y[u] = ld_any(ys + v * V);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (v0 + (int64_t)u * kRowBlock < nvec) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          if constexpr (LOG) s += elem_f<TG>(g[u], k);
+          else s = fmaf(elem_f<TG>(g[u], k), elem_f<TG>(y[u], k), s);
+        }
+      }
+  }
+  s = block_sum_all<kRowBlock / 64>(s, lds);
+  auto res = [&](float gk, float yk) {
+    if constexpr (LOG) return fmaf(-__builtin_amdgcn_exp2f(yk * kLog2e), s, gk);
+    else return yk * (gk - s);
+  };
+  for (int64_t v = tid; v < nvec; v += kRowBlock) {
+    const uint4 g = ld_any_stream(gs + v * V), y = ld_any_stream(ys + v * V);
+    float f[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) f[k] = res(elem_f<TG>(g, k), elem_f<TG>(y, k));
+    store_any<TO, V>(dst + v * V, f);
+  }
+  if (tid < rest) dst[nvec * V + tid] = from_arith<TO>(res(gt, yt));
 }
 
 // softmax backward: gi = y (g - sum(g y)).  Both rows stay in registers
@@ -324,19 +582,6 @@ k_sm_bwd_reg(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __res
       store_row_vec<TO, V>(dst, tid + j * kRowBlock, f);
     }
   }
-}
-
-template <typename TG, typename TO>
-__global__ void __launch_bounds__(kBlock)
-k_sm_bwd_stream(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restrict__ gin, int64_t cols) {
-  __shared__ float lds[kBlock / 64];
-  const int64_t base = (int64_t)blockIdx.x * cols;
-  float s = 0.0f;
-  for (int64_t c = threadIdx.x; c < cols; c += kBlock)
-    s = fmaf((float)to_arith(grad[base + c]), (float)to_arith(outp[base + c]), s);
-  s = block_sum_all<kBlock / 64>(s, lds);
-  for (int64_t c = threadIdx.x; c < cols; c += kBlock)
-    gin[base + c] = from_arith<TO>((float)to_arith(outp[base + c]) * ((float)to_arith(grad[base + c]) - s));
 }
 
 // ------------------------------------------------------- split rows
@@ -437,21 +682,111 @@ __device__ __forceinline__ void split_release(uint64_t* rs, uint32_t* done_row, 
 // loads are not split by divergent ones; a part that fills all but its
 // threads' last vector guards only that one.  `end` is one past the part's
 // last vector.
-template <int NV>
-__device__ __forceinline__ void split_load(uint4 (&x)[NV], const uint4* src, int base, int end) {
+// Loads are written at element alignment also for aligned rows: the same
+// instructions, and the float32 backward no longer spilled ([4096, 50304]
+// 425 -> 391 us, [4096, 65536] 521 -> 496 us).
+template <typename T, int NV>
+__device__ __forceinline__ void split_load(uint4 (&x)[NV], const T* row, int base, int end) {
+  constexpr int V = VecOf<T>::V;
   const int tid = threadIdx.x;
-  const int nvec = end;
-  if (base + kSplitBlock * NV <= nvec) {
+  auto at = [&](int v) { return ld_any_stream(row + (int64_t)v * V); };
+  if (base + kSplitBlock * NV <= end) {
 #pragma unroll
-    for (int j = 0; j < NV; ++j) x[j] = ld_stream(src + base + tid + j * kSplitBlock);
-  } else if (base + kSplitBlock * (NV - 1) <= nvec) {
+    for (int j = 0; j < NV; ++j) x[j] = at(base + tid + j * kSplitBlock);
+  } else if (base + kSplitBlock * (NV - 1) <= end) {
 #pragma unroll
-    for (int j = 0; j < NV - 1; ++j) x[j] = ld_stream(src + base + tid + j * kSplitBlock);
-    if (base + tid + (NV - 1) * kSplitBlock < nvec) x[NV - 1] = ld_stream(src + base + tid + (NV - 1) * kSplitBlock);
+    for (int j = 0; j < NV - 1; ++j) x[j] = at(base + tid + j * kSplitBlock);
+    if (base + tid + (NV - 1) * kSplitBlock < end) x[NV - 1] = at(base + tid + (NV - 1) * kSplitBlock);
   } else {
 #pragma unroll
     for (int j = 0; j < NV; ++j)
-      if (base + tid + j * kSplitBlock < nvec) x[j] = ld_stream(src + base + tid + j * kSplitBlock);
+      if (base + tid + j * kSplitBlock < end) x[j] = at(base + tid + j * kSplitBlock);
+  }
+}
+
+// RAGGED rows, whose cols is no multiple of the vector.  The forward moves
+// floor(cols / V) vectors at element alignment; its last part also holds the
+// rest of the row, element nvec V + t in thread t, as a float (-inf in every
+// other thread).
+template <bool RAGGED, typename T>
+__device__ __forceinline__ float split_rest(const T* row, int64_t cols, int nvec, bool last) {
+  if constexpr (!RAGGED) return -__builtin_inff();
+  const int64_t i = (int64_t)nvec * VecOf<T>::V + threadIdx.x;
+  return last && i < cols ? (float)to_arith(row[i]) : -__builtin_inff();
+}
+
+// The backward, with three streams, takes the vectors of the 16-byte grid
+// instead, so that every access is aligned; row r starts o = r cols mod V
+// elements into its first one.  The elements of the first and the last vector
+// outside the row are never read or written: those vectors load and store
+// element by element, with zeros in the places outside.  bf16 [4096, 50257]:
+// 239 us, at element alignment 306 us (the forward 160 and 151 us; aligned
+// rows of 50304 193 and 133 us; streaming the rows twice by scalars, as rows
+// of odd length did before, 501 and 551 us).
+struct SplitRow {
+  int o;         // elements of the first vector that precede the row
+  int vf0, vf1;  // vectors wholly inside the row
+  int nvec;      // vectors the row touches
+};
+template <typename T, bool RAGGED>
+__device__ __forceinline__ SplitRow split_row(int row, int64_t cols) {
+  constexpr int V = VecOf<T>::V;
+  SplitRow r;
+  r.o = RAGGED ? (int)(((int64_t)row * cols) % V) : 0;
+  r.vf0 = RAGGED && r.o ? 1 : 0;
+  r.vf1 = (int)((r.o + cols) / V);
+  r.nvec = RAGGED ? (int)((r.o + cols + V - 1) / V) : r.vf1;
+  return r;
+}
+// The row's elements in vector v are [lo, hi) of its V.
+template <typename T>
+__device__ __forceinline__ void split_edge(const SplitRow& r, int64_t cols, int v, int& lo, int& hi) {
+  constexpr int V = VecOf<T>::V;
+  lo = v == 0 ? r.o : 0;
+  const int64_t left = r.o + cols - (int64_t)v * V;
+  hi = left < V ? (int)left : V;
+}
+
+// `row` points at the first vector's first element (o before the row).
+template <typename T, int NV, bool RAGGED>
+__device__ __forceinline__ void split_load_grid(uint4 (&x)[NV], const T* row, const SplitRow& r, int64_t cols, int base,
+                                                int end) {
+  constexpr int V = VecOf<T>::V;
+  if (RAGGED && (base < r.vf0 || end > r.vf1)) {
+    using Bits = std::conditional_t<sizeof(T) == 2, uint16_t, uint32_t>;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int v = base + (int)threadIdx.x + j * kSplitBlock;
+      const T* p = row + (int64_t)v * V;
+      if (v >= r.vf0 && v < end && v < r.vf1) {
+        x[j] = ld_any_stream(p);
+      } else if (v < end) {
+        int lo, hi;
+        split_edge<T>(r, cols, v, lo, hi);
+        Bits b[V];
+#pragma unroll
+        for (int k = 0; k < V; ++k) b[k] = k >= lo && k < hi ? reinterpret_cast<const Bits*>(p)[k] : Bits(0);
+        __builtin_memcpy(&x[j], b, 16);
+      }
+    }
+  } else {
+    split_load<T, NV>(x, row, base, end);
+  }
+}
+
+// Stores vector v of a row's results (dst as `row` above).
+template <typename TI, typename TO, bool RAGGED>
+__device__ __forceinline__ void split_store(TO* dst, const SplitRow& r, int64_t cols, int v,
+                                            const float (&f)[VecOf<TI>::V]) {
+  constexpr int V = VecOf<TI>::V;
+  if (RAGGED && (v < r.vf0 || v >= r.vf1)) {
+    int lo, hi;
+    split_edge<TI>(r, cols, v, lo, hi);
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+      if (k >= lo && k < hi) dst[(int64_t)v * V + k] = from_arith<TO>(f[k]);
+  } else {
+    store_any<TO, V>(dst + (int64_t)v * V, f);
   }
 }
 
@@ -475,11 +810,11 @@ __device__ __forceinline__ float block_sum(const float* lds) {
 // The forward keeps its per-vector guards on whole parts too: a specialization
 // without them took 62 VGPRs against 57 and ran at 71.1-71.9 % of the HBM
 // roofline against 73.2-74.7 % on c3's rows.
-template <typename TI, int NV>
-__device__ __forceinline__ void thread_lse(uint4 (&x)[NV], int base, int nvec, float& m, float& s) {
+template <typename TI, int NV, bool RAGGED>
+__device__ __forceinline__ void thread_lse(uint4 (&x)[NV], float xt, int base, int nvec, float& m, float& s) {
   constexpr int V = VecOf<TI>::V;
   const int tid = threadIdx.x;
-  m = -__builtin_inff();
+  m = RAGGED ? xt : -__builtin_inff();
 #pragma unroll
   for (int j = 0; j < NV; ++j)
     if (base + tid + j * kSplitBlock < nvec) {
@@ -488,7 +823,7 @@ __device__ __forceinline__ void thread_lse(uint4 (&x)[NV], int base, int nvec, f
     }
   const float mb = m == -__builtin_inff() ? 0.0f : m;
   opaque<NV>(x);
-  s = 0.0f;
+  s = RAGGED ? __builtin_amdgcn_exp2f((xt - mb) * kLog2e) : 0.0f;
 #pragma unroll
   for (int j = 0; j < NV; ++j)
     if (base + tid + j * kSplitBlock < nvec) {
@@ -499,11 +834,11 @@ __device__ __forceinline__ void thread_lse(uint4 (&x)[NV], int base, int nvec, f
 
 // (max, sum of exp(x - max)) of one part, the same in every thread; the
 // sum's NaN is canonical.
-template <typename TI, int NV>
-__device__ __forceinline__ uint64_t part_lse(uint4 (&x)[NV], int base, int nvec, float* lds_m, float* lds_s) {
+template <typename TI, int NV, bool RAGGED>
+__device__ __forceinline__ uint64_t part_lse(uint4 (&x)[NV], float xt, int base, int nvec, float* lds_m, float* lds_s) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float m, s;
-  thread_lse<TI, NV>(x, base, nvec, m, s);
+  thread_lse<TI, NV, RAGGED>(x, xt, base, nvec, m, s);
   lanes_lse<64>(m, s);
   __syncthreads();
   if (lane == 0) {
@@ -518,8 +853,7 @@ __device__ __forceinline__ uint64_t part_lse(uint4 (&x)[NV], int base, int nvec,
 }
 
 template <typename TI, typename TO, bool LOG>
-__device__ __forceinline__ void fwd_split_out(const uint4 (&x)[kFwdNV], Vec<TO, VecOf<TI>::V>* dst, int base,
-                                              int nvec, float M, float logsum, float Mb, float inv) {
+__device__ __forceinline__ void fwd_split_out(const uint4 (&x)[kFwdNV], TO* dst, int base, int nvec, float M, float logsum, float Mb, float inv) {
   constexpr int V = VecOf<TI>::V;
 #pragma unroll
   for (int j = 0; j < kFwdNV; ++j) {
@@ -531,12 +865,12 @@ __device__ __forceinline__ void fwd_split_out(const uint4 (&x)[kFwdNV], Vec<TO, 
         if constexpr (LOG) f[k] = (elem_f<TI>(x[j], k) - M) - logsum;
         else f[k] = __builtin_amdgcn_exp2f((elem_f<TI>(x[j], k) - Mb) * kLog2e) * inv;
       }
-      store_row_vec<TO, V>(dst, v, f);
+      store_any<TO, V>(dst + (int64_t)v * V, f);
     }
   }
 }
 
-template <typename TI, typename TO, bool LOG>
+template <typename TI, typename TO, bool LOG, bool RAGGED>
 __global__ void __launch_bounds__(kSplitBlock, 8)
 k_lsm_fwd_split(const TI* __restrict__ in, TO* __restrict__ out, int64_t cols, int K, int plen,
                 uint64_t* __restrict__ slots, uint32_t* __restrict__ done, uint32_t spin_limit) {
@@ -550,10 +884,11 @@ k_lsm_fwd_split(const TI* __restrict__ in, TO* __restrict__ out, int64_t cols, i
   const int nvec = (int)(cols / V);
   const int base = part * plen;
   const int end = min(base + plen, nvec);
-  const uint4* src = reinterpret_cast<const uint4*>(in + (int64_t)row * cols);
+  const TI* src = in + (int64_t)row * cols;
   uint4 x[kFwdNV];
-  split_load<kFwdNV>(x, src, base, end);
-  const uint64_t mine = part_lse<TI, kFwdNV>(x, base, end, lds_m, lds_s);
+  split_load<TI, kFwdNV>(x, src, base, end);
+  const float xt = split_rest<RAGGED>(src, cols, nvec, part == K - 1);
+  const uint64_t mine = part_lse<TI, kFwdNV, RAGGED>(x, xt, base, end, lds_m, lds_s);
   opaque<kFwdNV>(x);
   uint64_t* rs = slots + (int64_t)row * K;
   if (threadIdx.x == 0) slot_publish(rs + part, mine);
@@ -564,11 +899,12 @@ k_lsm_fwd_split(const TI* __restrict__ in, TO* __restrict__ out, int64_t cols, i
       const int q = __builtin_ctz(miss);
       miss &= miss - 1;
       const int qb = q * plen, qe = min(qb + plen, nvec);
-      split_load<kFwdNV>(x, src, qb, qe);
-      const uint64_t w = part_lse<TI, kFwdNV>(x, qb, qe, lds_m, lds_s);
+      split_load<TI, kFwdNV>(x, src, qb, qe);
+      const float qt = split_rest<RAGGED>(src, cols, nvec, q == K - 1);
+      const uint64_t w = part_lse<TI, kFwdNV, RAGGED>(x, qt, qb, qe, lds_m, lds_s);
       if (threadIdx.x == 0) part_w[q] = w;
     } while (miss);
-    split_load<kFwdNV>(x, src, base, end);
+    split_load<TI, kFwdNV>(x, src, base, end);
   }
   __syncthreads();
   // the row's (max, sum) from the K part pairs, in part order: the max, then
@@ -582,8 +918,13 @@ k_lsm_fwd_split(const TI* __restrict__ in, TO* __restrict__ out, int64_t cols, i
   const float inv = LOG ? 0.0f : 1.0f / S;
   const float Mb = M == -__builtin_inff() ? 0.0f : M;
   opaque<kFwdNV>(x);
-  Vec<TO, V>* dst = reinterpret_cast<Vec<TO, V>*>(out + (int64_t)row * cols);
+  TO* dst = out + (int64_t)row * cols;
   fwd_split_out<TI, TO, LOG>(x, dst, base, end, M, logsum, Mb, inv);
+  if constexpr (RAGGED) {
+    const int64_t i = (int64_t)nvec * V + threadIdx.x;
+    if (part == K - 1 && i < cols)
+      dst[i] = from_arith<TO>(LOG ? (xt - M) - logsum : __builtin_amdgcn_exp2f((xt - Mb) * kLog2e) * inv);
+  }
 }
 
 template <typename TG, bool WHOLE>
@@ -611,9 +952,10 @@ __device__ __forceinline__ uint64_t part_sum(uint4 (&g)[kBwdNV], int base, int n
   return (uint64_t)__float_as_uint(block_sum(lds));
 }
 
-template <typename TG, typename TO, bool WHOLE>
+template <typename TG, typename TO, bool WHOLE, bool RAGGED>
 __device__ __forceinline__ void bwd_split_out(const uint4 (&gv)[kBwdNV], const uint4 (&yv)[kBwdNV],
-                                              Vec<TO, VecOf<TG>::V>* dst, int base, int nvec, float S) {
+                                              TO* dst, const SplitRow& r, int64_t cols, int base, int nvec,
+                                              float S) {
   constexpr int V = VecOf<TG>::V;
 #pragma unroll
   for (int j = 0; j < kBwdNV; ++j) {
@@ -623,12 +965,12 @@ __device__ __forceinline__ void bwd_split_out(const uint4 (&gv)[kBwdNV], const u
 #pragma unroll
       for (int k = 0; k < V; ++k)
         f[k] = fmaf(-__builtin_amdgcn_exp2f(elem_f<TG>(yv[j], k) * kLog2e), S, elem_f<TG>(gv[j], k));
-      store_row_vec<TO, V>(dst, v, f);
+      split_store<TG, TO, RAGGED>(dst, r, cols, v, f);
     }
   }
 }
 
-template <typename TG, typename TO>
+template <typename TG, typename TO, bool RAGGED>
 __global__ void __launch_bounds__(kSplitBlock, 8)
 k_lsm_bwd_split(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restrict__ gin, int64_t cols, int K,
                 int plen, uint64_t* __restrict__ slots, uint32_t* __restrict__ done, uint32_t spin_limit) {
@@ -638,14 +980,15 @@ k_lsm_bwd_split(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __
   __shared__ uint32_t lds_missing;
   const int row = (int)(blockIdx.x / (unsigned)K);
   const int part = (int)(blockIdx.x - (unsigned)row * (unsigned)K);
-  const int nvec = (int)(cols / V);
+  const SplitRow r = split_row<TG, RAGGED>(row, cols);
+  const int nvec = r.nvec;
   const int base = part * plen;
   const int end = min(base + plen, nvec);
-  const uint4* g = reinterpret_cast<const uint4*>(grad + (int64_t)row * cols);
-  const uint4* y = reinterpret_cast<const uint4*>(outp + (int64_t)row * cols);
+  const TG* g = grad + (int64_t)row * cols - r.o;
+  const TG* y = outp + (int64_t)row * cols - r.o;
   uint4 gv[kBwdNV], yv[kBwdNV];
-  split_load<kBwdNV>(gv, g, base, end);
-  split_load<kBwdNV>(yv, y, base, end);
+  split_load_grid<TG, kBwdNV, RAGGED>(gv, g, r, cols, base, end);
+  split_load_grid<TG, kBwdNV, RAGGED>(yv, y, r, cols, base, end);
   // every load of the part in flight before the sum: float32 parts, whose
   // sum is short, otherwise had it scheduled between the loads (75.2 ->
   // 76.3 % on [8192, 64128], 72.8 -> 75.3 % on [16384, 28672]; bf16 rows
@@ -663,20 +1006,20 @@ k_lsm_bwd_split(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __
       const int q = __builtin_ctz(miss);
       miss &= miss - 1;
       const int qb = q * plen, qe = min(qb + plen, nvec);
-      split_load<kBwdNV>(gv, g, qb, qe);
+      split_load_grid<TG, kBwdNV, RAGGED>(gv, g, r, cols, qb, qe);
       const uint64_t w = part_sum<TG>(gv, qb, qe, lds);
       if (threadIdx.x == 0) part_w[q] = w;
     } while (miss);
-    split_load<kBwdNV>(gv, g, base, end);
+    split_load_grid<TG, kBwdNV, RAGGED>(gv, g, r, cols, base, end);
   }
   __syncthreads();
   float S = __uint_as_float((uint32_t)part_w[0]);
   for (int q = 1; q < K; ++q) S += __uint_as_float((uint32_t)part_w[q]);
   opaque<kBwdNV>(gv);
   opaque<kBwdNV>(yv);
-  Vec<TO, V>* dst = reinterpret_cast<Vec<TO, V>*>(gin + (int64_t)row * cols);
-  if (base + kSplitBlock * kBwdNV <= end) bwd_split_out<TG, TO, true>(gv, yv, dst, base, end, S);
-  else bwd_split_out<TG, TO, false>(gv, yv, dst, base, end, S);
+  TO* dst = gin + (int64_t)row * cols - r.o;
+  if (base + kSplitBlock * kBwdNV <= end) bwd_split_out<TG, TO, true, RAGGED>(gv, yv, dst, r, cols, base, end, S);
+  else bwd_split_out<TG, TO, false, RAGGED>(gv, yv, dst, r, cols, base, end, S);
 }
 
 __global__ void __launch_bounds__(kBlock) k_split_init(uint64_t* slots, uint32_t* done, int64_t n) {
@@ -780,6 +1123,14 @@ inline int split_part_len(int64_t nvec, int K, int part, int whole_from) {
   return (int)(((nvec + K - 1) / K + 63) / 64 * 64);
 }
 
+// The most 16-byte grid vectors a row of cols elements touches.
+inline int64_t split_vecs(int64_t cols, int v) { return cols % v == 0 ? cols / v : (cols + 2 * v - 2) / v; }
+
+// Aligned backward rows of 513 to 2048 whole vectors stay on the unguarded
+// 1024-thread kernels (bf16 [8192, 10000] 78 us against 88 on k_row_bwd,
+// [4096, 16384] 62 against 65; float32 rows within 2 %).
+inline bool bwd_reg_rows(int64_t cols, int v) { return cols % v == 0 && cols / v > 512 && cols / v <= 2 * kRowBlock; }
+
 template <bool LOG>
 int softmax_forward(const void* in, int32_t in_dtype, void* out, int32_t out_dtype, int64_t rows, int64_t cols,
                     void* stream) {
@@ -790,42 +1141,54 @@ int softmax_forward(const void* in, int32_t in_dtype, void* out, int32_t out_dty
     return with_float_storage(out_dtype, [&](auto* to) -> int {
       using TI = std::remove_pointer_t<decltype(ti)>;
       using TO = std::remove_pointer_t<decltype(to)>;
-      if (in_dtype != out_dtype && out_dtype != SUPA_AMD_F32) return SUPA_AMD_EDTYPE;
+      if constexpr (!std::is_same<TI, TO>::value && !std::is_same<TO, float>::value) return SUPA_AMD_EDTYPE;
+      else {
       constexpr int V = VecOf<TI>::V;
-      const bool vec_ok = (cols % V) == 0 && aligned(in, 16) && aligned(out, V * sizeof(TO));
-      const int K = vec_ok ? split_parts(cols / V, kSplitBlock * kFwdNV, in, nullptr,
-                                         rows * cols * (int64_t)sizeof(TI), out, rows * cols * (int64_t)sizeof(TO))
-                           : 0;
+      const TI* pi = static_cast<const TI*>(in);
+      TO* po = static_cast<TO*>(out);
+      // aligned float32 rows of 1025 to 2048 vectors: the persistent kernel
+      // ([8192, 8192] 92 us, k_row_fwd 94)
+      if (sizeof(TI) == 4 && cols % V == 0 && cols / V > kRowBlock && cols / V <= 2 * kRowBlock && aligned(in, 16) &&
+          aligned(out, 16)) {
+        k_lsm_fwd_reg<TI, TO, 2, LOG>
+            <<<(unsigned)std::min<int64_t>(rows, kLsmGrid), kRowBlock, 0, st>>>(pi, po, rows, cols);
+        return launch_status();
+      }
+      if (row_split<V, kSplitBlock * kFwdNV, false>(rows, cols, [&](auto vw, auto g, auto nv, unsigned blocks) {
+            k_row_fwd<TI, TO, vw.value, g.value, nv.value, LOG>
+                <<<blocks, row_block<g.value>(), 0, st>>>(pi, po, rows, (int)cols);
+          }))
+        return launch_status();
+      const int64_t nvec = (cols + V - 1) / V;
+      const int K = split_parts(nvec, kSplitBlock * kFwdNV, in, nullptr, rows * cols * (int64_t)sizeof(TI), out,
+                                rows * cols * (int64_t)sizeof(TO));
       SplitScratch sb;
       uint32_t spin = 0;
       if (K > 0 && split_scratch(st, sb, spin)) {
-        const int plen = split_part_len(cols / V, K, kSplitBlock * kFwdNV, kSplitMaxK + 1);
+        const int plen = split_part_len(nvec, K, kSplitBlock * kFwdNV, kSplitMaxK + 1);
         const int64_t chunk = kSplitSlots / K;
         for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
           const int64_t nr = std::min(chunk, rows - r0);
-          k_lsm_fwd_split<TI, TO, LOG><<<(unsigned)(nr * K), kSplitBlock, 0, st>>>(
-              static_cast<const TI*>(in) + r0 * cols, static_cast<TO*>(out) + r0 * cols, cols, K, plen, sb.slots,
-              sb.done, spin);
+          if (cols % V)
+            k_lsm_fwd_split<TI, TO, LOG, true><<<(unsigned)(nr * K), kSplitBlock, 0, st>>>(
+                pi + r0 * cols, po + r0 * cols, cols, K, plen, sb.slots, sb.done, spin);
+          else
+            k_lsm_fwd_split<TI, TO, LOG, false><<<(unsigned)(nr * K), kSplitBlock, 0, st>>>(
+                pi + r0 * cols, po + r0 * cols, cols, K, plen, sb.slots, sb.done, spin);
         }
         return launch_status();
       }
-      const bool reg_ok = vec_ok && (cols / V) <= 16 * kRowBlock;
-      if (reg_ok) {
-        const int64_t nvec = cols / V;
+      if (cols % V == 0 && aligned(in, 16) && aligned(out, 16) && nvec <= 16 * kRowBlock) {
         const int vpt = (int)((nvec + kRowBlock - 1) / kRowBlock);
-        const TI* pi = static_cast<const TI*>(in);
-        TO* po = static_cast<TO*>(out);
         const unsigned grid = (unsigned)std::min<int64_t>(rows, kLsmGrid);
-        if (vpt <= 1) k_lsm_fwd_reg<TI, TO, 1, LOG><<<grid, kRowBlock, 0, st>>>(pi, po, rows, cols);
-        else if (vpt <= 2) k_lsm_fwd_reg<TI, TO, 2, LOG><<<grid, kRowBlock, 0, st>>>(pi, po, rows, cols);
-        else if (vpt <= 4) k_lsm_fwd_reg<TI, TO, 4, LOG><<<grid, kRowBlock, 0, st>>>(pi, po, rows, cols);
+        if (vpt <= 4) k_lsm_fwd_reg<TI, TO, 4, LOG><<<grid, kRowBlock, 0, st>>>(pi, po, rows, cols);
         else if (vpt <= 8) k_lsm_fwd_reg<TI, TO, 8, LOG><<<grid, kRowBlock, 0, st>>>(pi, po, rows, cols);
         else k_lsm_fwd_reg<TI, TO, 16, LOG><<<grid, kRowBlock, 0, st>>>(pi, po, rows, cols);
         return launch_status();
       }
-      k_lsm_fwd_stream<TI, TO, LOG><<<(unsigned)rows, kBlock, 0, st>>>(static_cast<const TI*>(in),
-                                                                       static_cast<TO*>(out), cols);
+      k_lsm_fwd_stream<TI, TO, LOG><<<(unsigned)rows, kRowBlock, 0, st>>>(pi, po, cols);
       return launch_status();
+      }
     });
   });
 }
@@ -855,41 +1218,53 @@ int supa_amd_log_softmax_backward(const void* grad, const void* output, int32_t 
     return with_float_storage(gin_dtype, [&](auto* to) -> int {
       using TG = std::remove_pointer_t<decltype(tg)>;
       using TO = std::remove_pointer_t<decltype(to)>;
-      if (gy_dtype != gin_dtype && gin_dtype != SUPA_AMD_F32) return SUPA_AMD_EDTYPE;
+      if constexpr (!std::is_same<TG, TO>::value && !std::is_same<TO, float>::value) return SUPA_AMD_EDTYPE;
+      else {
       constexpr int V = VecOf<TG>::V;
-      const bool vec_ok = (cols % V) == 0 && aligned(grad, 16) && aligned(output, 16) && aligned(grad_in, V * sizeof(TO));
       const TG* pg = static_cast<const TG*>(grad);
       const TG* py = static_cast<const TG*>(output);
       TO* po = static_cast<TO*>(grad_in);
-      const int K = vec_ok ? split_parts(cols / V, kSplitBlock * kBwdNV, grad, output,
-                                         rows * cols * (int64_t)sizeof(TG), grad_in, rows * cols * (int64_t)sizeof(TO))
-                           : 0;
+      const bool al = aligned(grad, 16) && aligned(output, 16) && aligned(grad_in, 16);
+      const int64_t nvec = split_vecs(cols, V);
+      if (al && bwd_reg_rows(cols, V)) {
+        if (nvec <= kRowBlock) k_lsm_bwd_reg<TG, TO, 1><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
+        else k_lsm_bwd_reg<TG, TO, 2><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
+        return launch_status();
+      }
+      if (row_split<V, kSplitBlock * kBwdNV, true>(rows, cols, [&](auto vw, auto g, auto nv, unsigned blocks) {
+            k_row_bwd<TG, TO, vw.value, g.value, nv.value, true>
+                <<<blocks, row_block<g.value>(), 0, st>>>(pg, py, po, rows, (int)cols);
+          }))
+        return launch_status();
+      const int K = al ? split_parts(nvec, kSplitBlock * kBwdNV, grad, output, rows * cols * (int64_t)sizeof(TG),
+                                     grad_in, rows * cols * (int64_t)sizeof(TO))
+                       : 0;
       SplitScratch sb;
       uint32_t spin = 0;
       if (K > 0 && split_scratch(st, sb, spin)) {
-        const int plen = split_part_len(cols / V, K, kSplitBlock * kBwdNV, 6);
+        const int plen = split_part_len(nvec, K, kSplitBlock * kBwdNV, 6);
         const int64_t chunk = kSplitSlots / K;
         for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
           const int64_t nr = std::min(chunk, rows - r0);
-          k_lsm_bwd_split<TG, TO><<<(unsigned)(nr * K), kSplitBlock, 0, st>>>(pg + r0 * cols, py + r0 * cols,
-                                                                           po + r0 * cols, cols, K, plen, sb.slots,
-                                                                           sb.done, spin);
+          if (cols % V)
+            k_lsm_bwd_split<TG, TO, true><<<(unsigned)(nr * K), kSplitBlock, 0, st>>>(
+                pg + r0 * cols, py + r0 * cols, po + r0 * cols, cols, K, plen, sb.slots, sb.done, spin);
+          else
+            k_lsm_bwd_split<TG, TO, false><<<(unsigned)(nr * K), kSplitBlock, 0, st>>>(
+                pg + r0 * cols, py + r0 * cols, po + r0 * cols, cols, K, plen, sb.slots, sb.done, spin);
         }
         return launch_status();
       }
-      const bool reg_ok = vec_ok && (cols / V) <= 16 * kRowBlock;
-      if (reg_ok) {
-        const int64_t nvec = cols / V;
+      if (al && cols % V == 0 && nvec <= 16 * kRowBlock) {
         const int vpt = (int)((nvec + kRowBlock - 1) / kRowBlock);
-        if (vpt <= 1) k_lsm_bwd_reg<TG, TO, 1><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
-        else if (vpt <= 2) k_lsm_bwd_reg<TG, TO, 2><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
-        else if (vpt <= 4) k_lsm_bwd_reg<TG, TO, 4><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
+        if (vpt <= 4) k_lsm_bwd_reg<TG, TO, 4><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         else if (vpt <= 8) k_lsm_bwd_reg<TG, TO, 8><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         else k_lsm_bwd_reg<TG, TO, 16><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         return launch_status();
       }
-      k_lsm_bwd_stream<TG, TO><<<(unsigned)rows, kBlock, 0, st>>>(pg, py, po, cols);
+      k_bwd_stream<TG, TO, true><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
       return launch_status();
+      }
     });
   });
 }
@@ -903,24 +1278,34 @@ int supa_amd_softmax_backward(const void* grad, const void* output, int32_t gy_d
     return with_float_storage(gin_dtype, [&](auto* to) -> int {
       using TG = std::remove_pointer_t<decltype(tg)>;
       using TO = std::remove_pointer_t<decltype(to)>;
-      if (gy_dtype != gin_dtype && gin_dtype != SUPA_AMD_F32) return SUPA_AMD_EDTYPE;
+      if constexpr (!std::is_same<TG, TO>::value && !std::is_same<TO, float>::value) return SUPA_AMD_EDTYPE;
+      else {
       constexpr int V = VecOf<TG>::V;
       const bool reg_ok = (cols % V) == 0 && aligned(grad, 16) && aligned(output, 16) && aligned(grad_in, V * sizeof(TO)) &&
                           (cols / V) <= 8 * kRowBlock;
       const TG* pg = static_cast<const TG*>(grad);
       const TG* py = static_cast<const TG*>(output);
       TO* po = static_cast<TO*>(grad_in);
+      if (reg_ok && bwd_reg_rows(cols, V)) {
+        if (cols / V <= kRowBlock) k_sm_bwd_reg<TG, TO, 1><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
+        else k_sm_bwd_reg<TG, TO, 2><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
+        return launch_status();
+      }
+      if (row_split<V, kSplitBlock * kBwdNV, true>(rows, cols, [&](auto vw, auto g, auto nv, unsigned blocks) {
+            k_row_bwd<TG, TO, vw.value, g.value, nv.value, false>
+                <<<blocks, row_block<g.value>(), 0, st>>>(pg, py, po, rows, (int)cols);
+          }))
+        return launch_status();
       if (reg_ok) {
         const int64_t nvec = cols / V;
         const int vpt = (int)((nvec + kRowBlock - 1) / kRowBlock);
-        if (vpt <= 1) k_sm_bwd_reg<TG, TO, 1><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
-        else if (vpt <= 2) k_sm_bwd_reg<TG, TO, 2><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
-        else if (vpt <= 4) k_sm_bwd_reg<TG, TO, 4><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
+        if (vpt <= 4) k_sm_bwd_reg<TG, TO, 4><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         else k_sm_bwd_reg<TG, TO, 8><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         return launch_status();
       }
-      k_sm_bwd_stream<TG, TO><<<(unsigned)rows, kBlock, 0, st>>>(pg, py, po, cols);
+      k_bwd_stream<TG, TO, false><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
       return launch_status();
+      }
     });
   });
 }

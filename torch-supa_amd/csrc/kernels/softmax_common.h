@@ -4,6 +4,7 @@
 
 #include "devmath.h"
 #include "ew_launch.h"
+#include "unaligned.h"
 
 namespace sa {
 
@@ -69,6 +70,32 @@ __device__ __forceinline__ void store_row_vec(Vec<TO, V>* dst, int v, const floa
 #pragma unroll
     for (int k = 0; k < V; ++k) o.v[k] = from_arith<TO>(f[k]);
     st_stream(dst + v, o);
+  }
+}
+
+// The same at any element alignment.
+template <typename TO, int V>
+__device__ __forceinline__ void store_any(TO* p, const float (&f)[V]) {
+  if constexpr (std::is_same<TO, bf16>::value) {
+    uint4 q;
+    uint32_t w[V / 2];
+#pragma unroll
+    for (int k = 0; k < V / 2; ++k) {
+      const float2_t v = {f[2 * k], f[2 * k + 1]};
+      w[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+    }
+    __builtin_memcpy(&q, w, 16);
+    st_any_stream(p, q);
+  } else {
+    Vec<TO, V> o;
+#pragma unroll
+    for (int k = 0; k < V; ++k) o.v[k] = from_arith<TO>(f[k]);
+#pragma unroll
+    for (int w = 0; w < (int)(sizeof(o) / 16); ++w) {
+      uint4 q;
+      __builtin_memcpy(&q, reinterpret_cast<const char*>(&o) + 16 * w, 16);
+      st_any_stream(reinterpret_cast<char*>(p) + 16 * w, q);
+    }
   }
 }
 

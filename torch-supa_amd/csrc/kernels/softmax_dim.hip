@@ -63,23 +63,15 @@ __device__ __forceinline__ float dim_elem(const dim_raw_t<T, VW>& w, int k) {
 // Stores elements [skip, VW) of f at p (p is the vector's first element).
 template <typename TO, int VW>
 __device__ __forceinline__ void dim_store(TO* p, const float (&f)[VW], int skip) {
-  Vec<TO, VW> o;
-#pragma unroll
-  for (int k = 0; k < VW; ++k) o.v[k] = from_arith<TO>(f[k]);
-  if constexpr (VW * sizeof(TO) % 16 == 0) {
+  if constexpr (VW > 1) {
     if (skip == 0) {
-#pragma unroll
-      for (int w = 0; w < (int)(VW * sizeof(TO) / 16); ++w) {
-        uint4 q;
-        __builtin_memcpy(&q, reinterpret_cast<const char*>(&o) + 16 * w, 16);
-        st_any_stream(reinterpret_cast<char*>(p) + 16 * w, q);
-      }
+      store_any<TO, VW>(p, f);
       return;
     }
   }
 #pragma unroll
   for (int k = 0; k < VW; ++k)
-    if (k >= skip) p[k] = o.v[k];
+    if (k >= skip) p[k] = from_arith<TO>(f[k]);
 }
 
 struct DimGeom {
