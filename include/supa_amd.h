@@ -447,6 +447,25 @@ int64_t supa_amd_sum_noalloc_max_workspace_bytes(void);
 int supa_amd_sum_rows(const void* in, int32_t in_dtype, void* out, int32_t out_dtype,
                       int64_t outer, int64_t inner, double scale, void* stream);
 
+/* Sums over dims of a dense tensor in its memory order, read once: out[o, i]
+ * = scale * sum_r in[o, r, i] of a contiguous [outer, red, inner] input
+ * (columns), and out[r] = scale * the sum of row r's `segs` runs of `len`
+ * contiguous elements, run s at element r * row_stride + s * seg_stride
+ * (segments; rows of a matrix are one run each).  Dtypes and accumulation as
+ * for supa_amd_sum_rows.  Long reductions with few results take two launches
+ * through a workspace of *_workspace_bytes (0: none needed; no content
+ * requirement).  Replaces sum_stub / mean_stub over dims, without the copy
+ * that moves the reduced dims last. */
+int64_t supa_amd_sum_cols_workspace_bytes(int32_t in_dtype, int32_t out_dtype, int64_t outer, int64_t red,
+                                          int64_t inner);
+int supa_amd_sum_cols(const void* in, int32_t in_dtype, void* out, int32_t out_dtype, int64_t outer, int64_t red,
+                      int64_t inner, double scale, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t supa_amd_sum_segments_workspace_bytes(int32_t in_dtype, int32_t out_dtype, int64_t rows, int64_t segs,
+                                              int64_t len);
+int supa_amd_sum_segments(const void* in, int32_t in_dtype, void* out, int32_t out_dtype, int64_t rows, int64_t segs,
+                          int64_t len, int64_t row_stride, int64_t seg_stride, double scale, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------ row softmax ops */
 
 /* out[r, :] = x[r, :] - max_r - log(sum exp(x[r, :] - max_r)) over rows of a

@@ -106,6 +106,68 @@ std::vector<int64_t> reduce_dims(const at::Tensor& self, at::OptionalIntArrayRef
   return dims;
 }
 
+// How a reduction over `red` dims reads x where it lies: x dense in some dim
+// order, the kept dims in their own order within it, the reduced dims first
+// (columns), last (segments of one run), between kept ones (columns) or around
+// them (segments: a channel's planes).  kNone: any other pattern.
+struct DimPlan {
+  enum Kind { kNone, kCols, kSegments } kind = kNone;
+  int64_t outer = 1, red = 1, inner = 1;                    // kCols; outer = rows of kSegments
+  int64_t segs = 1, len = 1, row_stride = 0, seg_stride = 0;  // kSegments
+};
+DimPlan dim_plan(const at::Tensor& x, const std::vector<bool>& red) {
+  DimPlan p;
+  int64_t order[64];  // dims of more than one element, slowest first
+  int n = 0;
+  const int64_t nd = x.dim();
+  if (nd > 64) return p;
+  for (int64_t i = 0; i < nd; ++i) {
+    if (x.size(i) == 1) continue;
+    int k = n++;
+    for (; k > 0 && x.stride(order[k - 1]) < x.stride(i); --k) order[k] = order[k - 1];
+    order[k] = i;
+  }
+  int64_t dense = 1, last_kept = nd;
+  for (int k = n; k-- > 0;) {
+    const int64_t d = order[k];
+    if (x.stride(d) != dense) return p;
+    dense *= x.size(d);
+    if (!red[d]) {
+      if (d > last_kept) return p;
+      last_kept = d;
+    }
+  }
+  c10::SmallVector<std::pair<bool, int64_t>, 8> g;  // runs of kept / reduced dims, slowest first
+  for (int k = 0; k < n; ++k) {
+    const int64_t d = order[k];
+    if (!g.empty() && g.back().first == (bool)red[d]) g.back().second *= x.size(d);
+    else g.emplace_back((bool)red[d], x.size(d));
+  }
+  if (g.empty() || g.size() > 3) return p;
+  if (g.size() == 1 && g[0].first) g.insert(g.begin(), std::make_pair(false, int64_t(1)));  // one row
+  else if (g.size() == 1) g.emplace_back(true, int64_t(1));
+  const bool first = g[0].first;
+  if (g.size() == 2 && !first) {  // [K, R]
+    p.kind = DimPlan::kSegments;
+    p.outer = g[0].second;
+    p.len = p.row_stride = g[1].second;
+  } else if (g.size() == 3 && first) {  // [R, K, R]
+    p.kind = DimPlan::kSegments;
+    p.segs = g[0].second;
+    p.outer = g[1].second;
+    p.len = p.row_stride = g[2].second;
+    p.seg_stride = p.outer * p.len;
+  } else {  // [R, K] or [K, R, K]
+    p.kind = DimPlan::kCols;
+    if (!first) p.outer = g[0].second;
+    p.red = g[first ? 0 : 1].second;
+    p.inner = g.back().second;
+  }
+  constexpr int64_t lim = int64_t(1) << 31;  // 32-bit rows, runs and positions
+  if (p.outer >= lim || p.outer * p.inner >= lim || p.segs * p.len >= lim) p.kind = DimPlan::kNone;
+  return p;
+}
+
 at::Tensor& sum_mean_into(const at::Tensor& self, at::OptionalIntArrayRef dim, bool keepdim,
                           std::optional<c10::ScalarType> dtype, bool mean, at::Tensor& out, const char* name) {
   c10::ScalarType acc_dt = dtype.value_or(self.scalar_type());
@@ -153,16 +215,42 @@ at::Tensor& sum_mean_into(const at::Tensor& self, at::OptionalIntArrayRef dim, b
     if (!res.is_same(out)) out.copy_(res.reshape(out.sizes()));
     return out;
   }
-  // move the reduced dims last, make rows contiguous, reduce each row
-  std::vector<int64_t> perm;
-  for (int64_t i = 0; i < x.dim(); ++i)
-    if (!red[i]) perm.push_back(i);
-  for (int64_t d : dims) perm.push_back(d);
-  at::Tensor rows = x.permute(perm).contiguous();
-  const int64_t outer = rows.numel() / nred;
-  at::Tensor res = out.is_contiguous() ? out : empty_supa(oshape, acc_dt, self.device().index());
-  const int rc = supa_amd_sum_rows(rows.data_ptr(), dtype_code(rows.scalar_type()), res.data_ptr(),
-                                   dtype_code(acc_dt), outer, nred, scale, current_stream(self.device().index()));
+  // an out= that shares x's storage gets its values after x is read
+  at::Tensor res = out.is_contiguous() && !out.is_alias_of(x) ? out : empty_supa(oshape, acc_dt, self.device().index());
+  DimPlan p = dim_plan(x, red);
+  at::Tensor src = x;
+  if (p.kind == DimPlan::kNone) {
+    // some other order: move the reduced dims last and make rows contiguous
+    std::vector<int64_t> perm;
+    for (int64_t i = 0; i < x.dim(); ++i)
+      if (!red[i]) perm.push_back(i);
+    for (int64_t d : dims) perm.push_back(d);
+    src = x.permute(perm).contiguous();
+    if (nred >= (int64_t(1) << 31)) {
+      check_status(supa_amd_sum_rows(src.data_ptr(), dtype_code(src.scalar_type()), res.data_ptr(), dtype_code(acc_dt),
+                                     src.numel() / nred, nred, scale, current_stream(self.device().index())),
+                   name);
+      if (!res.is_same(out)) out.copy_(res);
+      return out;
+    }
+    p = DimPlan();
+    p.kind = DimPlan::kSegments;
+    p.outer = src.numel() / nred;
+    p.len = p.row_stride = nred;
+  }
+  const int it = dtype_code(src.scalar_type()), ot = dtype_code(acc_dt);
+  void* const st = current_stream(self.device().index());
+  const int64_t wsb = p.kind == DimPlan::kCols
+                          ? supa_amd_sum_cols_workspace_bytes(it, ot, p.outer, p.red, p.inner)
+                          : supa_amd_sum_segments_workspace_bytes(it, ot, p.outer, p.segs, p.len);
+  at::Tensor ws;
+  if (wsb > 0) ws = empty_supa({wsb}, at::kByte, self.device().index());
+  void* const wp = wsb > 0 ? ws.data_ptr() : nullptr;
+  const int rc = p.kind == DimPlan::kCols
+                     ? supa_amd_sum_cols(src.data_ptr(), it, res.data_ptr(), ot, p.outer, p.red, p.inner, scale, wp,
+                                         wsb, st)
+                     : supa_amd_sum_segments(src.data_ptr(), it, res.data_ptr(), ot, p.outer, p.segs, p.len,
+                                             p.row_stride, p.seg_stride, scale, wp, wsb, st);
   check_status(rc, name);
   if (!res.is_same(out)) out.copy_(res);
   return out;

@@ -403,19 +403,6 @@ struct SmoothL1TermEwFactory {
   }
 };
 
-// ---------------------------------------------------------------- rows
-template <typename T, typename OT, typename ACC>
-__global__ void __launch_bounds__(kBlock)
-k_sum_rows(const T* __restrict__ in, OT* __restrict__ out, int64_t inner, ACC scale) {
-  __shared__ ACC lds[kBlock / 64];
-  const T* row = in + (int64_t)blockIdx.x * inner;
-  ACC acc = fold_strided<8>(
-      ACC(0), threadIdx.x, kBlock, inner, [&](int64_t i) { return (ACC)to_arith(row[i]); },
-      [](ACC a, ACC b) { return a + b; });
-  acc = block_sum<kBlock, ACC>(acc, lds);
-  if (threadIdx.x == 0) out[blockIdx.x] = from_arith<OT>(acc * scale);
-}
-
 }  // namespace sa
 
 using namespace sa;
@@ -477,49 +464,6 @@ int supa_amd_sum_noalloc(const supa_amd_ew_desc* d, double scale, void* stream) 
   const int rc = noalloc_scratch(&ws);
   if (rc != SUPA_AMD_OK) return rc;
   return run_reduce(IdentityFactory{}, d, scale, ws, kNoAllocScratchBytes, stream);
-}
-
-int supa_amd_sum_rows(const void* in, int32_t in_dtype, void* out, int32_t out_dtype, int64_t outer, int64_t inner,
-                      double scale, void* stream) {
-  if (!in || !out || outer < 0 || inner <= 0 || outer >= (int64_t(1) << 31)) return SUPA_AMD_EINVAL;
-  if (outer == 0) return SUPA_AMD_OK;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  auto go = [&](auto* ti, auto* to) -> int {
-    using T = std::remove_pointer_t<decltype(ti)>;
-    using OT = std::remove_pointer_t<decltype(to)>;
-    using ACC = typename std::conditional<
-        std::is_integral<OT>::value, int64_t,
-        typename std::conditional<std::is_same<T, double>::value || std::is_same<OT, double>::value, double,
-                                  float>::type>::type;
-    k_sum_rows<T, OT, ACC><<<(unsigned)outer, kBlock, 0, st>>>(static_cast<const T*>(in), static_cast<OT*>(out), inner,
-                                                              (ACC)scale);
-    return launch_status();
-  };
-  auto outsel = [&](auto* ti) -> int {
-    switch (out_dtype) {
-      case SUPA_AMD_F32: return go(ti, (float*)nullptr);
-      case SUPA_AMD_BF16: return go(ti, (bf16*)nullptr);
-      case SUPA_AMD_F16: return go(ti, (f16*)nullptr);
-      case SUPA_AMD_F64: return go(ti, (double*)nullptr);
-      default: return SUPA_AMD_EDTYPE;
-    }
-  };
-  auto intsel = [&](auto* ti) -> int {
-    return out_dtype == SUPA_AMD_I64 ? go(ti, (int64_t*)nullptr) : SUPA_AMD_EDTYPE;
-  };
-  switch (in_dtype) {
-    case SUPA_AMD_F32: return outsel((float*)nullptr);
-    case SUPA_AMD_BF16: return outsel((bf16*)nullptr);
-    case SUPA_AMD_F16: return outsel((f16*)nullptr);
-    case SUPA_AMD_F64: return outsel((double*)nullptr);
-    case SUPA_AMD_BOOL: return intsel((b8*)nullptr);
-    case SUPA_AMD_U8: return intsel((uint8_t*)nullptr);
-    case SUPA_AMD_I8: return intsel((int8_t*)nullptr);
-    case SUPA_AMD_I16: return intsel((int16_t*)nullptr);
-    case SUPA_AMD_I32: return intsel((int32_t*)nullptr);
-    case SUPA_AMD_I64: return intsel((int64_t*)nullptr);
-    default: return SUPA_AMD_EDTYPE;
-  }
 }
 
 int supa_amd_loss_forward(const supa_amd_ew_desc* d, int loss, int reduction, double beta, int has_pos_weight,
