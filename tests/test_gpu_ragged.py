@@ -1,0 +1,80 @@
+"""Elementwise ops over runs whose length is no multiple of the vector, at any
+alignment: bias broadcasts, slices of rows, misaligned views, in-place forms."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def seeded(shape, seed, dtype=torch.float32):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def exact(got, want):
+    assert got.shape == want.shape and got.dtype == want.dtype
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cols", [1, 3, 4, 5, 7, 8, 9, 15, 17, 255, 1021])
+def test_broadcasts_over_odd_runs(cols, dtype, no_fallback):
+    x, row, col = seeded((37, cols), 1, dtype), seeded((cols,), 2, dtype), seeded((37, 1), 3, dtype)
+    dx, drow, dcol = x.to("supa"), row.to("supa"), col.to("supa")
+    exact(dx + drow, x + row)
+    exact(dx * dcol, x * col)
+    exact(drow - dx, row - x)
+    exact(torch.where(dx > dcol, dx, drow), torch.where(x > col, x, row))
+    if dtype != torch.float32:
+        exact(dx + drow.float(), x + row.float())
+    y = seeded((5, 7, cols), 4, dtype)
+    ch = seeded((7, 1), 5, dtype)
+    exact(y.to("supa") + ch.to("supa"), y + ch)
+    z = dx.clone()
+    z += drow  # in place over overlapping vectors
+    z *= 2
+    exact(z, (x + row) * 2)
+    m = seeded((cols,), 6) > 0
+    exact(dx.masked_fill(m.to("supa"), -3.5), x.masked_fill(m, -3.5))
+    exact(dx.masked_fill((dx > 0), 1), x.masked_fill(x > 0, 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.bool, torch.uint8])
+@pytest.mark.parametrize("off", [1, 3, 7])
+def test_misaligned_and_sliced(off, dtype, no_fallback):
+    n = 1003
+    base = (seeded((6, n + 8), 7) * 3).to(dtype)
+    db = base.to("supa")
+    for v, dv in ((base[:, off:off + n], db[:, off:off + n]), (base.view(-1)[off:off + 5000], db.view(-1)[off:off + 5000]),
+                  (base[::2, off:], db[::2, off:])):
+        exact(dv.clone(), v.clone())
+        exact(dv.contiguous(), v.contiguous())
+        if dtype.is_floating_point:
+            exact(dv * 2 + dv, v * 2 + v)
+            exact(torch.relu(dv), torch.relu(v))
+            w = torch.zeros_like(db)
+            wv = w[:, off:off + n]
+            if dv.shape == wv.shape:
+                wv.copy_(dv)  # a misaligned destination
+                exact(w[:, off:off + n].contiguous(), v.contiguous())
+                assert (w[:, :off] == 0).all().item() and (w[:, off + n:] == 0).all().item()
+    h = base[:, :n - 1].chunk(2, -1)
+    dh = db[:, :n - 1].chunk(2, -1)
+    exact(torch.cat(dh, -1), torch.cat(h, -1))
+
+
+def test_masked_fill_shapes_and_errors(no_fallback):
+    x = seeded((4, 1, 6), 8)
+    m = seeded((5, 6), 9) > 0
+    got = x.to("supa").masked_fill(m.to("supa"), float("-inf"))
+    exact(got, x.masked_fill(m, float("-inf")))
+    assert got.is_contiguous()
+    exact(x.to("supa").masked_fill(m.to("supa"), torch.tensor(2.0)), x.masked_fill(m, torch.tensor(2.0)))
+    i = torch.arange(12).view(3, 4)
+    exact(i.to("supa").masked_fill(i.to("supa") > 5, -1), i.masked_fill(i > 5, -1))
+    with pytest.raises(RuntimeError, match="boolean masks"):
+        x.to("supa").masked_fill(x.to("supa"), 1.0)
+    p = x.to("supa").requires_grad_()
+    p.masked_fill(m.to("supa"), 0.0).sum().backward()
+    q = x.clone().requires_grad_()
+    q.masked_fill(m, 0.0).sum().backward()
+    exact(p.grad, q.grad)

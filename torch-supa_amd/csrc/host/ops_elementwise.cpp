@@ -992,11 +992,14 @@ at::Tensor& where_self_out(const at::Tensor& c, const at::Tensor& a, const at::T
 }
 
 // masked_fill_: self = mask ? value : self, the mask broadcast to self.
-at::Tensor& masked_fill_s(at::Tensor& self, const at::Tensor& mask, const c10::Scalar& value) {
+void check_fill_mask(const at::Tensor& self, const at::Tensor& mask) {
   TORCH_CHECK(mask.scalar_type() == at::kBool, "masked_fill_ only supports boolean masks, but got mask with dtype ",
               mask.scalar_type());
   TORCH_CHECK(self.device() == mask.device(), "expected self and mask to be on the same device, but got mask on ",
               mask.device(), " and self on ", self.device());
+}
+at::Tensor& masked_fill_s(at::Tensor& self, const at::Tensor& mask, const c10::Scalar& value) {
+  check_fill_mask(self, mask);
   ew_apply(self, self.scalar_type(), self.scalar_type(), {EwIn::of(mask), EwIn::num(value), EwIn::of(self)},
            where_launch(), "masked_fill_");
   return self;
@@ -1005,6 +1008,20 @@ at::Tensor& masked_fill_t(at::Tensor& self, const at::Tensor& mask, const at::Te
   TORCH_CHECK(value.dim() == 0, "masked_fill_ only supports a 0-dimensional value tensor, but got tensor with ",
               value.dim(), " dimension(s).");
   return masked_fill_s(self, mask, value.item());
+}
+// masked_fill: the contiguous result written in one pass (upstream's composite
+// clones self and fills the clone: bf16 [64, 1048576] 46 us of copy more).
+at::Tensor masked_fill_new_s(const at::Tensor& self, const at::Tensor& mask, const c10::Scalar& value) {
+  check_fill_mask(self, mask);
+  const at::Tensor out = empty_supa(at::infer_size(mask.sizes(), self.sizes()), self.scalar_type(),
+                                    self.device().index());
+  return ew_apply(out, self.scalar_type(), self.scalar_type(), {EwIn::of(mask), EwIn::num(value), EwIn::of(self)},
+                  where_launch(), "masked_fill");
+}
+at::Tensor masked_fill_new_t(const at::Tensor& self, const at::Tensor& mask, const at::Tensor& value) {
+  TORCH_CHECK(value.dim() == 0, "masked_fill_ only supports a 0-dimensional value tensor, but got tensor with ",
+              value.dim(), " dimension(s).");
+  return masked_fill_new_s(self, mask, value.item());
 }
 
 // ------------------------------------------------ parameterised activations
@@ -1416,6 +1433,8 @@ TORCH_LIBRARY_IMPL(aten, PrivateUse1, m) {
   m.impl("isnan", TORCH_FN(isnan_t));
   m.impl("where.self", TORCH_FN(where_self));
   m.impl("where.self_out", TORCH_FN(where_self_out));
+  m.impl("masked_fill.Scalar", TORCH_FN(masked_fill_new_s));
+  m.impl("masked_fill.Tensor", TORCH_FN(masked_fill_new_t));
   m.impl("masked_fill_.Scalar", TORCH_FN(masked_fill_s));
   m.impl("masked_fill_.Tensor", TORCH_FN(masked_fill_t));
   m.impl("leaky_relu", TORCH_FN(leaky_relu));

@@ -6,12 +6,14 @@
 //           dim, stride 1) or a one-element broadcast (stride 0).  Each thread
 //           moves one 16-byte vector per operand, in one-wavefront
 //           workgroups; the tail (< VEC elements) goes to the last one.
-//   VECND   N-d iteration whose innermost dim is a multiple of VEC and where
-//           every operand's innermost stride is 1 (vector load) or 0 (one
-//           element broadcast across the vector).  Coordinates of a vector's
+//   VECND   N-d iteration where every operand's innermost stride is 1 (vector
+//           load, at any alignment) or 0 (one element broadcast across the
+//           vector) and the innermost dim holds at least one vector; a last
+//           short vector ends at the dim's end.  Coordinates of a vector's
 //           first element come from a chain of magic-number divisions; this
-//           covers a bias broadcast along rows, a per-row scalar broadcast
-//           and inputs that are permuted but dense.
+//           covers a bias broadcast along rows of any width, a per-row scalar
+//           broadcast, slices of rows, misaligned views and inputs that are
+//           permuted but dense.
 //   ROW2D   two dims (or three, rows flattened), dense output, each input
 //           dense / row-broadcast / column-broadcast / middle-dim-broadcast /
 //           one element: bias adds without the divider chain and 64-bit
@@ -40,6 +42,7 @@
 #include "divmod.h"
 #include "dtypes.h"
 #include "supa_amd.h"
+#include "unaligned.h"
 
 namespace sa {
 
@@ -83,6 +86,20 @@ template <typename Op> struct DtypeModeOf<Op, std::void_t<decltype(Op::kDtypeMod
   static constexpr int value = Op::kDtypeMode;
 };
 
+// y = x with v inserted at position k.  Selects between fixed elements: a
+// running index into x (uniform, but unknown to the compiler) put every
+// thread's inputs in scratch memory (masked_fill_ of bf16 [64, 1048576] by a
+// [1048576] mask 163 us, 46 now).
+template <int A, typename C>
+__device__ __forceinline__ void bind_inputs(C (&y)[A], const C* x, int k, C v) {
+#pragma unroll
+  for (int i = 0; i < A; ++i) {
+    const C before = i < A - 1 ? x[i < A - 1 ? i : 0] : v;  // k > i
+    const C after = i > 0 ? x[i > 0 ? i - 1 : 0] : v;       // k < i
+    y[i] = i == k ? v : (i < k ? before : after);
+  }
+}
+
 template <typename Op, typename C>
 struct Bind1 {  // binds input position K to value v
   static constexpr int arity = Op::arity - 1;
@@ -92,15 +109,7 @@ struct Bind1 {  // binds input position K to value v
   C v;
   __device__ __forceinline__ C operator()(const C* x) const {
     C y[Op::arity];
-#pragma unroll
-    for (int i = 0, j = 0; i < Op::arity; ++i) {
-      if (i == k) {
-        y[i] = v;
-      } else {
-        y[i] = x[j];
-        ++j;
-      }
-    }
+    bind_inputs<Op::arity>(y, x, k, v);
     return op(y);
   }
 };
@@ -119,15 +128,7 @@ struct BindDev1 {
   __device__ __forceinline__ C operator()(const C* x) const {
     const C v = load_cvt<C, CT>(*p);
     C y[Op::arity];
-#pragma unroll
-    for (int i = 0, j = 0; i < Op::arity; ++i) {
-      if (i == k) {
-        y[i] = v;
-      } else {
-        y[i] = x[j];
-        ++j;
-      }
-    }
+    bind_inputs<Op::arity>(y, x, k, v);
     return op(y);
   }
 };
@@ -143,7 +144,7 @@ template <int NT>  // NT = number of tensor operands (output first)
 struct TArgs {
   void* p[NT];
   int64_t st[NT][SUPA_AMD_MAX_DIMS];
-  int32_t mode[NT];  // CONTIG: 0 dense, 1 one-element broadcast; VECND: 1 = re-read (broadcast) operand
+  int32_t mode[NT];  // CONTIG: 0 dense, 1 one-element broadcast; VECND: 1 = broadcast (re-read) operand
 };
 
 // ------------------------------------------------------- type plumbing
@@ -326,7 +327,20 @@ k_contig(Op op, TArgs<1 + sizeof...(S)> a, int64_t n, uint32_t nfull) {
 // OFF: the offset type, int32_t when the host has checked that every
 // operand's largest offset fits (one 32-bit multiply per dim and operand
 // instead of a 64-bit product), int64_t otherwise.
-template <int VEC, typename OFF, typename Op, typename C, typename CT, typename OT, typename... S>
+// g.div[0] divides by the vectors of an innermost run, ceil(inner / VEC); the
+// last vector of a run whose length is no multiple of VEC is moved back to
+// end at the run's end and stores only the elements no other vector covers
+// (so an output may still be an input).  Every access is at element
+// alignment.  Runs of odd length took one element per thread (k_strided)
+// before: [6007, 2047] + a row in float32 43.4 us, 17.0 now, in bf16 43.4, 9.6;
+// [5843, 8821] slices of odd rows in bf16: silu 173 us, 41 now, a product 173, 52.
+// Loads take no streaming hint: a run's ends share cache lines with its
+// neighbours and one-stream ops gain from what the last level still holds
+// (float32 silu of [4096, 11008] row slices 48.6 us, 55.9 with the hint; bf16
+// [32768, 4095] + a row 103, 119).  WHOLE is the variant for whole vectors
+// and two or more full-size inputs, which are streamed (those slices times a
+// dense tensor 82.0 us, 89.0 without the hint; bf16 41.2, 41.5).
+template <int VEC, typename OFF, bool WHOLE, typename Op, typename C, typename CT, typename OT, typename... S>
 __global__ void __launch_bounds__(kStreamBlock)
 k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
   constexpr int N = sizeof...(S);
@@ -334,7 +348,13 @@ k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
   if (v >= nvec) return;
   // coordinates of the vector's first element
   uint32_t q, r;
-  g.div[0].divmod(v * VEC, q, r);
+  g.div[0].divmod(v, q, r);
+  r *= VEC;
+  uint32_t skip = 0;
+  if (!WHOLE && r + VEC > g.size[0]) {
+    skip = r + VEC - g.size[0];
+    r = g.size[0] - VEC;
+  }
   OFF off[1 + N];
 #pragma unroll
   for (int k = 0; k <= N; ++k) off[k] = (OFF)r * (OFF)a.st[k][0];
@@ -355,8 +375,14 @@ k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
 #pragma unroll
          for (int k = 0; k < VEC; ++k) x[k][I] = s;
        } else {
-         const Vec<St, VEC> w = a.mode[1 + I] ? *reinterpret_cast<const Vec<St, VEC>*>(p)
-                                              : ld_stream(reinterpret_cast<const Vec<St, VEC>*>(p));
+         Vec<St, VEC> w;
+         if (!WHOLE || a.mode[1 + I]) {
+           if (WHOLE) asm volatile("");  // or the two loads become one, without the hint
+           w = ld_vec_any<false, St, VEC>(p);
+           if (WHOLE) asm volatile("");
+         } else {
+           w = ld_vec_any<true, St, VEC>(p);
+         }
 #pragma unroll
          for (int k = 0; k < VEC; ++k) x[k][I] = load_cvt<C, CT>(w.v[k]);
        }
@@ -366,7 +392,14 @@ k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
   Vec<OT, VEC> w;
 #pragma unroll
   for (int k = 0; k < VEC; ++k) w.v[k] = from_arith<OT>(op(x[k]));
-  st_stream(reinterpret_cast<Vec<OT, VEC>*>(static_cast<OT*>(a.p[0]) + off[0]), w);
+  OT* dst = static_cast<OT*>(a.p[0]) + off[0];
+  if (WHOLE || skip == 0) {
+    st_vec_any<OT, VEC>(dst, w);
+  } else {
+#pragma unroll
+    for (int k = 0; k < VEC; ++k)
+      if (k >= (int)skip) dst[k] = w.v[k];
+  }
 }
 
 // ------------------------------------------------------------- ROW2D

@@ -307,29 +307,43 @@ int launch_static(const Op& op, const supa_amd_ew_desc& d, const int* tin, hipSt
       for (int j = 0; j < p.ndim; ++j) mx += (p.sizes[j] - 1) * (b.st[k][j] < 0 ? -b.st[k][j] : b.st[k][j]);
       if (mx >= (int64_t(1) << 31)) off32 = false;
     }
-    // VECND?
-    bool vnd = p.ndim >= 1 && (p.sizes[0] % VEC) == 0 && b.st[0][0] == 1 && VEC > 1;
-    for (int k = 0; k <= N && vnd; ++k) {
-      const int64_t s0 = b.st[k][0];
-      if (s0 != 0 && s0 != 1) { vnd = false; break; }
-      if (s0 == 1) {
-        if (!aligned(b.p[k], VEC * sizes_of[k])) vnd = false;
-        for (int j = 1; j < p.ndim; ++j)
-          if (b.st[k][j] % VEC) vnd = false;
-      }
-    }
+    // VECND?  At least one vector a run, more runs than vectors fit 32 bits.
+    const int64_t ivec = VEC > 1 && p.ndim >= 1 ? (p.sizes[0] + VEC - 1) / VEC : 0;
+    const int64_t nvec64 = ivec ? ivec * (pn / p.sizes[0]) : 0;
+    bool vnd = VEC > 1 && p.ndim >= 1 && p.sizes[0] >= VEC && b.st[0][0] == 1 && nvec64 < (int64_t(1) << 31);
+    for (int k = 1; k <= N && vnd; ++k) vnd = b.st[k][0] == 0 || b.st[k][0] == 1;
     if (vnd) {
-      // operands broadcast along some outer dim are re-read: keep them cached
+      // operands broadcast along some outer dim are re-read: never streamed
+      int streams = 0;
       for (int k = 1; k <= N; ++k) {
-        b.mode[k] = 0;
+        b.mode[k] = b.st[k][0] == 0 ? 1 : 0;
         for (int j = 1; j < p.ndim; ++j)
           if (b.st[k][j] == 0 && p.sizes[j] > 1) b.mode[k] = 1;
+        streams += b.mode[k] ? 0 : 1;
       }
-      const uint32_t nvec = (uint32_t)(pn / VEC);
+      const bool whole = p.sizes[0] % VEC == 0 && streams >= 2;
+      NdGeom gv = g;
+      gv.div[0] = FastDiv((uint32_t)ivec);
+      const uint32_t nvec = (uint32_t)nvec64;
       const unsigned blocks = (nvec + kStreamBlock - 1) / kStreamBlock;
-      if (off32) k_vecnd<VEC, int32_t, Op, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(op, b, g, nvec);
-      else k_vecnd<VEC, int64_t, Op, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(op, b, g, nvec);
-      return launch_status();
+      auto go = [&](const auto& o) -> int {
+        using O = std::remove_cv_t<std::remove_reference_t<decltype(o)>>;
+        if constexpr (N >= 2) {
+          if (off32 && whole) {
+            k_vecnd<VEC, int32_t, true, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
+            return launch_status();
+          }
+        }
+        if (off32) k_vecnd<VEC, int32_t, false, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
+        else k_vecnd<VEC, int64_t, false, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
+        return launch_status();
+      };
+      if constexpr (IsRowB<Op>::value) {
+        // the functor's rounding and mean switches fixed at compile time, as for ROWB
+        constexpr int kRt = std::is_same<OT, bf16>::value ? 1 : (std::is_same<OT, f16>::value ? 2 : 0);
+        if (op.rt == kRt) return op.mean ? go(op.template fixed<kRt, 1>()) : go(op.template fixed<kRt, 0>());
+      }
+      return go(op);
     }
     const unsigned blocks = (unsigned)((pn + kStreamBlock - 1) / kStreamBlock);
     if (off32) k_strided<int32_t, Op, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(op, b, g, (uint32_t)pn);
