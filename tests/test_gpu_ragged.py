@@ -1,7 +1,9 @@
-"""Elementwise ops over runs whose length is no multiple of the vector, at any
-alignment: bias broadcasts, slices of rows, misaligned views, in-place forms."""
+"""Elementwise ops and full reductions over runs whose length is no multiple of
+the vector, at any alignment: bias broadcasts, slices of rows, misaligned
+views, in-place forms, and the losses over them."""
 import pytest
 import torch
+import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +80,21 @@ def test_masked_fill_shapes_and_errors(no_fallback):
     q = x.clone().requires_grad_()
     q.masked_fill(m, 0.0).sum().backward()
     exact(p.grad, q.grad)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("cols", [1, 3, 5, 8, 13, 8193])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+def test_losses_over_odd_runs(cols, dtype, reduction, no_fallback):
+    x, t, pw = seeded((19, cols), 10, dtype), (seeded((19, cols), 11) > 0).to(dtype), seeded((cols,), 12, dtype).abs() + 0.5
+    dx = x.to("supa").requires_grad_()
+    cx = x.double().requires_grad_()
+    loss = F.binary_cross_entropy_with_logits(dx, t.to("supa"), pos_weight=pw.to("supa"), reduction=reduction)
+    want = F.binary_cross_entropy_with_logits(cx, t.double(), pos_weight=pw.double(), reduction=reduction)
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    torch.testing.assert_close(loss.detach().cpu().double(), want.detach(), rtol=tol, atol=tol)
+    loss.sum().backward()
+    want.sum().backward()
+    torch.testing.assert_close(dx.grad.cpu().double(), cx.grad, rtol=tol, atol=tol / max(1, x.numel() if reduction == "mean" else 1))
+    torch.testing.assert_close(F.mse_loss(dx.detach(), t.to("supa"), reduction=reduction).cpu().double(),
+                               F.mse_loss(x.double(), t.double(), reduction=reduction), rtol=tol, atol=tol)

@@ -91,10 +91,16 @@ __device__ __forceinline__ ACC accumulate(const Op& op, const TArgs<1 + sizeof..
       acc += (ACC)op(y);
     }
   } else if constexpr (LAYOUT == R_VECND) {
-    const uint32_t nvec = (uint32_t)(n / VEC);
+    const uint32_t nvec = g.div[0].d * (uint32_t)(n / g.size[0]);
     for (uint32_t v = (uint32_t)tid; v < nvec; v += (uint32_t)nthreads) {
       uint32_t q, r;
-      g.div[0].divmod(v * VEC, q, r);
+      g.div[0].divmod(v, q, r);  // vectors of a run
+      r *= VEC;
+      uint32_t skip = 0;  // a run's last vector ends at its end; the elements another one holds do not count
+      if (r + VEC > g.size[0]) {
+        skip = r + VEC - g.size[0];
+        r = g.size[0] - VEC;
+      }
       int64_t off[1 + N];
 #pragma unroll
       for (int k = 0; k <= N; ++k) off[k] = (int64_t)r * a.st[k][0];
@@ -115,16 +121,20 @@ __device__ __forceinline__ ACC accumulate(const Op& op, const TArgs<1 + sizeof..
 #pragma unroll
              for (int k = 0; k < VEC; ++k) x[k][I] = s;
            } else {
-             const Vec<St, VEC> w = (BC && a.mode[1 + I]) ? *reinterpret_cast<const Vec<St, VEC>*>(p)
-                                                          : ld_stream(reinterpret_cast<const Vec<St, VEC>*>(p));
+             const Vec<St, VEC> w = ld_vec_any<!BC, St, VEC>(p);
 #pragma unroll
              for (int k = 0; k < VEC; ++k) x[k][I] = load_cvt<C, CT>(w.v[k]);
            }
          }()),
          ...);
       }(std::make_integer_sequence<int, N>{});
+      if (skip == 0) {
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) acc += (ACC)op(x[k]);
+        for (int k = 0; k < VEC; ++k) acc += (ACC)op(x[k]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc += k >= (int)skip ? (ACC)op(x[k]) : ACC(0);
+      }
     }
   } else {
     for (uint32_t i = (uint32_t)tid; i < (uint32_t)n; i += (uint32_t)nthreads) {
@@ -212,16 +222,9 @@ int launch_reduce(const Op& op, const supa_amd_ew_desc& d, const int* tin, doubl
   if (contig) layout = R_CONTIG;
   if (layout != R_CONTIG) {
     if (n >= (int64_t(1) << 31)) return SUPA_AMD_ELAYOUT;
-    bool vnd = VEC > 1 && d.ndim >= 1 && (d.sizes[0] % VEC) == 0;
-    for (int i = 0; i < N && vnd; ++i) {
-      const int64_t s0 = a.st[1 + i][0];
-      if (s0 != 0 && s0 != 1) vnd = false;
-      if (s0 == 1) {
-        if (!aligned(a.p[1 + i], VEC * sizes_of[i])) vnd = false;
-        for (int j = 1; j < d.ndim; ++j)
-          if (a.st[1 + i][j] % VEC) vnd = false;
-      }
-    }
+    // runs of any length (from one vector on) at any alignment
+    bool vnd = VEC > 1 && d.ndim >= 1 && d.sizes[0] >= VEC;
+    for (int i = 0; i < N && vnd; ++i) vnd = a.st[1 + i][0] == 0 || a.st[1 + i][0] == 1;
     layout = vnd ? R_VECND : R_STRIDED;
     if (vnd) {
       // operands broadcast along an outer dim are re-read: keep them cached
@@ -232,7 +235,8 @@ int launch_reduce(const Op& op, const supa_amd_ew_desc& d, const int* tin, doubl
       }
     }
   }
-  const NdGeom g = make_geom(d);
+  NdGeom g = make_geom(d);
+  if (layout == R_VECND) g.div[0] = FastDiv((uint32_t)((d.sizes[0] + VEC - 1) / VEC));
   const int64_t units = layout == R_STRIDED ? n : std::max<int64_t>(n / VEC, 1);
   const int64_t want = (units + 4 * kRedBlock - 1) / (4 * kRedBlock);
   const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, kRedBlocks));
