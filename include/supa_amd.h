@@ -705,6 +705,14 @@ int supa_amd_moments_rows(const void* in, int32_t dtype, int64_t outer, int64_t 
                           int take_sqrt, void* out_var, void* out_mean, void* workspace, int64_t ws_bytes,
                           void* stream);
 
+/* The same over rows made of runs: row r's `segs` runs of `len` contiguous
+ * elements, run s at element r * row_stride + s * seg_stride (a channel's
+ * planes over a batch), read where they lie. */
+int64_t supa_amd_moments_segments_workspace_bytes(int64_t rows, int64_t segs, int64_t len, int32_t dtype);
+int supa_amd_moments_segments(const void* in, int32_t dtype, int64_t rows, int64_t segs, int64_t len,
+                              int64_t row_stride, int64_t seg_stride, double correction, int take_sqrt, void* out_var,
+                              void* out_mean, void* workspace, int64_t ws_bytes, void* stream);
+
 /* Mixed-precision gradient unscale: every element of the `ntensors`
  * contiguous tensors (f32 / bf16 / f16 / f64) is multiplied in place by
  * *inv_scale (left as is when that is exactly 1), and *found_inf (device

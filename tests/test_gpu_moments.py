@@ -113,3 +113,21 @@ def test_integer_input_takes_the_counted_fallback(supa):
     with pytest.raises(RuntimeError, match="floating point"):
         torch.var(torch.tensor([1, 2, 3, 4, 5]).to("supa"))
     assert supa.supa.fallback_counts().get("aten::var.correction", 0) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("vecs", [1, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 4097])
+def test_moments_at_the_edges_of_a_chunk(dtype, vecs, no_fallback):
+    """The longest row of each thread split and one vector more, with and
+    without a short last vector, as one run and as runs of a channel."""
+    v = 16 // torch.empty(0, dtype=dtype).element_size()
+    for n in (vecs * v, vecs * v - 1):
+        if n < 2:
+            continue
+        x = (torch.randn(5, n, generator=torch.Generator().manual_seed(n)) + 3).to(dtype)
+        runs = x.reshape(5, 1, n)
+        many = (torch.randn(3, 4, n, generator=torch.Generator().manual_seed(n + 1)) - 2).to(dtype)
+        for t, dims in ((runs, (0, 2)), (x, 1), (many, (0, 2))):
+            var, mean = torch.var_mean(t.to("supa"), dim=dims)
+            torch.testing.assert_close(var.cpu().double(), t.double().var(dim=dims), rtol=RTOL[dtype], atol=0)
+            torch.testing.assert_close(mean.cpu().double(), t.double().mean(dim=dims), rtol=RTOL[dtype], atol=0)

@@ -1,8 +1,9 @@
 // PrivateUse1 registrations of var / std / var_mean / std_mean with a
 // correction (what var(unbiased=...), std(), and LayerNorm or BatchNorm
-// written out by hand resolve to).  The reduced dims go last in a contiguous
-// copy and one row kernel returns the variance or standard deviation, and the
-// mean beside it, for every row.  Complex and integer inputs go to the CPU
+// written out by hand resolve to).  The row kernels return the variance or
+// standard deviation, and the mean beside it, for every row; rows that are
+// runs of contiguous elements (trailing dims, a channel's planes) are read
+// where they lie, others through a contiguous copy with the reduced dims last.  Complex and integer inputs go to the CPU
 // fallback, which counts them (upstream raises for integers).
 #include <ATen/WrapDimUtilsMulti.h>
 #include <ATen/native/CPUFallback.h>
@@ -18,6 +19,7 @@
 #include <tuple>
 
 #include "common.h"
+#include "dim_plan.h"
 
 namespace supa {
 namespace {
@@ -72,15 +74,25 @@ MomentsResult moments(const at::Tensor& self, at::OptionalIntArrayRef dim, const
     if (want_mean) r.mean.fill_(std::numeric_limits<double>::quiet_NaN());
     return r;
   }
-  const at::Tensor rows = nd == 0 ? self.reshape({1}) : self.permute(perm).contiguous();
+  std::vector<bool> mask(nd);
+  for (int64_t i = 0; i < nd; ++i) mask[i] = red[i];
+  DimPlan p = dim_plan(self, mask);
+  at::Tensor rows = self;
+  if (p.kind != DimPlan::kSegments) {
+    rows = nd == 0 ? self.reshape({1}) : self.permute(perm).contiguous();
+    p = DimPlan();
+    p.outer = outer;
+    p.len = p.row_stride = inner;
+  }
   const int32_t dt = dtype_code(self.scalar_type());
-  const int64_t ws_bytes = supa_amd_moments_rows_workspace_bytes(outer, inner, dt);
+  const int64_t ws_bytes = supa_amd_moments_segments_workspace_bytes(p.outer, p.segs, p.len, dt);
   TORCH_CHECK(ws_bytes >= 0, name, ": ", supa_amd_status_string((int)ws_bytes));
   at::Tensor ws;
   if (ws_bytes > 0) ws = at::empty({ws_bytes}, opts.dtype(at::kByte));
-  check_status(supa_amd_moments_rows(rows.data_ptr(), dt, outer, inner, corr, take_sqrt ? 1 : 0, r.var.data_ptr(),
-                                     want_mean ? r.mean.data_ptr() : nullptr, ws_bytes > 0 ? ws.data_ptr() : nullptr,
-                                     ws_bytes, current_stream(self.device().index())),
+  check_status(supa_amd_moments_segments(rows.data_ptr(), dt, p.outer, p.segs, p.len, p.row_stride, p.seg_stride, corr,
+                                         take_sqrt ? 1 : 0, r.var.data_ptr(), want_mean ? r.mean.data_ptr() : nullptr,
+                                         ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
+                                         current_stream(self.device().index())),
                name);
   return r;
 }

@@ -1,40 +1,39 @@
-// Variance / standard deviation (and the mean beside them) along the last
-// dim of a contiguous [outer, inner] input: var / std / var_mean / std_mean
+// Variance / standard deviation (and the mean beside them) of rows made of
+// runs of contiguous elements (segments.h): var / std / var_mean / std_mean
 // with a correction, which LayerNorm and BatchNorm written by hand, and
 // normalisation statistics, call next to the loss path.
 //
-// Welford's running (count, mean, M2) per thread over a strided walk, merged
-// pairwise by Chan et al.'s update (wavefront shuffles, then LDS); the
-// result is M2 / max(0, count - correction), its square root for std.
-// Upstream's device reduction (WelfordOps in SharedReduceOps.h) accumulates
-// the same triple, so a NaN propagates and a row with count <= correction
-// divides by zero (inf or NaN) as it does there.  Every value is first
-// shifted by its row's first element K (the shifted-data algorithm): the
-// triple then tracks mean - K, which keeps its precision when the mean is
-// large against the spread (float Welford on unshifted data loses about
-// (ulp(mean) / sigma)^2 of the variance); the mean written out adds K back.
+// HBM-bound: one read of the input.  A chunk of up to 2048 16-byte vectors
+// stays in the registers of the threads that share it (16 lanes or a
+// wavefront, each with whole rows, or a workgroup of 256).  Two passes over
+// the registers: a mean, summed as x (1 / n), then the deviations d from it,
+// with the corrected two-pass formulas mean + sum d / n and M2 = sum d^2 -
+// (sum d)^2 / n: no division per value, and the first mean's rounding drops
+// out, however large the mean against the spread.  Longer rows are cut in such
+// chunks; each chunk's (count, mean - K, M2), K the row's first element (so
+// that the means keep their precision when they are merged), goes to the
+// workspace and a second launch merges a row's triples by Chan et al.'s
+// update.  The result is M2 / max(0, count - correction), its square root for
+// std; a NaN propagates and a row with count <= correction divides by zero
+// (inf or NaN), as upstream's device reduction (WelfordOps in
+// SharedReduceOps.h) does.
 //
-// Each thread takes its values eight at a time: the batch's own triple
-// (its mean, and the squared deviations from it, in registers) merges into
-// the running one, one division per batch instead of one per value.
-//
-// One workgroup per (row, chunk of `chunk` elements): a single wavefront for
-// rows up to kMomWaveRow elements (no LDS stage; more rows in flight per CU),
-// four for longer ones.  Long rows with few of them take two launches: the
-// first writes one triple per chunk into the workspace, the second merges
-// each row's triples.
+// Measured on MI355X, us, before (Welford triples per thread, one element a
+// load; planes copied to rows first) -> now: float32 [8192, 4096] 28.0 -> 20.5
+// (6.5 TB/s, HBM bound), bf16 25.0 -> 13.6; [65536, 512] 40.7 -> 22.7, bf16
+// 40.2 -> 20.7; [2048, 65536] 141 -> 83; dims (0, 2) of [32, 64, 12544]
+// 73.7 -> 18.7; [64, 512, 49] 26 -> 5.
 //
 // Replaces var.correction_out NF:6629, std.correction_out NF:6088,
 // var_mean.correction NF:6668, std_mean.correction NF:6063 (upstream
 // ReduceMomentKernel.cu: std_var_kernel_cuda over WelfordOps).
-#include "ew_launch.h"
+#include "segments.h"
 
 namespace sa {
 
 constexpr int kMomBlock = 256;
-constexpr int64_t kMomWaveRow = 4096;  // rows up to this length take one-wavefront workgroups
-constexpr int64_t kMomChunk = 16384;    // elements per workgroup in the first of two launches
-constexpr int64_t kMomTwoPass = 65536;  // rows longer than this (with few rows) take two launches
+constexpr int kMomVecs = 8;                                        // most vectors a thread holds
+constexpr uint32_t kMomChunk = (uint32_t)kMomBlock * kMomVecs;     // most vectors a chunk holds
 
 template <typename A> struct Welford {
   A n, mean, m2;
@@ -53,100 +52,173 @@ template <typename A> __device__ __forceinline__ Welford<A> wf_shfl(Welford<A> w
   return {__shfl_xor(w.n, off, 64), __shfl_xor(w.mean, off, 64), __shfl_xor(w.m2, off, 64)};
 }
 
-inline int64_t mom_chunks(int64_t outer, int64_t inner) {
-  return inner > kMomTwoPass && outer < 2048 ? (inner + kMomChunk - 1) / kMomChunk : 1;
+// Sums of two values over the G threads that share a chunk, in every one.
+template <int G, typename A> __device__ __forceinline__ void mom_sum(A& u, A& v, A (*lds)[kMomBlock / 64]) {
+#pragma unroll
+  for (int off = (G < 64 ? G : 64) / 2; off > 0; off >>= 1) {
+    u += __shfl_xor(u, off, 64);
+    v += __shfl_xor(v, off, 64);
+  }
+  if constexpr (G > 64) {
+    if ((threadIdx.x & 63) == 0) {
+      lds[0][threadIdx.x >> 6] = u;
+      lds[1][threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    u = lds[0][0];
+    v = lds[1][0];
+#pragma unroll
+    for (int w = 1; w < G / 64; ++w) {
+      u += lds[0][w];
+      v += lds[1][w];
+    }
+    __syncthreads();  // the slots are free for the next sum
+  }
 }
 
-// TERM: `in` holds elements of T (else the triples of an earlier launch, as
-// three A per chunk).  FINAL: write var-or-std (and the mean) in OT (else the
-// chunk's triple into `part`).
-// K of a row is kin[row * kstride] (the row's first input element, in both
-// launches).
-template <int BS, typename T, typename KT, typename OT, typename A, bool TERM, bool FINAL>
-__global__ void __launch_bounds__(BS)
-k_moments(const void* __restrict__ in, const KT* __restrict__ kin, int64_t kstride, int64_t inner, int64_t chunk,
-          uint32_t nchunks, A correction, int take_sqrt, OT* __restrict__ out_var, OT* __restrict__ out_mean,
-          A* __restrict__ part) {
-  __shared__ Welford<A> lds[BS / 64];
-  const uint32_t row = blockIdx.x / nchunks, c = blockIdx.x % nchunks;
-  const A K = (A)to_arith(kin[(int64_t)row * kstride]);
-  const int64_t lo = (int64_t)c * chunk;
-  const int64_t n = lo + chunk < inner ? chunk : inner - lo;
-  Welford<A> w{A(0), A(0), A(0)};
-  if constexpr (TERM) {
-    const T* src = static_cast<const T*>(in) + (int64_t)row * inner + lo;
-    constexpr int U = 8;
-    for (int64_t i0 = threadIdx.x; i0 < n; i0 += (int64_t)U * BS) {
-      A x[U];
-      int cnt = 0;
-      A sum = A(0);
+template <typename A, typename OT>
+__device__ __forceinline__ void mom_write(Welford<A> w, A correction, int take_sqrt, OT* var, OT* mean) {
+  const A div = w.n > correction ? w.n - correction : A(0);
+  const A v = w.m2 / div;
+  *var = from_arith<OT>(take_sqrt ? sqrt(v) : v);
+  if (mean) *mean = from_arith<OT>(w.mean);
+}
+
+// FINAL: the chunk is the whole row; else its triple goes to part[row nchunks
+// + chunk].
+template <typename T, typename A, int VW, int G, int NV, bool FINAL>
+__global__ void __launch_bounds__(kMomBlock)
+k_moments(const T* __restrict__ in, SegGeom g, FastDiv nch, A correction, int take_sqrt, T* __restrict__ out_var,
+          T* __restrict__ out_mean, A* __restrict__ part) {
+  __shared__ A lds[2][kMomBlock / 64];
+  const int l = threadIdx.x & (G - 1);
+  // G = 256: workgroup b takes chunk b % nch of row b / nch
+  uint32_t wrow = blockIdx.x, c = 0;
+  if constexpr (!FINAL) nch.divmod(blockIdx.x, wrow, c);
+  const int64_t row = G < 256 ? (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G : (int64_t)wrow;
+  if (row >= g.rows) return;
+  const T* src = in + row * g.row_stride;
+  const int64_t lo = (int64_t)c * g.chunk;
+  const int64_t hi = g.nvec - lo < g.chunk ? g.nvec : lo + g.chunk;
+  sum_raw_t<T, VW> x[NV];
+  uint32_t valid[NV];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + (int64_t)u * BS;
-        x[u] = i < n ? (A)to_arith(src[i]) - K : A(0);
-        cnt += i < n ? 1 : 0;
-        sum += x[u];
-      }
-      const A bn = (A)cnt;
-      const A bmean = sum / bn;
-      A bm2 = A(0);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const A d = x[u] - bmean;
-        if (u < cnt) bm2 += d * d;
-      }
-      w = wf_merge(w, Welford<A>{bn, bmean, bm2});
-    }
-  } else {
-    const A* src = static_cast<const A*>(in) + ((int64_t)row * inner + lo) * 3;
-    for (int64_t i = threadIdx.x; i < n; i += BS)
-      w = wf_merge(w, Welford<A>{src[3 * i], src[3 * i + 1], src[3 * i + 2]});
+  for (int j = 0; j < NV; ++j) {
+    valid[j] = 0;
+    if (lo + l + j * G < hi) x[j] = seg_load<T, VW>(src, g, lo + l + j * G, valid[j]);
   }
+  constexpr uint32_t kAll = (1u << VW) - 1u;
+  auto in_row = [&](int j, int k) { return valid[j] == kAll || (valid[j] >> k & 1u); };
+  A count;
+  if constexpr (FINAL) {
+    count = (A)(g.runs * g.len);
+  } else {  // whole vectors but for the runs' ends
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) n += __popc(valid[j]);
+    A dummy = A(0);
+    count = (A)n;
+    mom_sum<G, A>(count, dummy, lds);
+  }
+  const A inv = A(1) / count;
+  A s = A(0), unused = A(0);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    if (valid[j] == 0) continue;
+#pragma unroll
+    for (int k = 0; k < VW; ++k) s = fma(sum_elem<T, VW, A>(x[j], k), inv, s);  // zeros outside the row
+  }
+  mom_sum<G, A>(s, unused, lds);
+  const A mean = s;
+  A sd = A(0), m2 = A(0);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    if (valid[j] == 0) continue;
+#pragma unroll
+    for (int k = 0; k < VW; ++k) {
+      const A d = in_row(j, k) ? sum_elem<T, VW, A>(x[j], k) - mean : A(0);
+      sd += d;
+      m2 = fma(d, d, m2);
+    }
+  }
+  mom_sum<G, A>(sd, m2, lds);
+  if (l == 0) {
+    const A corr = sd / count;
+    const A q = m2 - sd * corr;
+    Welford<A> w{count, mean + corr, q < A(0) ? A(0) : q};
+    if constexpr (FINAL) {
+      mom_write<A, T>(w, correction, take_sqrt, out_var + row, out_mean ? out_mean + row : nullptr);
+    } else {
+      A* p = part + 3 * (int64_t)blockIdx.x;
+      p[0] = w.n;
+      p[1] = (mean - (A)to_arith(src[0])) + corr;
+      p[2] = w.m2;
+    }
+  }
+}
+
+// One wavefront merges a row's chunk triples.
+template <typename T, typename A>
+__global__ void __launch_bounds__(64)
+k_moments_final(const T* __restrict__ in, int64_t row_stride, const A* __restrict__ part, int64_t nch, A correction,
+                int take_sqrt, T* __restrict__ out_var, T* __restrict__ out_mean) {
+  const int64_t row = blockIdx.x;
+  const A* src = part + 3 * row * nch;
+  Welford<A> w{A(0), A(0), A(0)};
+  for (int64_t i = threadIdx.x; i < nch; i += 64) w = wf_merge(w, Welford<A>{src[3 * i], src[3 * i + 1], src[3 * i + 2]});
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) w = wf_merge(w, wf_shfl(w, off));
-  if constexpr (BS > 64) {
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int k = 1; k < BS / 64; ++k) w = wf_merge(w, lds[k]);
-    if constexpr (FINAL) {
-      const A div = w.n > correction ? w.n - correction : A(0);
-      const A var = w.m2 / div;
-      out_var[blockIdx.x] = from_arith<OT>(take_sqrt ? sqrt(var) : var);
-      if (out_mean) out_mean[blockIdx.x] = from_arith<OT>(w.mean + K);
-    } else {
-      part[3 * (int64_t)blockIdx.x] = w.n;
-      part[3 * (int64_t)blockIdx.x + 1] = w.mean;
-      part[3 * (int64_t)blockIdx.x + 2] = w.m2;
-    }
-  }
+  w.mean += (A)to_arith(in[row * row_stride]);
+  if (threadIdx.x == 0)
+    mom_write<A, T>(w, correction, take_sqrt, out_var + row,
+                    out_mean ? out_mean + row : nullptr);
 }
 
+inline int64_t mom_vecs(int64_t segs, int64_t len, int vw) { return segs * ((len + vw - 1) / vw); }
+inline int64_t mom_chunks(int64_t nvec) { return (nvec + kMomChunk - 1) / kMomChunk; }
+
 template <typename T>
-int moments_launch(const T* in, T* out_var, T* out_mean, int64_t outer, int64_t inner, double correction,
-                   int take_sqrt, void* ws, hipStream_t st) {
+int moments_launch(const T* in, T* out_var, T* out_mean, int64_t rows, int64_t segs, int64_t len, int64_t row_stride,
+                   int64_t seg_stride, double correction, int take_sqrt, void* ws, hipStream_t st) {
   using A = opmath_t<T>;
-  const int64_t nch = mom_chunks(outer, inner);
-  if (nch == 1 && inner <= kMomWaveRow) {
-    k_moments<64, T, T, T, A, true, true><<<(unsigned)outer, 64, 0, st>>>(
-        in, in, inner, inner, inner, 1u, (A)correction, take_sqrt, out_var, out_mean, nullptr);
+  constexpr int VW = 16 / (int)sizeof(T);
+  const int64_t nvec = mom_vecs(segs, len, VW), nch = mom_chunks(nvec);
+  const int64_t chunk = (nvec + nch - 1) / nch;
+  const SegGeom g{rows, row_stride, seg_stride, segs, len, FastDiv(segs > 1 ? (uint32_t)((len + VW - 1) / VW) : 1u), nvec,
+                  (uint32_t)chunk};
+  if (nch > 1) {
+    A* part = static_cast<A*>(ws);
+    k_moments<T, A, VW, 256, kMomVecs, false>
+        <<<(unsigned)(rows * nch), kMomBlock, 0, st>>>(in, g, FastDiv((uint32_t)nch), (A)correction, take_sqrt, nullptr,
+                                                      nullptr, part);
+    const int rc = launch_status();
+    if (rc) return rc;
+    k_moments_final<T, A><<<(unsigned)rows, 64, 0, st>>>(in, row_stride, part, nch, (A)correction, take_sqrt, out_var,
+                                                         out_mean);
     return launch_status();
   }
-  if (nch == 1) {
-    k_moments<kMomBlock, T, T, T, A, true, true><<<(unsigned)outer, kMomBlock, 0, st>>>(
-        in, in, inner, inner, inner, 1u, (A)correction, take_sqrt, out_var, out_mean, nullptr);
+  auto go = [&](auto G, auto NV) {
+    const unsigned blocks = (unsigned)((rows + 256 / G.value - 1) / (256 / G.value));
+    k_moments<T, A, VW, G.value, NV.value, true>
+        <<<blocks, kMomBlock, 0, st>>>(in, g, FastDiv(), (A)correction, take_sqrt, out_var, out_mean, nullptr);
     return launch_status();
-  }
-  A* part = static_cast<A*>(ws);
-  k_moments<kMomBlock, T, T, T, A, true, false><<<(unsigned)(outer * nch), kMomBlock, 0, st>>>(
-      in, in, inner, inner, kMomChunk, (uint32_t)nch, (A)correction, take_sqrt, nullptr, nullptr, part);
-  const int rc = launch_status();
-  if (rc) return rc;
-  k_moments<kMomBlock, A, T, T, A, false, true><<<(unsigned)outer, kMomBlock, 0, st>>>(
-      part, in, inner, nch, nch, 1u, (A)correction, take_sqrt, out_var, out_mean, nullptr);
-  return launch_status();
+  };
+  using std::integral_constant;
+  using G16 = integral_constant<int, 16>;
+  using G64 = integral_constant<int, 64>;
+  using G256 = integral_constant<int, 256>;
+  using N1 = integral_constant<int, 1>;
+  using N2 = integral_constant<int, 2>;
+  using N4 = integral_constant<int, 4>;
+  using N8 = integral_constant<int, 8>;
+  // the fewest threads a row, and of those the fewest vectors a thread
+  if (nvec <= 16) return go(G16{}, N1{});
+  if (nvec <= 64) return go(G64{}, N1{});
+  if (nvec <= 128) return go(G64{}, N2{});
+  if (nvec <= 256) return go(G64{}, N4{});
+  if (nvec <= 512) return go(G256{}, N2{});
+  if (nvec <= 1024) return go(G256{}, N4{});
+  return go(G256{}, N8{});
 }
 
 }  // namespace sa
@@ -155,28 +227,33 @@ using namespace sa;
 
 extern "C" {
 
-int64_t supa_amd_moments_rows_workspace_bytes(int64_t outer, int64_t inner, int32_t dtype) {
-  if (outer < 0 || inner <= 0) return SUPA_AMD_EINVAL;
+int64_t supa_amd_moments_segments_workspace_bytes(int64_t rows, int64_t segs, int64_t len, int32_t dtype) {
+  if (rows < 0 || segs <= 0 || len <= 0) return SUPA_AMD_EINVAL;
   if (dtype != SUPA_AMD_F32 && dtype != SUPA_AMD_BF16 && dtype != SUPA_AMD_F16 && dtype != SUPA_AMD_F64)
     return SUPA_AMD_EDTYPE;
-  const int64_t nch = mom_chunks(outer, inner);
-  return nch == 1 ? 0 : outer * nch * 3 * (dtype == SUPA_AMD_F64 ? 8 : 4);
+  const int64_t nch = mom_chunks(mom_vecs(segs, len, 16 / dtype_size(dtype)));
+  return nch == 1 ? 0 : rows * nch * 3 * (dtype == SUPA_AMD_F64 ? 8 : 4);
 }
 
-int supa_amd_moments_rows(const void* in, int32_t dtype, int64_t outer, int64_t inner, double correction,
-                          int take_sqrt, void* out_var, void* out_mean, void* workspace, int64_t ws_bytes,
-                          void* stream) {
-  if (!in || !out_var || outer < 0 || inner <= 0 || correction != correction) return SUPA_AMD_EINVAL;
-  if (outer == 0) return SUPA_AMD_OK;
-  if (outer * mom_chunks(outer, inner) >= (int64_t(1) << 31)) return SUPA_AMD_ELAYOUT;
-  const int64_t need = supa_amd_moments_rows_workspace_bytes(outer, inner, dtype);
+int64_t supa_amd_moments_rows_workspace_bytes(int64_t outer, int64_t inner, int32_t dtype) {
+  return supa_amd_moments_segments_workspace_bytes(outer, 1, inner, dtype);
+}
+
+int supa_amd_moments_segments(const void* in, int32_t dtype, int64_t rows, int64_t segs, int64_t len,
+                              int64_t row_stride, int64_t seg_stride, double correction, int take_sqrt, void* out_var,
+                              void* out_mean, void* workspace, int64_t ws_bytes, void* stream) {
+  if (!in || !out_var || rows < 0 || segs <= 0 || len <= 0 || correction != correction) return SUPA_AMD_EINVAL;
+  if (rows == 0) return SUPA_AMD_OK;
+  const int64_t need = supa_amd_moments_segments_workspace_bytes(rows, segs, len, dtype);
   if (need < 0) return (int)need;
+  const int64_t nvec = mom_vecs(segs, len, 16 / dtype_size(dtype));
+  if (rows * mom_chunks(nvec) >= (int64_t(1) << 31) || (segs > 1 && nvec >= (int64_t(1) << 31))) return SUPA_AMD_ELAYOUT;
   if (need > 0 && (!workspace || ws_bytes < need)) return SUPA_AMD_EWORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto go = [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
-    return moments_launch<T>(static_cast<const T*>(in), static_cast<T*>(out_var), static_cast<T*>(out_mean), outer,
-                             inner, correction, take_sqrt ? 1 : 0, workspace, st);
+    return moments_launch<T>(static_cast<const T*>(in), static_cast<T*>(out_var), static_cast<T*>(out_mean), rows,
+                             segs, len, row_stride, seg_stride, correction, take_sqrt ? 1 : 0, workspace, st);
   };
   switch (dtype) {
     case SUPA_AMD_F32: return go((float*)nullptr);
@@ -185,6 +262,13 @@ int supa_amd_moments_rows(const void* in, int32_t dtype, int64_t outer, int64_t 
     case SUPA_AMD_F64: return go((double*)nullptr);
     default: return SUPA_AMD_EDTYPE;
   }
+}
+
+int supa_amd_moments_rows(const void* in, int32_t dtype, int64_t outer, int64_t inner, double correction,
+                          int take_sqrt, void* out_var, void* out_mean, void* workspace, int64_t ws_bytes,
+                          void* stream) {
+  return supa_amd_moments_segments(in, dtype, outer, 1, inner, inner, 0, correction, take_sqrt, out_var, out_mean,
+                                   workspace, ws_bytes, stream);
 }
 
 }  // extern "C"

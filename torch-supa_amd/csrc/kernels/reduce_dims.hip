@@ -21,40 +21,12 @@
 //
 // Replaces sum_stub / mean_stub over dims
 // (.../kernels/reduce/ReduceSumKernel.cu:102-113, ReduceMomentKernel.cu:37-55).
-#include "ew_launch.h"
-#include "unaligned.h"
+#include "segments.h"
 
 namespace sa {
 
 constexpr int kDimSumBlock = 256;
 constexpr int64_t kDimSumBlocks = 1024;  // workgroups to aim at when cutting chunks: four per CU
-
-template <typename T> constexpr bool dim_sum_vec() { return is_floating_st<T>::value; }
-template <typename T> constexpr int dim_sum_vw() { return dim_sum_vec<T>() ? 16 / (int)sizeof(T) : 1; }
-
-// VW elements of T as loaded, and element k as ACC.
-template <typename T, int VW> struct SumRaw {
-  using type = uint4;
-};
-template <typename T> struct SumRaw<T, 1> {
-  using type = T;
-};
-template <typename T, int VW> using sum_raw_t = typename SumRaw<T, VW>::type;
-
-template <typename T, int VW> __device__ __forceinline__ sum_raw_t<T, VW> sum_load(const T* p) {
-  if constexpr (VW == 1) return *p;
-  else return ld_any_stream(p);
-}
-template <typename T, int VW, typename ACC>
-__device__ __forceinline__ ACC sum_elem(const sum_raw_t<T, VW>& w, int k) {
-  if constexpr (VW == 1) {
-    return (ACC)to_arith(w);
-  } else {
-    T v[VW];
-    __builtin_memcpy(v, &w, 16);
-    return (ACC)to_arith(v[k]);
-  }
-}
 
 // --------------------------------------------------------------- columns
 // Thread (tx, ty) adds rows ty, ty + TY, ... of its chunk for VW columns; TX =
@@ -207,41 +179,6 @@ int cols_run(const T* in, OT* out, int64_t outer, int64_t red, int64_t inner, co
 // numbered across the runs; G threads share a row: 16 lanes or a wavefront
 // for short rows, a workgroup of 256 for long ones, and chunks of `chunk`
 // vectors in blockIdx.y for few long ones.
-struct SegGeom {
-  int64_t rows, row_stride, seg_stride;
-  FastDiv vps;      // vectors per run
-  uint32_t nvec;    // vectors per row
-  uint32_t chunk;   // vectors per chunk
-  int64_t len;
-};
-
-template <typename T, int VW>
-__device__ __forceinline__ sum_raw_t<T, VW> seg_load(const T* row, const SegGeom& g, uint32_t i) {
-  uint32_t s, v;
-  g.vps.divmod(i, s, v);
-  const T* p = row + (int64_t)s * g.seg_stride + (int64_t)v * VW;
-  if constexpr (VW == 1) {
-    return *p;
-  } else {
-    const int64_t left = g.len - (int64_t)v * VW;
-    if (left >= VW) return ld_any_stream(p);
-    T w[VW];
-    uint4 q;
-    if (g.len >= VW) {  // the run's last vector, zeros for what the one before holds
-      q = ld_any(p + left - VW);
-      __builtin_memcpy(w, &q, 16);
-#pragma unroll
-      for (int k = 0; k < VW; ++k)
-        if (k < VW - left) w[k] = T{};
-    } else {
-#pragma unroll
-      for (int k = 0; k < VW; ++k) w[k] = k < left ? p[k] : T{};
-    }
-    __builtin_memcpy(&q, w, 16);
-    return q;
-  }
-}
-
 template <typename T, typename OT, typename ACC, int VW, int G>
 __global__ void __launch_bounds__(kDimSumBlock)
 k_sum_segs(const T* __restrict__ in, OT* __restrict__ out, SegGeom g, ACC scale) {
@@ -251,13 +188,15 @@ k_sum_segs(const T* __restrict__ in, OT* __restrict__ out, SegGeom g, ACC scale)
   if (row >= g.rows) return;
   const T* src = in + row * g.row_stride;
   const uint32_t lo = blockIdx.y * g.chunk;
-  const uint32_t hi = g.nvec - lo < g.chunk ? g.nvec : lo + g.chunk;
+  const uint32_t nvec = (uint32_t)g.nvec;
+  const uint32_t hi = nvec - lo < g.chunk ? nvec : lo + g.chunk;
   ACC acc = ACC(0);
   for (uint32_t i0 = lo + l; i0 < hi; i0 += U * G) {
     sum_raw_t<T, VW> w[U];
+    uint32_t valid;  // elements past a run's end are zeros
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i0 + u * G < hi) w[u] = seg_load<T, VW>(src, g, i0 + u * G);
+      if (i0 + u * G < hi) w[u] = seg_load<T, VW>(src, g, i0 + u * G, valid);
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (i0 + u * G < hi) {
@@ -312,12 +251,12 @@ int segs_run(const T* in, OT* out, int64_t rows, int64_t segs, int64_t len, int6
   if (nvec >= (int64_t(1) << 31) || rows >= (int64_t(1) << 31)) return SUPA_AMD_ELAYOUT;
   const int64_t want = ws ? seg_chunks(rows, nvec) : 1;
   const int64_t chunk = (nvec + want - 1) / want, nch = (nvec + chunk - 1) / chunk;
-  SegGeom g{rows, row_stride, seg_stride, FastDiv((uint32_t)vps), (uint32_t)nvec, (uint32_t)chunk, len};
+  SegGeom g{rows, row_stride, seg_stride, segs, len, FastDiv((uint32_t)vps), nvec, (uint32_t)chunk};
   if (nch == 1) return segs_launch<T, OT, ACC, VW>(in, out, g, 1, scale, st);
   ACC* part = static_cast<ACC*>(ws);
   const int rc = segs_launch<T, ACC, ACC, VW>(in, part, g, (unsigned)nch, ACC(1), st);
   if (rc) return rc;
-  SegGeom h{rows, nch, 0, FastDiv((uint32_t)nch), (uint32_t)nch, (uint32_t)nch, nch};
+  SegGeom h{rows, nch, 0, 1, nch, FastDiv((uint32_t)nch), nch, (uint32_t)nch};
   return segs_launch<ACC, OT, ACC, 1>(part, out, h, 1, scale, st);
 }
 
