@@ -1,6 +1,7 @@
 """Elementwise ops and full reductions over runs whose length is no multiple of
 the vector, at any alignment: bias broadcasts, slices of rows, misaligned
-views, in-place forms, and the losses over them."""
+views, in-place forms, and the losses over them; the nll gradients of
+odd class counts."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -98,3 +99,31 @@ def test_losses_over_odd_runs(cols, dtype, reduction, no_fallback):
     torch.testing.assert_close(dx.grad.cpu().double(), cx.grad, rtol=tol, atol=tol / max(1, x.numel() if reduction == "mean" else 1))
     torch.testing.assert_close(F.mse_loss(dx.detach(), t.to("supa"), reduction=reduction).cpu().double(),
                                F.mse_loss(x.double(), t.double(), reduction=reduction), rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("c", [1, 2, 3, 7, 8, 9, 100, 2047, 2048, 2049, 5003])
+def test_nll_backward_of_odd_classes(c, dtype, no_fallback):
+    n = 301
+    t = torch.randint(0, c, (n,), generator=torch.Generator().manual_seed(13))
+    t[::7] = -100
+    lp = seeded((n, c), 14, dtype)
+    w = (seeded((c,), 15).abs() + 0.5).to(dtype)
+    for red, weight in (("mean", None), ("sum", w), ("none", w)):
+        d = lp.to("supa").requires_grad_()
+        r = lp.clone().requires_grad_()
+        ld = F.nll_loss(d, t.to("supa"), None if weight is None else weight.to("supa"), reduction=red)
+        lr = F.nll_loss(r, t, weight, reduction=red)
+        g = seeded((n,), 16, dtype) if red == "none" else torch.ones((), dtype=dtype)
+        ld.backward(g.to("supa"))
+        lr.backward(g)
+        tol = 1e-2 if dtype == torch.bfloat16 else 1e-5
+        torch.testing.assert_close(d.grad.cpu(), r.grad, rtol=tol, atol=0)
+
+
+def test_nll_backward_flags_a_bad_target(no_fallback):
+    for c in (5, 3001):
+        t = torch.tensor([0, c, 1], device="supa")
+        with pytest.raises(IndexError):
+            torch.ops.aten.nll_loss_backward(torch.ones((), device="supa"), torch.zeros(3, c, device="supa"), t, None, 2,
+                                             -100, torch.ones((), device="supa")).cpu()

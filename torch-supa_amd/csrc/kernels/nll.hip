@@ -10,7 +10,9 @@
 //
 // Backward: writes every element of grad_input once -- 16-byte vectors of
 // zeros, with the row's target element replaced by its gradient -- so the
-// [n, c] tensor costs one HBM write and no separate zero fill.
+// [n, c] tensor costs one HBM write and no separate zero fill.  Rows of any
+// length: long ones by row, on the line grid, short ones as one flat range
+// of aligned vectors that may span rows.
 //
 // Spatial form (nll_loss2d: logp [n, c, s], target [n, s], s = H * W): the
 // forward gathers with a multi-workgroup two-stage reduction (a fixed number
@@ -22,6 +24,7 @@
 // the host reads the flag lazily.
 #include "ew_launch.h"
 #include "divmod.h"
+#include "unaligned.h"
 
 namespace sa {
 
@@ -118,6 +121,23 @@ constexpr int kNllBwdBlock = 256;
 // kNllBwdBlock * VEC elements.  g_row is the row's gradient before the weight:
 // -(g_i) for none, -(g / total_weight) for mean, -g for sum, formed in the data
 // dtype as upstream does.
+template <typename T>
+__device__ __forceinline__ bool nll_active(int64_t t, int64_t c, int64_t ignore_index) {
+  return t != ignore_index && t >= 0 && t < c;
+}
+// The gradient at row `row`'s target t.
+template <typename T>
+__device__ __forceinline__ T nll_grad(const T* grad_out, const T* weight, const T* total_weight, int64_t row, int64_t t,
+                                      int reduction) {
+  using C = opmath_t<T>;
+  C g;
+  if (reduction == SUPA_AMD_REDUCTION_NONE) g = (C)to_arith(grad_out[row]);
+  else if (reduction == SUPA_AMD_REDUCTION_MEAN) g = (C)to_arith(grad_out[0]) / (C)to_arith(total_weight[0]);
+  else g = (C)to_arith(grad_out[0]);
+  const T gs = from_arith<T>(-g);  // rounded to the storage type, as upstream forms it
+  return weight ? from_arith<T>((C)to_arith(weight[t]) * (C)to_arith(gs)) : gs;
+}
+
 template <typename T, int VEC>
 __global__ void __launch_bounds__(kNllBwdBlock)
 k_nll_bwd(const T* __restrict__ grad_out, const int64_t* __restrict__ target, const T* __restrict__ weight,
@@ -126,32 +146,74 @@ k_nll_bwd(const T* __restrict__ grad_out, const int64_t* __restrict__ target, co
   using C = opmath_t<T>;
   const int64_t row = blockIdx.y;
   const int64_t t = target[row];
-  const bool active = t != ignore_index && t >= 0 && t < c;
+  const bool active = nll_active<T>(t, c, ignore_index);
   if (threadIdx.x == 0 && blockIdx.x == 0 && t != ignore_index && (t < 0 || t >= c) && error_flag) *error_flag = 1;
-  T gval = from_arith<T>(C(0));
-  if (active) {
-    C g;
-    if (reduction == SUPA_AMD_REDUCTION_NONE) g = (C)to_arith(grad_out[row]);
-    else if (reduction == SUPA_AMD_REDUCTION_MEAN) g = (C)to_arith(grad_out[0]) / (C)to_arith(total_weight[0]);
-    else g = (C)to_arith(grad_out[0]);
-    const T gs = from_arith<T>(-g);  // rounded to the storage type, as upstream forms it
-    gval = weight ? from_arith<T>((C)to_arith(weight[t]) * (C)to_arith(gs)) : gs;
-  }
-  T* dst = gin + row * c;
   const T zero = from_arith<T>(C(0));
+  const T gval = active ? nll_grad<T>(grad_out, weight, total_weight, row, t, reduction) : zero;
+  T* dst = gin + row * c;
+  // the row's vectors start o elements before it (unaligned.h's grid); a row's
+  // first and last partial vectors go element by element (bf16 [4096, 50257]:
+  // 74 us, with the 16-byte grid 90, at element alignment 94, one element a
+  // thread 334)
+  const int o = grid_off<T, VEC>(dst, c);
 #pragma unroll
   for (int u = 0; u < kNllUnroll; ++u) {
-    const int64_t col0 = (((int64_t)blockIdx.x * kNllUnroll + u) * kNllBwdBlock + threadIdx.x) * VEC;
+    const int64_t col0 = (((int64_t)blockIdx.x * kNllUnroll + u) * kNllBwdBlock + threadIdx.x) * VEC - o;
     if (col0 >= c) break;
-    if (VEC > 1 && col0 + VEC <= c) {
+    if (col0 >= 0 && col0 + VEC <= c) {
       Vec<T, VEC> w;
 #pragma unroll
       for (int k = 0; k < VEC; ++k) w.v[k] = zero;
       if (active && t >= col0 && t < col0 + VEC) w.v[t - col0] = gval;
       st_stream(reinterpret_cast<Vec<T, VEC>*>(dst + col0), w);
     } else {
-      for (int k = 0; k < VEC && col0 + k < c; ++k) dst[col0 + k] = (active && col0 + k == t) ? gval : zero;
+      for (int k = col0 < 0 ? (int)-col0 : 0; k < VEC && col0 + k < c; ++k)  // none before the row
+        dst[col0 + k] = (active && col0 + k == t) ? gval : zero;
     }
+  }
+}
+
+// Rows of fewer than kNllFlat elements: vector v of the flat [n c] range, its
+// first element's row by magic division; the rows it touches are walked, a
+// row's target element written where it falls.  A 256-thread workgroup per
+// row left most threads idle there (bf16 [262144, 19] 122 us, 5.2 now;
+// [8192, 1000] 18.7 and 5.2).
+constexpr int64_t kNllFlat = 2048;
+
+template <typename T, int VEC>
+__global__ void __launch_bounds__(kNllBwdBlock)
+k_nll_bwd_flat(const T* __restrict__ grad_out, const int64_t* __restrict__ target, const T* __restrict__ weight,
+               const T* __restrict__ total_weight, uint32_t total, FastDiv cdiv, int reduction, int64_t ignore_index,
+               T* __restrict__ gin, int32_t* error_flag) {
+  using C = opmath_t<T>;
+  const uint32_t e = (blockIdx.x * kNllBwdBlock + threadIdx.x) * VEC;
+  if (e >= total) return;
+  const uint32_t c = cdiv.d;
+  const uint32_t end = total - e < (uint32_t)VEC ? total : e + VEC;
+  Vec<T, VEC> w;
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) w.v[k] = from_arith<T>(C(0));
+  uint32_t row = cdiv.div(e);
+  for (uint32_t start = row * c; start < end; start += c, ++row) {
+    const int64_t t = target[row];
+    if (!nll_active<T>(t, c, ignore_index)) {
+      if (t != ignore_index && start >= e && error_flag) *error_flag = 1;  // by the vector that holds the row's start
+      continue;
+    }
+    const uint32_t at = start + (uint32_t)t;
+    if (at >= e && at < end) {
+      const T g = nll_grad<T>(grad_out, weight, total_weight, row, t, reduction);
+#pragma unroll
+      for (int k = 0; k < VEC; ++k)
+        if (e + k == at) w.v[k] = g;
+    }
+  }
+  if (end - e == (uint32_t)VEC) {
+    st_vec_any<T, VEC>(gin + e, w);
+  } else {
+#pragma unroll
+    for (int k = 0; k < VEC; ++k)
+      if (e + k < end) gin[e + k] = w.v[k];
   }
 }
 
@@ -337,38 +399,28 @@ int supa_amd_nll_loss_backward(const void* grad_out, int32_t dtype, const int64_
   return with_nll_storage(dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     constexpr int VEC = 16 / sizeof(T);
-    const bool vec_ok = (c % VEC) == 0 && aligned(grad_in, 16);
     const T* g = static_cast<const T*>(grad_out);
     const T* w = static_cast<const T*>(weight);
     const T* tw = static_cast<const T*>(total_weight);
     T* gi = static_cast<T*>(grad_in);
-    if (n > 65535) {
-      // grid.y is limited; launch in row slabs
-      for (int64_t r0 = 0; r0 < n; r0 += 65535) {
-        const int64_t rows = std::min<int64_t>(65535, n - r0);
-        const T* gslab = reduction == SUPA_AMD_REDUCTION_NONE ? g + r0 : g;
-        if (vec_ok) {
-          dim3 grid((unsigned)((c / VEC + kNllBwdBlock * kNllUnroll - 1) / (kNllBwdBlock * kNllUnroll)), (unsigned)rows);
-          k_nll_bwd<T, VEC><<<grid, kNllBwdBlock, 0, st>>>(gslab, target + r0, w, tw, c, reduction, ignore_index,
-                                                      gi + r0 * c, error_flag);
-        } else {
-          dim3 grid((unsigned)((c + kNllBwdBlock * kNllUnroll - 1) / (kNllBwdBlock * kNllUnroll)), (unsigned)rows);
-          k_nll_bwd<T, 1><<<grid, kNllBwdBlock, 0, st>>>(gslab, target + r0, w, tw, c, reduction, ignore_index,
-                                                    gi + r0 * c, error_flag);
-        }
-        const int rc = launch_status();
-        if (rc) return rc;
-      }
-      return SUPA_AMD_OK;
+    if (c < kNllFlat && n * c < (int64_t(1) << 32) - kNllBwdBlock * VEC) {
+      const unsigned blocks = (unsigned)((n * c + kNllBwdBlock * VEC - 1) / (kNllBwdBlock * VEC));
+      k_nll_bwd_flat<T, VEC><<<blocks, kNllBwdBlock, 0, st>>>(g, target, w, tw, (uint32_t)(n * c), FastDiv((uint32_t)c),
+                                                              reduction, ignore_index, gi, error_flag);
+      return launch_status();
     }
-    if (vec_ok) {
-      dim3 grid((unsigned)((c / VEC + kNllBwdBlock * kNllUnroll - 1) / (kNllBwdBlock * kNllUnroll)), (unsigned)n);
-      k_nll_bwd<T, VEC><<<grid, kNllBwdBlock, 0, st>>>(g, target, w, tw, c, reduction, ignore_index, gi, error_flag);
-    } else {
-      dim3 grid((unsigned)((c + kNllBwdBlock * kNllUnroll - 1) / (kNllBwdBlock * kNllUnroll)), (unsigned)n);
-      k_nll_bwd<T, 1><<<grid, kNllBwdBlock, 0, st>>>(g, target, w, tw, c, reduction, ignore_index, gi, error_flag);
+    // grid.y is limited; launch in row slabs
+    for (int64_t r0 = 0; r0 < n; r0 += 65535) {
+      const int64_t rows = std::min<int64_t>(65535, n - r0);
+      const T* gslab = reduction == SUPA_AMD_REDUCTION_NONE ? g + r0 : g;
+      const dim3 grid((unsigned)((grid_vecs<T, VEC>(gi, c) + kNllBwdBlock * kNllUnroll - 1) / (kNllBwdBlock * kNllUnroll)),
+                      (unsigned)rows);
+      k_nll_bwd<T, VEC><<<grid, kNllBwdBlock, 0, st>>>(gslab, target + r0, w, tw, c, reduction, ignore_index,
+                                                       gi + r0 * c, error_flag);
+      const int rc = launch_status();
+      if (rc) return rc;
     }
-    return launch_status();
+    return SUPA_AMD_OK;
   });
 }
 
