@@ -1,7 +1,7 @@
 """Elementwise ops and full reductions over runs whose length is no multiple of
 the vector, at any alignment: bias broadcasts, slices of rows, misaligned
-views, in-place forms, and the losses over them; the nll gradients of
-odd class counts."""
+views, in-place forms, and the losses over them; the nll and cross-entropy
+gradients of odd class counts."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -127,3 +127,22 @@ def test_nll_backward_flags_a_bad_target(no_fallback):
         with pytest.raises(IndexError):
             torch.ops.aten.nll_loss_backward(torch.ones((), device="supa"), torch.zeros(3, c, device="supa"), t, None, 2,
                                              -100, torch.ones((), device="supa")).cpu()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("c", [3, 9, 1001, 50257])
+def test_fused_cross_entropy_of_odd_classes(c, dtype, no_fallback, fused_ce):
+    n = 33
+    x = (seeded((n, c), 17) * 2).to(dtype)
+    t = torch.randint(0, c, (n,), generator=torch.Generator().manual_seed(18))
+    t[5] = -100
+    prob = torch.softmax(seeded((n, c), 19), 1).to(dtype)
+    for target in (t, prob):
+        d, r = x.to("supa").requires_grad_(), x.double().requires_grad_()
+        ld = F.cross_entropy(d, target.to("supa"))
+        lr = F.cross_entropy(r, target if target is t else target.double())
+        ld.backward()
+        lr.backward()
+        tol = 1e-5 if dtype == torch.float32 else 1e-2
+        torch.testing.assert_close(ld.detach().cpu().double(), lr.detach(), rtol=tol, atol=0)
+        torch.testing.assert_close(d.grad.cpu().double(), r.grad, rtol=tol, atol=tol / n / 10)

@@ -22,8 +22,7 @@
 // sum of t T, sum of t (x - m) B) state, combines it across the workgroup and
 // writes loss = T log(s) - B = sum_j t_j (lse - x_j) with lse and T saved per
 // row; the backward writes g_i (exp(x - lse_i) T_i - t) in one pass.
-#include "devmath.h"
-#include "ew_launch.h"
+#include "softmax_common.h"
 
 namespace sa {
 
@@ -66,20 +65,39 @@ __device__ __forceinline__ bool ce_kept(int64_t t, int64_t c, int64_t ignore_ind
 // loss_rows[i] (float32): the row's loss, 0 for an ignored row.  lse[i]: the
 // row's log-sum-exp (0 for an ignored row).  out_none (may be null): the loss
 // in the logits dtype, for reduction 'none'.
-// VECOK: rows are 16-byte aligned and c % V == 0, so rows stream as 16-byte
-// vectors; otherwise every element takes the scalar path.
-template <typename T, bool VECOK>
+// Rows stream as 16-byte vectors at any alignment, their last c mod V elements
+// one to a thread (rows of odd length took two exponentials per element
+// through the pairwise update: float32 [4096, 50257] 259 us, 130 now, HBM
+// bound at 6.3 TB/s; with the gradient 900, 384).
+// G threads share a row: a wavefront (four rows a workgroup) up to
+// kCeWaveVecs vectors, else the workgroup (float32 [65536, 1000] 109 us with
+// a workgroup per row, 46 with a wavefront; from 257 vectors on a wavefront
+// would hold a second batch of loads while the next row's wait).
+constexpr int kCeWaveVecs = 64 * kCeUnroll;
+
+template <typename T, int G>
 __global__ void __launch_bounds__(kCeBlock)
-k_ce_fwd(const T* __restrict__ x, const int64_t* __restrict__ target, int64_t c, int64_t ignore_index,
+k_ce_fwd(const T* __restrict__ x, const int64_t* __restrict__ target, int64_t n, int64_t c, int64_t ignore_index,
          float* __restrict__ loss_rows, float* __restrict__ lse, T* __restrict__ out_none, int32_t* error_flag) {
   constexpr int V = CeVec<T>::V;
-  constexpr int NW = kCeBlock / 64;
-  __shared__ float lds_m[NW];
-  __shared__ float lds_s[NW];
-  const int64_t row = blockIdx.x;
+  constexpr int NW = G / 64;
+  const int l = threadIdx.x & (G - 1);
+  int64_t row = blockIdx.x;
+  if constexpr (G < kCeBlock) row = (int64_t)blockIdx.x * (kCeBlock / G) + threadIdx.x / G;
+  if (row >= n) return;
+  const T* xr = x + row * c;
+  const int64_t nvec = c / V;
+  // a wavefront's rows issue their loads before the target arrives (an
+  // ignored row then reads logits it does not need)
+  uint4 first[kCeUnroll];
+  if constexpr (G < kCeBlock) {
+#pragma unroll
+    for (int u = 0; u < kCeUnroll; ++u)
+      if (l + u * G < nvec) first[u] = ld_any_stream(xr + (int64_t)(l + u * G) * V);
+  }
   const int64_t t = target[row];
-  if (!ce_kept(t, c, ignore_index)) {
-    if (threadIdx.x == 0) {
+  if (!ce_kept(t, c, ignore_index)) {  // the whole row's threads
+    if (l == 0) {
       if (t != ignore_index && error_flag) *error_flag = 1;
       loss_rows[row] = 0.0f;
       lse[row] = 0.0f;
@@ -87,21 +105,24 @@ k_ce_fwd(const T* __restrict__ x, const int64_t* __restrict__ target, int64_t c,
     }
     return;
   }
-  const T* xr = x + row * c;
-  const uint4* src = reinterpret_cast<const uint4*>(xr);
-  const int64_t nvec = VECOK ? c / V : 0;
+  float xt = 0.0f;  // a wavefront's, early; a workgroup reads it at the end
+  if constexpr (G < kCeBlock) xt = (float)to_arith(xr[t]);
   float m = -__builtin_inff(), s = 0.0f;
-  for (int64_t v0 = threadIdx.x; v0 < nvec; v0 += (int64_t)kCeBlock * kCeUnroll) {
+  for (int64_t v0 = l; v0 < nvec; v0 += (int64_t)G * kCeUnroll) {
     uint4 w[kCeUnroll];
 #pragma unroll
     for (int u = 0; u < kCeUnroll; ++u) {
-      const int64_t v = v0 + (int64_t)u * kCeBlock;
-      if (v < nvec) w[u] = ld_stream(src + v);
+      const int64_t v = v0 + (int64_t)u * G;
+      if constexpr (G < kCeBlock) {  // the row's only step
+        w[u] = first[u];
+      } else {
+        if (v < nvec) w[u] = ld_any_stream(xr + v * V);
+      }
     }
     float mb = -__builtin_inff();
 #pragma unroll
     for (int u = 0; u < kCeUnroll; ++u) {
-      if (v0 + (int64_t)u * kCeBlock < nvec) {
+      if (v0 + (int64_t)u * G < nvec) {
 #pragma unroll
         for (int k = 0; k < V; ++k) mb = fmaxf(mb, ce_elem<T>(w[u], k));
       }
@@ -111,7 +132,7 @@ k_ce_fwd(const T* __restrict__ x, const int64_t* __restrict__ target, int64_t c,
       float sb = 0.0f;
 #pragma unroll
       for (int u = 0; u < kCeUnroll; ++u) {
-        if (v0 + (int64_t)u * kCeBlock < nvec) {
+        if (v0 + (int64_t)u * G < nvec) {
 #pragma unroll
           for (int k = 0; k < V; ++k) sb += __builtin_amdgcn_exp2f((ce_elem<T>(w[u], k) - M) * kCeLog2e);
         }
@@ -120,57 +141,73 @@ k_ce_fwd(const T* __restrict__ x, const int64_t* __restrict__ target, int64_t c,
       m = M;
     }
   }
-  // elements not covered by whole vectors (all of them when !VECOK)
-  for (int64_t j = nvec * V + threadIdx.x; j < c; j += kCeBlock) {
+  // the elements after the whole vectors
+  for (int64_t j = nvec * V + l; j < c; j += G) {
     const float xv = (float)to_arith(xr[j]);
     ce_combine(m, s, xv, 1.0f);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) ce_combine(m, s, __shfl_xor(m, off, 64), __shfl_xor(s, off, 64));
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    lds_m[wave] = m;
-    lds_s[wave] = s;
+  lanes_lse<64>(m, s);
+  if constexpr (NW > 1) {
+    __shared__ float lds_m[NW];
+    __shared__ float lds_s[NW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) {
+      lds_m[wave] = m;
+      lds_s[wave] = s;
+    }
+    __syncthreads();
+    m = lds_m[lane & (NW - 1)];
+    s = lds_s[lane & (NW - 1)];
+    lanes_lse<NW>(m, s);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float M = lds_m[0], S = lds_s[0];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) ce_combine(M, S, lds_m[w], lds_s[w]);
-    const float l = M + sa_logf(S);
-    const float loss = l - (float)to_arith(xr[t]);
+  if (l == 0) {
+    const float lg = m + sa_logf(s);
+    if constexpr (G == kCeBlock) xt = (float)to_arith(xr[t]);
+    const float loss = lg - xt;
     loss_rows[row] = loss;
-    lse[row] = l;
+    lse[row] = lg;
     if (out_none) out_none[row] = from_arith<T>(loss);
   }
 }
 
 // Stage 2: sum of the row losses and the kept-row count, fixed order
-// (target null: every row counts, the probability-target form).
-template <typename T>
-__global__ void __launch_bounds__(kCeBlock)
-k_ce_final(const float* __restrict__ loss_rows, const int64_t* __restrict__ target, int64_t n, int64_t c,
+// (target null: every row counts, the probability-target form).  Up to
+// kCeSumRows rows one workgroup, all loads in flight; of more, a first launch
+// (PART) sums whole chunks of that many, each workgroup leaving (sum, count) in
+// its chunk's first two loss slots, which nobody else reads, and the last
+// launch adds those and the rows after the chunks.
+constexpr int kCeSumBlock = 1024;
+constexpr int64_t kCeSumRows = 8192;
+
+template <typename T, bool PART>
+__global__ void __launch_bounds__(kCeSumBlock)
+k_ce_final(float* __restrict__ loss_rows, const int64_t* __restrict__ target, int64_t n, int64_t nparts, int64_t c,
            int64_t ignore_index, int mean, T* __restrict__ out, float* __restrict__ count) {
-  constexpr int NW = kCeBlock / 64;
+  constexpr int NW = kCeSumBlock / 64;
+  constexpr int U = (int)(kCeSumRows / kCeSumBlock);
   __shared__ float lds_v[NW];
   __shared__ float lds_c[NW];
   float v = 0.0f, k = 0.0f;
-  constexpr int U = 8;  // loads in flight per step; the sums keep the row order
-  for (int64_t i0 = threadIdx.x; i0 < n; i0 += (int64_t)U * kCeBlock) {
-    float lv[U];
-    int64_t tg[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t i = i0 + (int64_t)u * kCeBlock;
-      lv[u] = i < n ? loss_rows[i] : 0.0f;
-      tg[u] = i < n && target ? target[i] : ignore_index;
+  if constexpr (!PART) {
+    for (int64_t p = threadIdx.x; p < nparts; p += kCeSumBlock) {
+      v += loss_rows[p * kCeSumRows];
+      k += loss_rows[p * kCeSumRows + 1];
     }
+  }
+  const int64_t i0 = (PART ? (int64_t)blockIdx.x : nparts) * kCeSumRows + threadIdx.x;
+  float lv[U];
+  int64_t tg[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (i0 + (int64_t)u * kCeBlock < n) {
-        v += lv[u];
-        k += (!target || ce_kept(tg[u], c, ignore_index)) ? 1.0f : 0.0f;
-      }
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = i0 + (int64_t)u * kCeSumBlock;
+    lv[u] = i < n ? loss_rows[i] : 0.0f;
+    tg[u] = i < n && target ? target[i] : ignore_index;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (i0 + (int64_t)u * kCeSumBlock < n) {
+      v += lv[u];
+      k += (!target || ce_kept(tg[u], c, ignore_index)) ? 1.0f : 0.0f;
     }
   }
 #pragma unroll
@@ -191,19 +228,43 @@ k_ce_final(const float* __restrict__ loss_rows, const int64_t* __restrict__ targ
       sv += lds_v[w];
       sk += lds_c[w];
     }
-    out[0] = from_arith<T>(mean ? sv / sk : sv);  // 0/0 = NaN for a mean over no rows
-    if (count) count[0] = sk;
+    if constexpr (PART) {  // every row of the chunk is read: the barrier
+      loss_rows[(int64_t)blockIdx.x * kCeSumRows] = sv;
+      loss_rows[(int64_t)blockIdx.x * kCeSumRows + 1] = sk;
+    } else {
+      out[0] = from_arith<T>(mean ? sv / sk : sv);  // 0/0 = NaN for a mean over no rows
+      if (count) count[0] = sk;
+    }
   }
 }
 
+template <typename T>
+int ce_final(float* rows, const int64_t* target, int64_t n, int64_t c, int64_t ignore_index, int reduction, T* out,
+             float* count, hipStream_t st) {
+  const int mean = reduction == SUPA_AMD_REDUCTION_MEAN ? 1 : 0;
+  const int64_t nparts = n > kCeSumRows ? n / kCeSumRows : 0;
+  if (nparts > 0) {
+    k_ce_final<T, true><<<(unsigned)nparts, kCeSumBlock, 0, st>>>(rows, target, n, 0, c, ignore_index, mean, nullptr,
+                                                                 nullptr);
+    const int rc = launch_status();
+    if (rc) return rc;
+  }
+  k_ce_final<T, false><<<1, kCeSumBlock, 0, st>>>(rows, target, n, nparts, c, ignore_index, mean, out, count);
+  return launch_status();
+}
+
+// A row's output vectors are those of unaligned.h's grid, which starts
+// grid_off elements before the row: its stores, and with the logits at the
+// same alignment its loads, are aligned; the first and the last partial vector
+// go element by element.
+//
 // grad[i, :] over a 2-d grid: blockIdx.y = row in the slab, x = column blocks
-// of kCeBwdBlock vectors.  VECOK (c % V == 0, aligned rows: every vector is
-// whole): the logits load goes out unconditionally, before the row's target,
+// of kCeBwdBlock vectors.  A whole vector's logits load goes out unconditionally, before the row's target,
 // and the scale and lse that depend on it, have arrived (an ignored row then
 // reads logits it does not need); waiting for the target first held the
 // kernel at 75 % of the HBM roofline on c3's bf16 rows, against 85 % with the
 // load first.
-template <typename T, bool VECOK>
+template <typename T>
 __global__ void __launch_bounds__(kCeBwdBlock)
 k_ce_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const int64_t* __restrict__ target,
          const float* __restrict__ lse, const float* __restrict__ count, int64_t c, int64_t ignore_index,
@@ -212,10 +273,11 @@ k_ce_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const int64_t*
   const int64_t row = blockIdx.y;
   const T* xr = x + row * c;
   T* dst = gx + row * c;
-  const int64_t col0 = ((int64_t)blockIdx.x * kCeBwdBlock + threadIdx.x) * V;
+  const int64_t col0 = ((int64_t)blockIdx.x * kCeBwdBlock + threadIdx.x) * V - grid_off<T, V>(dst, c);
   if (col0 >= c) return;
   Vec<T, V> w;
-  if constexpr (VECOK) w = ld_stream(reinterpret_cast<const Vec<T, V>*>(xr + col0));
+  const bool whole = col0 >= 0 && col0 + V <= c;
+  if (whole) w = ld_vec_any<true, T, V>(xr + col0);
   const int64_t t = target[row];
   const bool kept = ce_kept(t, c, ignore_index);
   float g = 0.0f;
@@ -225,7 +287,7 @@ k_ce_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const int64_t*
     else g = (float)to_arith(grad_out[0]);
   }
   const float l = kept ? lse[row] : 0.0f;
-  if constexpr (VECOK) {
+  if (whole) {
     // p g everywhere, (p - 1) g at the target: the one thread of the row that
     // holds the target patches its element in a branch, so the other threads
     // spend no compare or select per element (the same values as
@@ -249,9 +311,9 @@ k_ce_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const int64_t*
 #pragma unroll
       for (int k = 0; k < V; ++k) o.v[k] = from_arith<T>(0.0f);
     }
-    st_stream(reinterpret_cast<Vec<T, V>*>(dst + col0), o);
+    st_vec_any<T, V>(dst + col0, o);
   } else {
-    for (int k = 0; k < V && col0 + k < c; ++k) {
+    for (int k = col0 < 0 ? (int)-col0 : 0; k < V && col0 + k < c; ++k) {
       float r = 0.0f;
       if (kept) {
         const float p = __builtin_amdgcn_exp2f(((float)to_arith(xr[col0 + k]) - l) * kCeLog2e);
@@ -291,7 +353,7 @@ __device__ __forceinline__ void ce_prob_combine(CeProbState& a, const CeProbStat
 
 // loss_rows[i] = T log(s) - B (float32); lse[i] = m + log(s); tsum[i] = T;
 // out_none (may be null): the loss in the logits dtype.
-template <typename T, bool VECOK>
+template <typename T>
 __global__ void __launch_bounds__(kCeBlock)
 k_ce_prob_fwd(const T* __restrict__ x, const T* __restrict__ tgt, int64_t c, float* __restrict__ loss_rows,
               float* __restrict__ lse, float* __restrict__ tsum, T* __restrict__ out_none) {
@@ -302,9 +364,7 @@ k_ce_prob_fwd(const T* __restrict__ x, const T* __restrict__ tgt, int64_t c, flo
   const int64_t row = blockIdx.x;
   const T* xr = x + row * c;
   const T* tr = tgt + row * c;
-  const uint4* xs = reinterpret_cast<const uint4*>(xr);
-  const uint4* ts = reinterpret_cast<const uint4*>(tr);
-  const int64_t nvec = VECOK ? c / V : 0;
+  const int64_t nvec = c / V;
   CeProbState st{-__builtin_inff(), 0.0f, 0.0f, 0.0f};
   for (int64_t v0 = threadIdx.x; v0 < nvec; v0 += (int64_t)kCeBlock * U) {
     uint4 wx[U], wt[U];
@@ -312,8 +372,8 @@ k_ce_prob_fwd(const T* __restrict__ x, const T* __restrict__ tgt, int64_t c, flo
     for (int u = 0; u < U; ++u) {
       const int64_t v = v0 + (int64_t)u * kCeBlock;
       if (v < nvec) {
-        wx[u] = ld_stream(xs + v);
-        wt[u] = ld_stream(ts + v);
+        wx[u] = ld_any_stream(xr + v * V);
+        wt[u] = ld_any_stream(tr + v * V);
       }
     }
     float mb = -__builtin_inff();
@@ -354,7 +414,7 @@ k_ce_prob_fwd(const T* __restrict__ x, const T* __restrict__ tgt, int64_t c, flo
         }
     }
   }
-  // elements not covered by whole vectors (all of them when !VECOK)
+  // the elements after the whole vectors
   for (int64_t j = nvec * V + threadIdx.x; j < c; j += kCeBlock)
     ce_prob_combine(st, ce_prob_elem((float)to_arith(xr[j]), (float)to_arith(tr[j])));
 #pragma unroll
@@ -381,7 +441,7 @@ k_ce_prob_fwd(const T* __restrict__ x, const T* __restrict__ tgt, int64_t c, flo
 
 // grad[i, j] = g_i (exp(x - lse_i) T_i - t_ij); g_i = grad_out[i] (none),
 // grad_out[0] (sum) or grad_out[0] / n (mean).
-template <typename T, bool VECOK>
+template <typename T>
 __global__ void __launch_bounds__(kCeBwdBlock)
 k_ce_prob_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const T* __restrict__ tgt,
               const float* __restrict__ lse, const float* __restrict__ tsum, int64_t c, int reduction, float inv_n,
@@ -397,20 +457,20 @@ k_ce_prob_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const T* 
   const T* xr = x + row * c;
   const T* tr = tgt + row * c;
   T* dst = gx + row * c;
-  const int64_t col0 = ((int64_t)blockIdx.x * kCeBwdBlock + threadIdx.x) * V;
+  const int64_t col0 = ((int64_t)blockIdx.x * kCeBwdBlock + threadIdx.x) * V - grid_off<T, V>(dst, c);
   if (col0 >= c) return;
-  if (VECOK && col0 + V <= c) {
-    const Vec<T, V> w = ld_stream(reinterpret_cast<const Vec<T, V>*>(xr + col0));
-    const Vec<T, V> wt = ld_stream(reinterpret_cast<const Vec<T, V>*>(tr + col0));
+  if (col0 >= 0 && col0 + V <= c) {
+    const Vec<T, V> w = ld_vec_any<true, T, V>(xr + col0);
+    const Vec<T, V> wt = ld_vec_any<true, T, V>(tr + col0);
     Vec<T, V> o;
 #pragma unroll
     for (int k = 0; k < V; ++k) {
       const float p = __builtin_amdgcn_exp2f(((float)to_arith(w.v[k]) - l) * kCeLog2e);
       o.v[k] = from_arith<T>(fmaf(p, Tr, -(float)to_arith(wt.v[k])) * g);
     }
-    st_stream(reinterpret_cast<Vec<T, V>*>(dst + col0), o);
+    st_vec_any<T, V>(dst + col0, o);
   } else {
-    for (int k = 0; k < V && col0 + k < c; ++k) {
+    for (int k = col0 < 0 ? (int)-col0 : 0; k < V && col0 + k < c; ++k) {
       const float p = __builtin_amdgcn_exp2f(((float)to_arith(xr[col0 + k]) - l) * kCeLog2e);
       dst[col0 + k] = from_arith<T>(fmaf(p, Tr, -(float)to_arith(tr[col0 + k])) * g);
     }
@@ -447,23 +507,22 @@ int supa_amd_cross_entropy_forward(const void* logits, int32_t dtype, const int6
   hipStream_t st = static_cast<hipStream_t>(stream);
   return with_ce_storage(dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
-    constexpr int V = CeVec<T>::V;
     float* rows = static_cast<float*>(workspace);
     T* o = static_cast<T*>(out);
     if (n > 0) {
       const T* x = static_cast<const T*>(logits);
       T* on = reduction == SUPA_AMD_REDUCTION_NONE ? o : nullptr;
-      if (aligned(logits, 16) && (c % V) == 0)
-        k_ce_fwd<T, true><<<(unsigned)n, kCeBlock, 0, st>>>(x, target, c, ignore_index, rows, lse, on, error_flag);
+      if ((c + CeVec<T>::V - 1) / CeVec<T>::V <= kCeWaveVecs)
+        k_ce_fwd<T, 64><<<(unsigned)((n + 3) / 4), kCeBlock, 0, st>>>(x, target, n, c, ignore_index, rows, lse, on,
+                                                                      error_flag);
       else
-        k_ce_fwd<T, false><<<(unsigned)n, kCeBlock, 0, st>>>(x, target, c, ignore_index, rows, lse, on, error_flag);
+        k_ce_fwd<T, kCeBlock><<<(unsigned)n, kCeBlock, 0, st>>>(x, target, n, c, ignore_index, rows, lse, on,
+                                                                error_flag);
       const int rc = launch_status();
       if (rc) return rc;
     }
     if (reduction == SUPA_AMD_REDUCTION_NONE) return SUPA_AMD_OK;
-    k_ce_final<T><<<1, kCeBlock, 0, st>>>(rows, target, n, c, ignore_index, reduction == SUPA_AMD_REDUCTION_MEAN ? 1 : 0,
-                                          o, count);
-    return launch_status();
+    return ce_final<T>(rows, target, n, c, ignore_index, reduction, o, count, st);
   });
 }
 
@@ -482,21 +541,16 @@ int supa_amd_cross_entropy_backward(const void* grad_out, const void* logits, in
   return with_ce_storage(dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     constexpr int V = CeVec<T>::V;
-    const bool vecok = aligned(logits, 16) && aligned(grad_logits, 16) && (c % V) == 0;
     const T* g = static_cast<const T*>(grad_out);
     const T* x = static_cast<const T*>(logits);
     T* gx = static_cast<T*>(grad_logits);
-    const unsigned gx_blocks = (unsigned)((c + (int64_t)kCeBwdBlock * V - 1) / ((int64_t)kCeBwdBlock * V));
+    const unsigned gx_blocks = (unsigned)((grid_vecs<T, V>(gx, c) + kCeBwdBlock - 1) / kCeBwdBlock);
     for (int64_t r0 = 0; r0 < n; r0 += 65535) {
       const int64_t rows = std::min<int64_t>(65535, n - r0);
       const T* gs = reduction == SUPA_AMD_REDUCTION_NONE ? g + r0 : g;
       const dim3 grid(gx_blocks, (unsigned)rows);
-      if (vecok)
-        k_ce_bwd<T, true><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, target + r0, lse + r0, count, c, ignore_index,
-                                                     reduction, gx + r0 * c);
-      else
-        k_ce_bwd<T, false><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, target + r0, lse + r0, count, c, ignore_index,
-                                                      reduction, gx + r0 * c);
+      k_ce_bwd<T><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, target + r0, lse + r0, count, c, ignore_index,
+                                                reduction, gx + r0 * c);
       const int rc = launch_status();
       if (rc) return rc;
     }
@@ -516,24 +570,18 @@ int supa_amd_cross_entropy_prob_forward(const void* logits, const void* target, 
   hipStream_t st = static_cast<hipStream_t>(stream);
   return with_ce_storage(dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
-    constexpr int V = CeVec<T>::V;
     float* rows = static_cast<float*>(workspace);
     T* o = static_cast<T*>(out);
     if (n > 0) {
       const T* x = static_cast<const T*>(logits);
       const T* t = static_cast<const T*>(target);
       T* on = reduction == SUPA_AMD_REDUCTION_NONE ? o : nullptr;
-      if (aligned(logits, 16) && aligned(target, 16) && (c % V) == 0)
-        k_ce_prob_fwd<T, true><<<(unsigned)n, kCeBlock, 0, st>>>(x, t, c, rows, lse, tsum, on);
-      else
-        k_ce_prob_fwd<T, false><<<(unsigned)n, kCeBlock, 0, st>>>(x, t, c, rows, lse, tsum, on);
+      k_ce_prob_fwd<T><<<(unsigned)n, kCeBlock, 0, st>>>(x, t, c, rows, lse, tsum, on);
       const int rc = launch_status();
       if (rc) return rc;
     }
     if (reduction == SUPA_AMD_REDUCTION_NONE) return SUPA_AMD_OK;
-    k_ce_final<T><<<1, kCeBlock, 0, st>>>(rows, nullptr, n, c, 0, reduction == SUPA_AMD_REDUCTION_MEAN ? 1 : 0, o,
-                                          nullptr);
-    return launch_status();
+    return ce_final<T>(rows, nullptr, n, c, 0, reduction, o, nullptr, st);
   });
 }
 
@@ -550,23 +598,18 @@ int supa_amd_cross_entropy_prob_backward(const void* grad_out, const void* logit
   return with_ce_storage(dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     constexpr int V = CeVec<T>::V;
-    const bool vecok = aligned(logits, 16) && aligned(target, 16) && aligned(grad_logits, 16) && (c % V) == 0;
     const T* g = static_cast<const T*>(grad_out);
     const T* x = static_cast<const T*>(logits);
     const T* t = static_cast<const T*>(target);
     T* gx = static_cast<T*>(grad_logits);
     const float inv_n = 1.0f / (float)n;
-    const unsigned gx_blocks = (unsigned)((c + (int64_t)kCeBwdBlock * V - 1) / ((int64_t)kCeBwdBlock * V));
+    const unsigned gx_blocks = (unsigned)((grid_vecs<T, V>(gx, c) + kCeBwdBlock - 1) / kCeBwdBlock);
     for (int64_t r0 = 0; r0 < n; r0 += 65535) {
       const int64_t rows = std::min<int64_t>(65535, n - r0);
       const T* gs = reduction == SUPA_AMD_REDUCTION_NONE ? g + r0 : g;
       const dim3 grid(gx_blocks, (unsigned)rows);
-      if (vecok)
-        k_ce_prob_bwd<T, true><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, t + r0 * c, lse + r0, tsum + r0, c,
-                                                          reduction, inv_n, gx + r0 * c);
-      else
-        k_ce_prob_bwd<T, false><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, t + r0 * c, lse + r0, tsum + r0, c,
-                                                           reduction, inv_n, gx + r0 * c);
+      k_ce_prob_bwd<T><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, t + r0 * c, lse + r0, tsum + r0, c, reduction,
+                                                     inv_n, gx + r0 * c);
       const int rc = launch_status();
       if (rc) return rc;
     }

@@ -71,22 +71,6 @@ __device__ __forceinline__ float block_sum_all(float v, float* lds) {
 // NaN, as in the upstream kernels.
 constexpr int kLsmGrid = 512;  // 2 workgroups per CU on MI355X's 256 CUs
 
-// (max, sum of exp) pairs of `width` lanes (a power of two; lanes w apart in
-// the XOR pattern hold the other pairs) combined: a max butterfly, one
-// rescale per lane to that max, and a sum butterfly -- one exponential per
-// lane where pairwise (m, s) combining takes two per step.  Every butterfly
-// step is symmetric in its operands, so every lane ends with the same value.
-template <int WIDTH>
-__device__ __forceinline__ void lanes_lse(float& m, float& s) {
-  float M = m;
-#pragma unroll
-  for (int off = WIDTH / 2; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-  s = lse_rescale(s, m, M);
-#pragma unroll
-  for (int off = WIDTH / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  m = M;
-}
-
 // ------------------------------------------------- rows in registers
 // G threads share a row: 16 or 64 lanes of a wavefront (a 256-thread workgroup
 // then holds 256 / G rows) or a workgroup of G = 256 or 512.  Thread l holds
@@ -715,34 +699,36 @@ __device__ __forceinline__ float split_rest(const T* row, int64_t cols, int nvec
   return last && i < cols ? (float)to_arith(row[i]) : -__builtin_inff();
 }
 
-// The backward, with three streams, takes the vectors of the 16-byte grid
-// instead, so that every access is aligned; row r starts o = r cols mod V
-// elements into its first one.  The elements of the first and the last vector
-// outside the row are never read or written: those vectors load and store
-// element by element, with zeros in the places outside.  bf16 [4096, 50257]:
-// 239 us, at element alignment 306 us (the forward 160 and 151 us; aligned
-// rows of 50304 193 and 133 us; streaming the rows twice by scalars, as rows
-// of odd length did before, 501 and 551 us).
+// The backward, with three streams, takes the vectors of the grid of 128-byte
+// lines of grad instead, so that every access is aligned and a wavefront
+// stores whole lines; a row starts o elements into its first line.  The
+// elements of a row's first and last partial vectors that lie outside the row
+// are never read or written: those vectors load and store element by element,
+// with zeros in the places outside.  bf16 [4096, 50257]: 233 us, on the
+// 16-byte grid 239, at element alignment 306 (the forward, 16-byte
+// grid and element alignment, 160 and 151 us;
+// aligned rows of 50304 193 and 133 us; streaming the rows twice by scalars,
+// as rows of odd length did before, 501 and 551 us).
 struct SplitRow {
-  int o;         // elements of the first vector that precede the row
+  int o;         // elements between the line boundary and the row
   int vf0, vf1;  // vectors wholly inside the row
-  int nvec;      // vectors the row touches
+  int nvec;      // one past the last vector the row touches
 };
 template <typename T, bool RAGGED>
-__device__ __forceinline__ SplitRow split_row(int row, int64_t cols) {
+__device__ __forceinline__ SplitRow split_row(int o, int64_t cols) {
   constexpr int V = VecOf<T>::V;
   SplitRow r;
-  r.o = RAGGED ? (int)(((int64_t)row * cols) % V) : 0;
-  r.vf0 = RAGGED && r.o ? 1 : 0;
+  r.o = RAGGED ? o : 0;
+  r.vf0 = RAGGED ? (r.o + V - 1) / V : 0;
   r.vf1 = (int)((r.o + cols) / V);
   r.nvec = RAGGED ? (int)((r.o + cols + V - 1) / V) : r.vf1;
   return r;
 }
-// The row's elements in vector v are [lo, hi) of its V.
+// The row's elements in vector v are [lo, hi) of its V (none before the row).
 template <typename T>
 __device__ __forceinline__ void split_edge(const SplitRow& r, int64_t cols, int v, int& lo, int& hi) {
   constexpr int V = VecOf<T>::V;
-  lo = v == 0 ? r.o : 0;
+  lo = max(r.o - v * V, 0);
   const int64_t left = r.o + cols - (int64_t)v * V;
   hi = left < V ? (int)left : V;
 }
@@ -980,7 +966,7 @@ k_lsm_bwd_split(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __
   __shared__ uint32_t lds_missing;
   const int row = (int)(blockIdx.x / (unsigned)K);
   const int part = (int)(blockIdx.x - (unsigned)row * (unsigned)K);
-  const SplitRow r = split_row<TG, RAGGED>(row, cols);
+  const SplitRow r = split_row<TG, RAGGED>(RAGGED ? grid_off<TG, VecOf<TG>::V>(grad + (int64_t)row * cols, cols) : 0, cols);
   const int nvec = r.nvec;
   const int base = part * plen;
   const int end = min(base + plen, nvec);
@@ -1123,8 +1109,9 @@ inline int split_part_len(int64_t nvec, int K, int part, int whole_from) {
   return (int)(((nvec + K - 1) / K + 63) / 64 * 64);
 }
 
-// The most 16-byte grid vectors a row of cols elements touches.
-inline int64_t split_vecs(int64_t cols, int v) { return cols % v == 0 ? cols / v : (cols + 2 * v - 2) / v; }
+// The most vectors a backward row of cols elements takes: those of the line
+// grid when cols is no multiple of the vector.
+inline int64_t split_vecs(int64_t cols, int v) { return cols % v == 0 ? cols / v : (cols + 8 * v - 1 + v - 1) / v; }
 
 // Aligned backward rows of 513 to 2048 whole vectors stay on the unguarded
 // 1024-thread kernels (bf16 [8192, 10000] 78 us against 88 on k_row_bwd,

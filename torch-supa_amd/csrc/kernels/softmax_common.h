@@ -105,6 +105,22 @@ __device__ __forceinline__ float lse_rescale(float s, float m, float M) {
   return M != -__builtin_inff() ? s * __builtin_amdgcn_exp2f((m - M) * kLog2e) : s;
 }
 
+// (max, sum of exp) pairs of `width` lanes (a power of two; lanes w apart in
+// the XOR pattern hold the other pairs) combined: a max butterfly, one
+// rescale per lane to that max, and a sum butterfly -- one exponential per
+// lane where pairwise (m, s) combining takes two per step.  Every butterfly
+// step is symmetric in its operands, so every lane ends with the same value.
+template <int WIDTH>
+__device__ __forceinline__ void lanes_lse(float& m, float& s) {
+  float M = m;
+#pragma unroll
+  for (int off = WIDTH / 2; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+  s = lse_rescale(s, m, M);
+#pragma unroll
+  for (int off = WIDTH / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  m = M;
+}
+
 template <typename F>
 int with_float_storage(int dtype, F&& f) {
   switch (dtype) {
