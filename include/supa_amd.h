@@ -763,6 +763,13 @@ int supa_amd_argext_rows(const void* in, int32_t dtype, const int64_t* in_idx, i
                          int64_t inner, int64_t chunk, int is_min, void* out_val,
                          int64_t* out_idx, void* stream);
 
+/* The same along the middle dim of a contiguous [outer, red, inner] input, read
+ * where it lies: the winner of each of the outer * inner positions, in that
+ * order.  SUPA_AMD_ELAYOUT (nothing launched) when inner is below one 16-byte
+ * vector or outer * inner or red exceed 32 bits. */
+int supa_amd_argext_dim(const void* in, int32_t dtype, int64_t outer, int64_t red, int64_t inner, int is_min,
+                        void* out_val, int64_t* out_idx, void* stream);
+
 /* Fused Adam (weight decay added to the gradient, upstream adam_math's
  * ADAM_MODE::ORIGINAL: grad += param * weight_decay after the maximize
  * negation); otherwise as supa_amd_fused_adamw.  Replaces _fused_adam_

@@ -94,3 +94,44 @@ def test_logsumexp_and_errors(no_fallback):
         torch.amax(torch.empty(3, 0, device="supa"), dim=1)
     with pytest.raises(RuntimeError):
         torch.max(torch.empty(0, device="supa"))
+
+
+# rows at the edges of a vector, of 16 / 64 / 256 threads and of a batch of
+# loads, off the vector's alignment; planes of the same reduced dim
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64, torch.uint8, torch.bool])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 255, 257, 1025, 4099, 16387, 40001])
+def test_rows_and_planes_at_the_edges(n, dtype, no_fallback):
+    base = data((5 * n + 3,), 114, dtype)
+    db = base.to("supa")
+    x, dx = base[3:].view(5, n), db[3:].view(5, n)
+    if dtype.is_floating_point and n > 2:
+        x[1, n // 2], x[1, n - 1] = float("nan"), float("nan")
+        x[2] = float("-inf")
+        x[3] = float("inf")
+        x[4, ::2], x[4, 1::2] = 0.0, -0.0
+        dx.copy_(x)
+    planes = base[: 5 * n].view(5, n).t().contiguous()  # [n, 5], and a batch of [n, 37]
+    wide = data((2, n, 37), 115, dtype) if n < 5000 else data((1, n, 17), 115, dtype)
+    if dtype.is_floating_point:
+        wide[:, n // 2, 5] = float("nan")
+        wide[:, :, 7] = float("-inf")
+    for c, d, dim in ((x, dx, 1), (planes, planes.to("supa"), 0), (wide, wide.to("supa"), 1),
+                      (wide.transpose(0, 1), wide.to("supa").transpose(0, 1), 0)):
+        for fn in (torch.max, torch.min):
+            gv, gi = fn(d, dim=dim)
+            wv, wi = fn(c, dim=dim)
+            eq(gv, wv)
+            eq(gi, wi)
+        eq(torch.amax(d, dim), torch.amax(c, dim))
+        if dtype != torch.bool:
+            eq(torch.argmin(d, dim, keepdim=True), torch.argmin(c, dim, keepdim=True))
+
+
+@pytest.mark.parametrize("shape", [(1, 5, 600001), (1, 70, 600001), (3, 19, 200003), (130, 300, 1030)])
+def test_planes_over_every_split(shape, no_fallback):
+    x = data(shape, 116, torch.float32)
+    x[:, shape[1] // 2, ::7] = float("nan")
+    gv, gi = torch.max(x.to("supa"), dim=1)
+    wv, wi = torch.max(x, dim=1)
+    eq(gv, wv)
+    eq(gi, wi)

@@ -11,11 +11,19 @@
 #include <tuple>
 
 #include "common.h"
+#include "dim_plan.h"
 
 namespace supa {
 namespace {
 
 constexpr int64_t kExtChunk = 16384;     // elements per workgroup in the first of two launches
+// A reduced dim with planes of positions behind it is read in place when they
+// make this many 16-byte vectors, or when it is short; fewer leave the chip to
+// a few workgroups' long walks and transposed rows are faster (float32
+// [4096, 4096] over dim 0, 1024 vectors: 96 us in place, 39 transposed;
+// [1000, 40000], 10000 vectors: 29 in place).
+constexpr int64_t kExtDimVecs = 8192;
+constexpr int64_t kExtDimShort = 64;
 constexpr int64_t kExtTwoPassRow = 65536;  // rows longer than this (with few rows) take two launches
 
 struct ExtResult {
@@ -57,6 +65,22 @@ ExtResult argext(const at::Tensor& self, std::vector<int64_t> dims, bool keepdim
   }
   for (int64_t d : dims) perm.push_back(d);
   const auto dev = self.device().index();
+  // one dim between or before kept ones: read where it lies
+  if (dims.size() == 1 && inner > 1 && self.numel() > 0) {
+    const DimPlan p = dim_plan(self, red);
+    const int64_t vec = 16 / (int64_t)self.element_size();
+    if (p.kind == DimPlan::kCols && p.inner >= vec && p.red < (int64_t(1) << 31) &&
+        (p.outer * p.inner / vec >= kExtDimVecs || p.red <= kExtDimShort)) {
+      ExtResult r;
+      if (want_val) r.values = empty_supa(oshape, self.scalar_type(), dev);
+      if (want_idx) r.indices = empty_supa(oshape, at::kLong, dev);
+      check_status(supa_amd_argext_dim(self.data_ptr(), dtype_code(self.scalar_type()), p.outer, p.red, p.inner,
+                                       is_min ? 1 : 0, want_val ? r.values.data_ptr() : nullptr,
+                                       want_idx ? r.indices.data_ptr<int64_t>() : nullptr, current_stream(dev)),
+                   name);
+      return r;
+    }
+  }
   at::Tensor rows = nd == 0 ? self.reshape({1}) : self.permute(perm).contiguous();
   const int64_t outer = inner > 0 ? rows.numel() / inner : 0;
   ExtResult r;
