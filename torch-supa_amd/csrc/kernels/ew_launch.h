@@ -189,6 +189,14 @@ int launch_static(const Op& op, const supa_amd_ew_desc& d, const int* tin, hipSt
       }
       int dense = 0;  // tensor inputs (not one-element broadcasts)
       for (int k = 1; k <= N; ++k) dense += a.mode[k] == 0 ? 1 : 0;
+      if constexpr (HasTable<Op>::value && std::is_same<OT, bf16>::value && (std::is_same<S, bf16>::value && ...)) {
+        if (dense == N && n >= kTabMin) {
+          const int64_t want = (n / VEC + kTabBlock - 1) / kTabBlock;
+          const int64_t grid = std::min<int64_t>(want, std::max<int64_t>(kTabGrid, want / kTabVecs));
+          k_contig_tab<Op><<<(unsigned)grid, kTabBlock, 0, st>>>(a, n);
+          return launch_status();
+        }
+      }
       const unsigned lds = CapsOccupancy<Op>::value && dense >= 3 && blocks >= (1 << 17) ? kStreamCapLds : 0u;
       k_contig<BS, VEC, Op, C, CT, OT, S...><<<dim3((unsigned)blocks), dim3(BS), lds, st>>>(op, a, n,
                                                                                             (uint32_t)nfull);

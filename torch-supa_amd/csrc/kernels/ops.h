@@ -128,12 +128,15 @@ template <typename C> __device__ __forceinline__ C gelu_none(C x) {
   if constexpr (std::is_same<C, float>::value) return (x * 0.5f) * (1.0f + sa_erff_nn(x * (float)kSqrt1_2));
   else return (x * C(0.5)) * (C(1) + erf(x * C(kSqrt1_2)));
 }
+__device__ __forceinline__ float gelu_tanh_inner(float x) {
+  const float x3 = (x * x) * x;
+  return (float)kGeluBetaTanh * fmaf((float)kGeluKappa, x3, x);
+}
 template <typename C> __device__ __forceinline__ C gelu_tanh(C x) {
-  const C x3 = (x * x) * x;
   if constexpr (std::is_same<C, float>::value) {
-    const float inner = (float)kGeluBetaTanh * fmaf((float)kGeluKappa, x3, x);
-    return (0.5f * x) * (1.0f + sa_tanhf_fast_nn(inner));  // a NaN x makes 0.5 x NaN
+    return (0.5f * x) * (1.0f + sa_tanhf_fast_nn(gelu_tanh_inner(x)));  // a NaN x makes 0.5 x NaN
   } else {
+    const C x3 = (x * x) * x;
     const C inner = C(kGeluBetaTanh) * fma(C(kGeluKappa), x3, x);
     return (C(0.5) * x) * (C(1) + tanh(inner));
   }
@@ -194,6 +197,21 @@ template <int K, typename C> struct UnaryOp {
   // activations keep one vector per thread: their ranges are branches, and
   // with two vectors live across them c1 gelu measured slower)
   static constexpr bool kHeavy = std::is_same<C, float>::value && (K == U_GELU_TANH || K == U_TANH);
+  // k_contig_tab: the tanh of input kTableArg as a table over bf16 magnitudes
+  static constexpr bool kTable = kHeavy;
+  static constexpr int kTableArg = 0;
+  __device__ __forceinline__ static float table(float x) {
+    if constexpr (K == U_GELU_TANH) return sa_tanhf_fast_nn(gelu_tanh_inner(x));
+    else return sa_tanhf(x);
+  }
+  __device__ __forceinline__ static float table_small(float x) {
+    return K == U_GELU_TANH ? (float)kGeluBetaTanh * x : x;
+  }
+  __device__ __forceinline__ static float with_table(const float* v, float t) {
+    const float x = v[0];
+    if constexpr (K == U_GELU_TANH) return (0.5f * x) * (1.0f + t);
+    else return x != x ? x : t;
+  }
   __device__ __forceinline__ C operator()(const C* v) const {
     const C x = v[0];
     if constexpr (K == U_GELU) return gelu_none<C>(x);
@@ -253,6 +271,25 @@ template <int K, typename C> struct UnaryOp {
 template <int K, typename C> struct UnaryBwdOp {
   static constexpr int arity = 2;
   static constexpr bool kHeavy = std::is_same<C, float>::value && K == U_GELU_TANH;
+  // k_contig_tab, as in UnaryOp
+  static constexpr bool kTable = kHeavy;
+  static constexpr int kTableArg = 1;
+  __device__ __forceinline__ static float table(float x) {
+    const float x2 = x * x;
+    return tanhx<float>((float)kGeluBetaTanh * muladd<float>((float)kGeluKappa, x2 * x, x));
+  }
+  __device__ __forceinline__ static float table_small(float x) { return (float)kGeluBetaTanh * x; }
+  __device__ __forceinline__ static C with_table(const C* v, C t) { return gelu_tanh_bwd(v[0], v[1], t); }
+  // 'tanh' from t = tanh(inner(x))
+  __device__ __forceinline__ static C gelu_tanh_bwd(C dy, C x, C t) {
+    const C left = C(0.5) * x;
+    const C right = C(1) + t;
+    const C left_d = C(0.5) * right;
+    const C right_d = muladd<C>(-t, t, C(1));
+    const C three_kappa = std::is_same<C, float>::value ? C(3.0f * (float)kGeluKappa) : C(3.0 * kGeluKappa);
+    const C inner_d = C(kGeluBetaTanh) * muladd<C>(three_kappa, x * x, C(1));
+    return dy * muladd<C>(left * right_d, inner_d, left_d);
+  }
   __device__ __forceinline__ C operator()(const C* v) const {
     const C dy = v[0], x = v[1];
     if constexpr (K == U_GELU || K == U_GELU_LOGERFC) {
@@ -266,14 +303,7 @@ template <int K, typename C> struct UnaryBwdOp {
       const C x2 = x * x;
       const C x3 = x2 * x;
       const C inner = C(kGeluBetaTanh) * muladd<C>(C(kGeluKappa), x3, x);
-      const C t = tanhx<C>(inner);
-      const C left = C(0.5) * x;
-      const C right = C(1) + t;
-      const C left_d = C(0.5) * right;
-      const C right_d = muladd<C>(-t, t, C(1));
-      const C three_kappa = std::is_same<C, float>::value ? C(3.0f * (float)kGeluKappa) : C(3.0 * kGeluKappa);
-      const C inner_d = C(kGeluBetaTanh) * muladd<C>(three_kappa, x2, C(1));
-      return dy * muladd<C>(left * right_d, inner_d, left_d);
+      return gelu_tanh_bwd(dy, x, tanhx<C>(inner));
     } else if constexpr (K == U_SILU) {
       const C s = C(1) / (C(1) + expx<C>(-x));
       return (dy * s) * muladd<C>(x, C(1) - s, C(1));
