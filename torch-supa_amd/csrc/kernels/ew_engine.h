@@ -427,11 +427,11 @@ k_contig_tab(TArgs<1 + Op::arity> a, int64_t n) {
 // before: [6007, 2047] + a row in float32 43.4 us, 17.0 now, in bf16 43.4, 9.6;
 // [5843, 8821] slices of odd rows in bf16: silu 173 us, 41 now, a product 173, 52.
 // Loads take no streaming hint: a run's ends share cache lines with its
-// neighbours and one-stream ops gain from what the last level still holds
-// (float32 silu of [4096, 11008] row slices 48.6 us, 55.9 with the hint; bf16
-// [32768, 4095] + a row 103, 119).  WHOLE is the variant for whole vectors
-// and two or more full-size inputs, which are streamed (those slices times a
-// dense tensor 82.0 us, 89.0 without the hint; bf16 41.2, 41.5).
+// neighbours (bf16 [32768, 4095] + a row 103 us, 119 with the hint).  WHOLE is
+// the variant for whole vectors, whose full-size inputs are streamed (float32
+// row slices [4096, 11008] times a dense tensor 82.0 us, 89.0 without the hint;
+// a gated activation of such slices, forward and backward over new buffers,
+// 268.5 us, 270.6 with the hint on two or more inputs only).
 template <int VEC, typename OFF, bool WHOLE, typename Op, typename C, typename CT, typename OT, typename... S>
 __global__ void __launch_bounds__(kStreamBlock)
 k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {

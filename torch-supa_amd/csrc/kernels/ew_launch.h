@@ -329,14 +329,14 @@ int launch_static(const Op& op, const supa_amd_ew_desc& d, const int* tin, hipSt
           if (b.st[k][j] == 0 && p.sizes[j] > 1) b.mode[k] = 1;
         streams += b.mode[k] ? 0 : 1;
       }
-      const bool whole = p.sizes[0] % VEC == 0 && streams >= 2;
+      const bool whole = p.sizes[0] % VEC == 0 && streams >= 1;
       NdGeom gv = g;
       gv.div[0] = FastDiv((uint32_t)ivec);
       const uint32_t nvec = (uint32_t)nvec64;
       const unsigned blocks = (nvec + kStreamBlock - 1) / kStreamBlock;
       auto go = [&](const auto& o) -> int {
         using O = std::remove_cv_t<std::remove_reference_t<decltype(o)>>;
-        if constexpr (N >= 2) {
+        if constexpr (N >= 1) {
           if (off32 && whole) {
             k_vecnd<VEC, int32_t, true, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
             return launch_status();
