@@ -65,6 +65,26 @@ def test_misaligned_and_sliced(off, dtype, no_fallback):
     exact(torch.cat(dh, -1), torch.cat(h, -1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.int64, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("cols", [2, 5, 16, 31, 32, 33, 510, 511, 512, 513])
+def test_slices_by_run_length(cols, dtype, no_fallback):
+    """Whole vectors aligned and not, and for 8-byte types the run lengths on
+    both sides of the line between vectors and single elements, with one and
+    with several full-size inputs."""
+    x, y = (seeded((9, 2 * cols + 3), 21) * 50).to(dtype), (seeded((9, cols + 1), 22) * 50).to(dtype)
+    m = seeded((9, cols), 23) > 0
+    dx, dy, dm = x.to("supa"), y.to("supa"), m.to("supa")
+    for o in (0, 1, 2, cols):
+        exact(-dx[:, o:o + cols], -x[:, o:o + cols])
+        exact(dx[:, o:o + cols] * dy[:, 1:], x[:, o:o + cols] * y[:, 1:])
+        exact(dx[:, o:o + cols] + dy[0, :cols], x[:, o:o + cols] + y[0, :cols])
+        exact(torch.where(dm, dx[:, o:o + cols], dy[:, :cols]), torch.where(m, x[:, o:o + cols], y[:, :cols]))
+    w, dw = x.clone(), dx.clone()
+    w[:, 1:1 + cols] *= y[:, :cols]
+    dw[:, 1:1 + cols] *= dy[:, :cols]
+    exact(dw, w)
+
+
 def test_masked_fill_shapes_and_errors(no_fallback):
     x = seeded((4, 1, 6), 8)
     m = seeded((5, 6), 9) > 0

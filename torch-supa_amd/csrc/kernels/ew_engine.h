@@ -8,9 +8,9 @@
 //           workgroups; the tail (< VEC elements) goes to the last one.
 //   VECND   N-d iteration where every operand's innermost stride is 1 (vector
 //           load, at any alignment) or 0 (one element broadcast across the
-//           vector) and the innermost dim holds at least one vector; a last
-//           short vector ends at the dim's end.  Coordinates of a vector's
-//           first element come from a chain of magic-number divisions; this
+//           vector): runs of whole vectors (k_vecnd), or of any length from
+//           one vector on, a last short one ending at the run's end
+//           (k_vecnd_any).  Coordinates of a vector's first element come from a chain of magic-number divisions; this
 //           covers a bias broadcast along rows of any width, a per-row scalar
 //           broadcast, slices of rows, misaligned views and inputs that are
 //           permuted but dense.
@@ -419,20 +419,12 @@ k_contig_tab(TArgs<1 + Op::arity> a, int64_t n) {
 // OFF: the offset type, int32_t when the host has checked that every
 // operand's largest offset fits (one 32-bit multiply per dim and operand
 // instead of a 64-bit product), int64_t otherwise.
-// g.div[0] divides by the vectors of an innermost run, ceil(inner / VEC); the
-// last vector of a run whose length is no multiple of VEC is moved back to
-// end at the run's end and stores only the elements no other vector covers
-// (so an output may still be an input).  Every access is at element
-// alignment.  Runs of odd length took one element per thread (k_strided)
-// before: [6007, 2047] + a row in float32 43.4 us, 17.0 now, in bf16 43.4, 9.6;
-// [5843, 8821] slices of odd rows in bf16: silu 173 us, 41 now, a product 173, 52.
-// Loads take no streaming hint: a run's ends share cache lines with its
-// neighbours (bf16 [32768, 4095] + a row 103 us, 119 with the hint).  WHOLE is
-// the variant for whole vectors, whose full-size inputs are streamed (float32
-// row slices [4096, 11008] times a dense tensor 82.0 us, 89.0 without the hint;
-// a gated activation of such slices, forward and backward over new buffers,
-// 268.5 us, 270.6 with the hint on two or more inputs only).
-template <int VEC, typename OFF, bool WHOLE, typename Op, typename C, typename CT, typename OT, typename... S>
+// Runs of whole vectors, at element alignment.  The position comes from the
+// element index v VEC and the innermost size: dividing v by a run's vectors
+// instead made the compiler wait for the divisor before it asked for the
+// strides (bf16 row slices [4096, 11008] times a dense tensor 42.7 us, 41.6
+// this way).
+template <int VEC, typename OFF, typename Op, typename C, typename CT, typename OT, typename... S>
 __global__ void __launch_bounds__(kStreamBlock)
 k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
   constexpr int N = sizeof...(S);
@@ -440,13 +432,7 @@ k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
   if (v >= nvec) return;
   // coordinates of the vector's first element
   uint32_t q, r;
-  g.div[0].divmod(v, q, r);
-  r *= VEC;
-  uint32_t skip = 0;
-  if (!WHOLE && r + VEC > g.size[0]) {
-    skip = r + VEC - g.size[0];
-    r = g.size[0] - VEC;
-  }
+  g.div[0].divmod(v * VEC, q, r);
   OFF off[1 + N];
 #pragma unroll
   for (int k = 0; k <= N; ++k) off[k] = (OFF)r * (OFF)a.st[k][0];
@@ -468,10 +454,10 @@ k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
          for (int k = 0; k < VEC; ++k) x[k][I] = s;
        } else {
          Vec<St, VEC> w;
-         if (!WHOLE || a.mode[1 + I]) {
-           if (WHOLE) asm volatile("");  // or the two loads become one, without the hint
+         if (a.mode[1 + I]) {
+           asm volatile("");  // or the two loads become one, without the hint
            w = ld_vec_any<false, St, VEC>(p);
-           if (WHOLE) asm volatile("");
+           asm volatile("");
          } else {
            w = ld_vec_any<true, St, VEC>(p);
          }
@@ -484,8 +470,67 @@ k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
   Vec<OT, VEC> w;
 #pragma unroll
   for (int k = 0; k < VEC; ++k) w.v[k] = from_arith<OT>(op(x[k]));
+  st_vec_any<OT, VEC>(static_cast<OT*>(a.p[0]) + off[0], w);
+}
+
+// Runs of any length and alignment, from one vector on.
+// g.div[0] divides by the vectors of an innermost run, ceil(inner / VEC); the
+// last vector of a run whose length is no multiple of VEC is moved back to
+// end at the run's end and stores only the elements no other vector covers
+// (so an output may still be an input).  Every access is at element
+// alignment.  Runs of odd length took one element per thread (k_strided)
+// before: [6007, 2047] + a row in float32 43.4 us, 17.0 now, in bf16 43.4, 9.6;
+// [5843, 8821] slices of odd rows in bf16: silu 173 us, 41 now, a product 173, 52.
+// Loads take no streaming hint: a run's ends share cache lines with its
+// neighbours (bf16 [32768, 4095] + a row 103 us, 119 with the hint).
+template <int VEC, typename OFF, typename Op, typename C, typename CT, typename OT, typename... S>
+__global__ void __launch_bounds__(kStreamBlock)
+k_vecnd_any(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
+  constexpr int N = sizeof...(S);
+  const uint32_t v = blockIdx.x * kStreamBlock + threadIdx.x;
+  if (v >= nvec) return;
+  // coordinates of the vector's first element
+  uint32_t q, r;
+  g.div[0].divmod(v, q, r);
+  r *= VEC;
+  uint32_t skip = 0;
+  if (r + VEC > g.size[0]) {
+    skip = r + VEC - g.size[0];
+    r = g.size[0] - VEC;
+  }
+  OFF off[1 + N];
+  off[0] = (OFF)r;
+#pragma unroll
+  for (int k = 1; k <= N; ++k) off[k] = (OFF)r * (OFF)a.st[k][0];
+  for (int d = 1; d < g.ndim; ++d) {
+    uint32_t qq, rr;
+    g.div[d].divmod(q, qq, rr);
+    q = qq;
+#pragma unroll
+    for (int k = 0; k <= N; ++k) off[k] += (OFF)rr * (OFF)a.st[k][d];
+  }
+  C x[VEC][N > 0 ? N : 1];
+  [&]<int... I>(std::integer_sequence<int, I...>) {
+    (([&] {
+       using St = typename NthT<I, S...>::type;
+       const St* p = static_cast<const St*>(a.p[1 + I]) + off[1 + I];
+       if (a.st[1 + I][0] == 0) {
+         const C s = load_cvt<C, CT>(p[0]);
+#pragma unroll
+         for (int k = 0; k < VEC; ++k) x[k][I] = s;
+       } else {
+         const Vec<St, VEC> w = ld_vec_any<false, St, VEC>(p);
+#pragma unroll
+         for (int k = 0; k < VEC; ++k) x[k][I] = load_cvt<C, CT>(w.v[k]);
+       }
+     }()),
+     ...);
+  }(std::make_integer_sequence<int, N>{});
+  Vec<OT, VEC> w;
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) w.v[k] = from_arith<OT>(op(x[k]));
   OT* dst = static_cast<OT*>(a.p[0]) + off[0];
-  if (WHOLE || skip == 0) {
+  if (skip == 0) {
     st_vec_any<OT, VEC>(dst, w);
   } else {
 #pragma unroll

@@ -315,35 +315,43 @@ int launch_static(const Op& op, const supa_amd_ew_desc& d, const int* tin, hipSt
       for (int j = 0; j < p.ndim; ++j) mx += (p.sizes[j] - 1) * (b.st[k][j] < 0 ? -b.st[k][j] : b.st[k][j]);
       if (mx >= (int64_t(1) << 31)) off32 = false;
     }
-    // VECND?  At least one vector a run, more runs than vectors fit 32 bits.
+    // VECND?  At least one vector a run, no more vectors than fit 32 bits.
     const int64_t ivec = VEC > 1 && p.ndim >= 1 ? (p.sizes[0] + VEC - 1) / VEC : 0;
     const int64_t nvec64 = ivec ? ivec * (pn / p.sizes[0]) : 0;
     bool vnd = VEC > 1 && p.ndim >= 1 && p.sizes[0] >= VEC && b.st[0][0] == 1 && nvec64 < (int64_t(1) << 31);
     for (int k = 1; k <= N && vnd; ++k) vnd = b.st[k][0] == 0 || b.st[k][0] == 1;
+    int streams = 0;  // inputs that move at full size
+    for (int k = 1; k <= N && vnd; ++k) {
+      // operands broadcast along some outer dim are re-read: keep them cached
+      b.mode[k] = 0;
+      for (int j = 1; j < p.ndim; ++j)
+        if (b.st[k][j] == 0 && p.sizes[j] > 1) b.mode[k] = 1;
+      streams += b.st[k][0] == 1 && b.mode[k] == 0 ? 1 : 0;
+    }
+    const bool whole = vnd && p.sizes[0] % VEC == 0;
+    // Two-element vectors (8-byte types) of runs of odd length, against one
+    // element a thread, which writes 512 whole bytes a wavefront: they lose on
+    // short runs, and with several full-size inputs also up to 512 elements and
+    // on tensors past the last-level cache.  Measured on MI355X, us, vectors /
+    // elements, float64: a negated slice of 5 columns 130 / 60, of 17 71 / 61,
+    // of 33 55 / 62, of 2047 44 / 60; a product of two slices of 257 columns 95
+    // / 68, of 513 60 / 68, [32768, 4095] 600 / 528.
+    if (VEC == 2 && !whole && (p.sizes[0] < 32 || (streams > 1 && (p.sizes[0] < 512 || pn >= (int64_t(3) << 23)))))
+      vnd = false;
     if (vnd) {
-      // operands broadcast along some outer dim are re-read: never streamed
-      int streams = 0;
-      for (int k = 1; k <= N; ++k) {
-        b.mode[k] = b.st[k][0] == 0 ? 1 : 0;
-        for (int j = 1; j < p.ndim; ++j)
-          if (b.st[k][j] == 0 && p.sizes[j] > 1) b.mode[k] = 1;
-        streams += b.mode[k] ? 0 : 1;
-      }
-      const bool whole = p.sizes[0] % VEC == 0 && streams >= 1;
       NdGeom gv = g;
-      gv.div[0] = FastDiv((uint32_t)ivec);
       const uint32_t nvec = (uint32_t)nvec64;
       const unsigned blocks = (nvec + kStreamBlock - 1) / kStreamBlock;
+      if (!whole) gv.div[0] = FastDiv((uint32_t)ivec);
       auto go = [&](const auto& o) -> int {
         using O = std::remove_cv_t<std::remove_reference_t<decltype(o)>>;
-        if constexpr (N >= 1) {
-          if (off32 && whole) {
-            k_vecnd<VEC, int32_t, true, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
-            return launch_status();
-          }
+        if (whole) {
+          if (off32) k_vecnd<VEC, int32_t, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
+          else k_vecnd<VEC, int64_t, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
+        } else {
+          if (off32) k_vecnd_any<VEC, int32_t, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
+          else k_vecnd_any<VEC, int64_t, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
         }
-        if (off32) k_vecnd<VEC, int32_t, false, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
-        else k_vecnd<VEC, int64_t, false, O, C, CT, OT, S...><<<blocks, kStreamBlock, 0, st>>>(o, b, gv, nvec);
         return launch_status();
       };
       if constexpr (IsRowB<Op>::value) {
