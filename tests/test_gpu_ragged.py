@@ -166,3 +166,32 @@ def test_fused_cross_entropy_of_odd_classes(c, dtype, no_fallback, fused_ce):
         tol = 1e-5 if dtype == torch.float32 else 1e-2
         torch.testing.assert_close(ld.detach().cpu().double(), lr.detach(), rtol=tol, atol=0)
         torch.testing.assert_close(d.grad.cpu().double(), r.grad, rtol=tol, atol=tol / n / 10)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("c", [1, 3, 7, 19, 255, 1001, 1024, 4100])
+def test_fused_cross_entropy_special_values(c, dtype, no_fallback, fused_ce):
+    """A NaN or +inf logit anywhere makes its row's loss and gradient NaN,
+    also where every logit that one thread holds is one; -inf logits count
+    nothing; a row of -inf alone is NaN.  Index and probability targets."""
+    rows, nan, inf = [], float("nan"), float("inf")
+    spans = sorted({(0, 1), (c // 2, c // 2 + 1), (c - 1, c), (0, min(c, 8)), (max(0, c - 9), c), (0, c)})
+    for lo, hi in spans:  # (span, its value, whether every other logit is -inf)
+        rows += [(lo, hi, nan, False), (lo, hi, nan, True), (lo, hi, inf, False), (lo, hi, -inf, False)]
+    x = seeded((len(rows), c), 24).to(dtype)
+    for i, (lo, hi, v, alone) in enumerate(rows):
+        if alone:
+            x[i] = -inf
+        x[i, lo:hi] = v
+    for at in (0, c - 1, c // 3):
+        t = torch.full((len(rows),), at)
+        prob = torch.softmax(seeded((len(rows), c), 25), 1).to(dtype)
+        for target in (t, prob):
+            d, r = x.to("supa").requires_grad_(), x.double().requires_grad_()
+            ld = F.cross_entropy(d, target.to("supa"), reduction="none")
+            lr = F.cross_entropy(r, target if target is t else target.double(), reduction="none")
+            ld.sum().backward()
+            lr.sum().backward()
+            tol = 1e-5 if dtype == torch.float32 else 1e-2
+            torch.testing.assert_close(ld.detach().cpu().double(), lr.detach(), rtol=tol, atol=tol, equal_nan=True)
+            torch.testing.assert_close(d.grad.cpu().double(), r.grad, rtol=tol, atol=tol, equal_nan=True)

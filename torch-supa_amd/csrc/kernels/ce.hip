@@ -50,14 +50,6 @@ __device__ __forceinline__ float ce_elem(const uint4& w, int k) {
   }
 }
 
-// (m, s) (+) (m2, s2) with s relative to m; a pair with m = -inf has s = 0.
-__device__ __forceinline__ void ce_combine(float& m, float& s, float m2, float s2) {
-  const float M = fmaxf(m, m2);
-  if (M != -__builtin_inff())
-    s = s * __builtin_amdgcn_exp2f((m - M) * kCeLog2e) + s2 * __builtin_amdgcn_exp2f((m2 - M) * kCeLog2e);
-  m = M;
-}
-
 __device__ __forceinline__ bool ce_kept(int64_t t, int64_t c, int64_t ignore_index) {
   return t != ignore_index && t >= 0 && t < c;
 }
@@ -127,24 +119,26 @@ k_ce_fwd(const T* __restrict__ x, const int64_t* __restrict__ target, int64_t n,
         for (int k = 0; k < V; ++k) mb = fmaxf(mb, ce_elem<T>(w[u], k));
       }
     }
-    const float M = fmaxf(m, mb);
-    if (M != -__builtin_inff()) {
-      float sb = 0.0f;
+    // fmaxf passes over a NaN, so M says nothing of them: the sum is always
+    // taken, and a NaN (or +inf) logit makes it, and the row's loss, NaN
+    const float M = fmaxf(m, mb), base = M == -__builtin_inff() ? 0.0f : M;
+    float sb = 0.0f;
 #pragma unroll
-      for (int u = 0; u < kCeUnroll; ++u) {
-        if (v0 + (int64_t)u * G < nvec) {
+    for (int u = 0; u < kCeUnroll; ++u) {
+      if (v0 + (int64_t)u * G < nvec) {
 #pragma unroll
-          for (int k = 0; k < V; ++k) sb += __builtin_amdgcn_exp2f((ce_elem<T>(w[u], k) - M) * kCeLog2e);
-        }
+        for (int k = 0; k < V; ++k) sb += __builtin_amdgcn_exp2f((ce_elem<T>(w[u], k) - base) * kCeLog2e);
       }
-      s = s * __builtin_amdgcn_exp2f((m - M) * kCeLog2e) + sb;
-      m = M;
     }
+    s = lse_rescale(s, m, M) + sb;
+    m = M;
   }
   // the elements after the whole vectors
   for (int64_t j = nvec * V + l; j < c; j += G) {
     const float xv = (float)to_arith(xr[j]);
-    ce_combine(m, s, xv, 1.0f);
+    const float M = fmaxf(m, xv), base = M == -__builtin_inff() ? 0.0f : M;
+    s = lse_rescale(s, m, M) + __builtin_amdgcn_exp2f((xv - base) * kCeLog2e);
+    m = M;
   }
   lanes_lse<64>(m, s);
   if constexpr (NW > 1) {
@@ -401,13 +395,14 @@ k_ce_prob_fwd(const T* __restrict__ x, const T* __restrict__ tgt, int64_t c, flo
             st.B = fmaf(tv, xv - M, st.B);
           }
         }
-    } else {  // every value so far -inf: s stays 0, B = sum t x
+    } else {  // every value so far -inf, or NaN: s stays 0, or NaN; B = sum t x
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if (v0 + (int64_t)u * kCeBlock < nvec) {
 #pragma unroll
           for (int k = 0; k < V; ++k) {
             const float xv = ce_elem<T>(wx[u], k), tv = ce_elem<T>(wt[u], k);
+            st.s += __builtin_amdgcn_exp2f(xv);
             st.T += tv;
             st.B = fmaf(tv, xv, st.B);
           }
