@@ -215,13 +215,15 @@ k_ce_final(float* __restrict__ loss_rows, const int64_t* __restrict__ target, in
     lds_c[wave] = k;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float sv = 0.0f, sk = 0.0f;
+  // the wavefronts' sums by a tree too: one after another their roundings, at
+  // the size of the whole sum, were half of the mean's error
+  float sv = lds_v[lane & (NW - 1)], sk = lds_c[lane & (NW - 1)];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      sv += lds_v[w];
-      sk += lds_c[w];
-    }
+  for (int off = NW / 2; off > 0; off >>= 1) {
+    sv += __shfl_xor(sv, off, 64);
+    sk += __shfl_xor(sk, off, 64);
+  }
+  if (threadIdx.x == 0) {
     if constexpr (PART) {  // every row of the chunk is read: the barrier
       loss_rows[(int64_t)blockIdx.x * kCeSumRows] = sv;
       loss_rows[(int64_t)blockIdx.x * kCeSumRows + 1] = sk;
