@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import oracle as O
+from helpers import bf16_ulp_dist
 
 pytestmark = pytest.mark.gpu
 
@@ -28,14 +29,26 @@ def planes_of(a, shape):
     return np.moveaxis(a.reshape(shape[0], shape[2], shape[1]), 2, 1)
 
 
-# one unit in the last place of each type, relative: 16-bit results are one
-# rounding of a float32 value, so they move by at most one unit
+def check_forward(got, ref, dtype):
+    got = got.cpu()
+    if dtype == torch.float32:
+        np.testing.assert_allclose(got.numpy(), ref, rtol=1e-5, atol=1e-6)
+    else:  # one rounding to the storage type of a float32 value: at most one unit in the last place
+        r = torch.from_numpy(np.ascontiguousarray(ref)).to(dtype)
+        a, b = (v.view(torch.int16).numpy().view(np.uint16) for v in (got.contiguous(), r))
+        assert bf16_ulp_dist(a, b).max() <= 1
+
+
+# a 16-bit gradient is one rounding too, of a difference whose terms' sum moves
+# by `atol`: one unit in the last place, relative, on top of that
 ULP = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
+# the smallest gradients: float32's own floor, half a unit of a float16 subnormal
+FLOOR = {torch.float32: 1e-6, torch.bfloat16: 0.0, torch.float16: 2.0 ** -24}
 
 
-def check(got, ref, dtype, atol=0.0):
+def check_gradient(got, ref, dtype, atol):
     err = np.abs(got.cpu().float().numpy() - ref)
-    assert (err <= ULP[dtype] * np.abs(ref) + 1e-6 + atol).all()
+    assert (err <= ULP[dtype] * np.abs(ref) + FLOOR[dtype] + (1 + ULP[dtype]) * atol).all(), float(err.max())
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
@@ -50,7 +63,7 @@ def test_spatial_softmax_matches_oracle(shape, dtype, no_fallback):
                                       (False, torch.softmax, SM_BWD, O.softmax, O.softmax_backward)):
         y = fwd(dx, 1)
         assert y.is_contiguous()
-        check(y, planes_of(ofwd(rows_of(x)), shape), dtype)
+        check_forward(y, planes_of(ofwd(rows_of(x)), shape), dtype)
         gi = bwd(dg, y, 1, dtype)
         # a gradient is p (g - S) or g - p S: two float32 sums of the same C
         # terms differ by at most 2 (chain) 2^-24 sum|term|, chains of at most
@@ -58,7 +71,7 @@ def test_spatial_softmax_matches_oracle(shape, dtype, no_fallback):
         yc = y.cpu().double().numpy()
         p, terms = (np.exp(yc), g.double().numpy()) if log else (yc, g.double().numpy() * yc)
         atol = 2 * (shape[1] / 16 + 16) * 2.0 ** -24 * np.abs(terms).sum(1, keepdims=True) * p
-        check(gi, planes_of(obwd(rows_of(g), rows_of(y.cpu())), shape), dtype, atol)
+        check_gradient(gi, planes_of(obwd(rows_of(g), rows_of(y.cpu())), shape), dtype, atol)
 
 
 @pytest.mark.parametrize("shape", [(2, 19, 37), (2, 300, 4101), (2, 5, 3)])
