@@ -1,18 +1,8 @@
-"""log_softmax and softmax over a dim that is not the last one (the spatial
-kernels): class counts around the edges of each split of the classes over
-class groups, planes of every remainder of the vector, special values, and
-the output written over the input."""
-import numpy as np
-import pytest
-import torch
-
-import oracle as O
-from helpers import bf16_ulp_dist
-
-pytestmark = pytest.mark.gpu
-
-LSM_BWD = torch.ops.aten._log_softmax_backward_data
-SM_BWD = torch.ops.aten._softmax_backward_data
+# a 16-bit gradient is one rounding too, of a difference whose terms' sum moves
+# by `atol`: one unit in the last place, relative, on top of that
+ULP = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
+# the smallest gradients: float32's own floor, half a unit of a float16 subnormal
+FLOOR = {torch.float32: 1e-6, torch.bfloat16: 0.0, torch.float16: 2.0 ** -24}
 
 
 def seeded(shape, seed, scale=1.0, dtype=torch.float32):
@@ -104,3 +94,22 @@ def test_spatial_softmax_layouts_and_special_values(no_fallback):
     assert h.dtype == torch.float32
     np.testing.assert_allclose(h.cpu().numpy(), torch.log_softmax(seeded((2, 5, 9), 6, 2.0, torch.bfloat16).float(), 1),
                                rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("log", [True, False])
+def test_more_positions_than_one_launch(log, no_fallback):
+    """2^28 positions of 33 classes: more threads than a launch holds."""
+    if torch.supa.mem_get_info()[0] < 80 << 30:
+        pytest.skip("takes 54 GiB of device memory")
+    f = torch.log_softmax if log else torch.softmax
+    small = seeded((64, 33, 2), 12, 2.0, torch.bfloat16).to("supa")
+    want = f(small, 1)
+    x = torch.empty(1 << 21, 64, 33, 2, dtype=torch.bfloat16, device="supa")
+    x.copy_(small)
+    y = f(x.view(-1, 33, 2), 1).view_as(x)
+    for i in (0, (1 << 20) - 1, 1 << 20, (1 << 21) - 3, (1 << 21) - 1):
+        assert torch.equal(y[i].cpu(), want.cpu())
+    del x
+    assert bool((y == want).all())
+    del y
+    torch.supa.empty_cache()

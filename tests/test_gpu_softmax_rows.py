@@ -1,19 +1,5 @@
-"""Row softmax, log_softmax and their gradients at the edges of the row
-kernels: the longest row of each thread split and one element more, rows of
-every remainder of the vector, rows whose base is not 16-byte aligned, the
-output over the input, special values in every position of a short row."""
-import numpy as np
-import pytest
-import torch
-
-import oracle as O
-from helpers import bf16_ulp_dist
-
-pytestmark = pytest.mark.gpu
-
-LSM_BWD = torch.ops.aten._log_softmax_backward_data
-SM_BWD = torch.ops.aten._softmax_backward_data
-ULP = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
+# vectors a row: the last of each thread split, and one more
+VECS = [1, 2, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 2560, 2561, 5121]
 
 
 def seeded(shape, seed, scale=1.0, dtype=torch.float32):
@@ -29,8 +15,8 @@ def shifted(t):
     return v
 
 
-# the smallest gradients: float32's own floor, half a unit of a float16 subnormal
-FLOOR = {torch.float32: 1e-6, torch.bfloat16: 0.0, torch.float16: 2.0 ** -24}
+# vectors a row: the last of each thread split, and one more
+VECS = [1, 2, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 2560, 2561, 5121]
 
 
 def check_forward(got, ref, dtype, atol):
@@ -77,6 +63,25 @@ def test_rows_at_the_edges(vecs, dtype, no_fallback):
         x, g = seeded((rows, cols), cols, 2.0, dtype), seeded((rows, cols), cols + 1, 1.0, dtype)
         compare(x, g, dtype, lambda t: t.to("supa"))
         compare(x, g, dtype, shifted)
+
+
+def test_more_rows_than_one_launch(no_fallback):
+    """2^28 rows of 8: more threads than a launch holds."""
+    if torch.supa.mem_get_info()[0] < 30 << 30:
+        pytest.skip("takes 14 GiB of device memory")
+    small, g = (seeded((64, 8), 12 + i, 2.0, torch.bfloat16).to("supa") for i in range(2))
+    x = torch.empty(1 << 22, 64, 8, dtype=torch.bfloat16, device="supa")
+    for f, b in ((torch.log_softmax, LSM_BWD), (torch.softmax, SM_BWD)):
+        want = f(small, 1)
+        x.copy_(small)
+        y = f(x.view(-1, 8), 1)
+        assert bool((y.view_as(x) == want).all())
+        x.copy_(g)
+        gi = b(x.view(-1, 8), y, 1, torch.bfloat16)
+        assert bool((gi.view_as(x) == b(g, want, 1, torch.bfloat16)).all())
+        del y, gi
+    del x
+    torch.supa.empty_cache()
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

@@ -248,37 +248,52 @@ k_row_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restri
   if (VW > 1 && l < rest) dst[nvec * VW + l] = from_arith<TO>(res(gt, yt));
 }
 
-// Calls launch(VW, G, NV as integral constants, workgroups) for a row of
-// `cols` elements in vectors of V; false when the row has more than MAXV
-// vectors.  Up to 16 elements one lane per element; else the fewest lanes
-// that hold the row in one vector each (16, 64), then 2, 4 and 8 vectors a
-// lane of one wavefront, then workgroups: forward 256 threads by 4 and 512 by
-// 4 or 5, backward 1024 by 1 or 2 (bf16 [8192, 8192] forward 45 us against 56
-// with 1024 threads, backward 64 us against 66 with 256).
+// Calls launch(VW, G, NV as integral constants, first row, rows, workgroups)
+// for rows of `cols` elements in vectors of V and stores its status in rc;
+// false when a row has more than MAXV vectors.  Up to 16 elements one lane per
+// element; else the fewest lanes that hold the row in one vector each (16,
+// 64), then 2, 4 and 8 vectors a lane of one wavefront, then workgroups:
+// forward 256 threads by 4 and 512 by 4 or 5, backward 1024 by 1 or 2 (bf16
+// [8192, 8192] forward 45 us against 56 with 1024 threads, backward 64 us
+// against 66 with 256).
+// Launches stay below HIP's 2^32 threads: more rows go in several.
 template <int V, int MAXV, bool BWD, typename F>
-bool row_split(int64_t rows, int64_t cols, F&& launch) {
+bool row_split(int64_t rows, int64_t cols, int& rc, F&& launch) {
   using std::integral_constant;
   const int64_t nv = (cols + V - 1) / V;
   if (nv > MAXV) return false;
+  rc = SUPA_AMD_OK;
   auto go = [&](auto vw, auto g, auto n) {
     const int64_t per = g.value <= 64 ? 256 / g.value : 1;
-    launch(vw, g, n, (unsigned)((rows + per - 1) / per));
+    const int64_t slab = per * (((int64_t(1) << 32) - 1) / row_block<g.value>());
+    for (int64_t r0 = 0; r0 < rows && rc == SUPA_AMD_OK; r0 += slab) {
+      const int64_t nr = std::min(slab, rows - r0);
+      rc = launch(vw, g, n, r0, nr, (unsigned)((nr + per - 1) / per));
+    }
+    return true;
   };
   using I1 = integral_constant<int, 1>;
+  using I2 = integral_constant<int, 2>;
+  using I4 = integral_constant<int, 4>;
   using IV = integral_constant<int, V>;
-  if (cols <= 16) go(I1{}, integral_constant<int, 16>{}, I1{});
-  else if (nv <= 16) go(IV{}, integral_constant<int, 16>{}, I1{});
-  else if (nv <= 64) go(IV{}, integral_constant<int, 64>{}, I1{});
-  else if (nv <= 128) go(IV{}, integral_constant<int, 64>{}, integral_constant<int, 2>{});
-  else if (nv <= 256) go(IV{}, integral_constant<int, 64>{}, integral_constant<int, 4>{});
-  else if (nv <= 512) go(IV{}, integral_constant<int, 64>{}, integral_constant<int, 8>{});
-  else if constexpr (BWD) {
-    if (nv <= 1024) go(IV{}, integral_constant<int, 1024>{}, I1{});
-    else go(IV{}, integral_constant<int, 1024>{}, integral_constant<int, 2>{});
-  } else if (nv <= 1024) go(IV{}, integral_constant<int, 256>{}, integral_constant<int, 4>{});
-  else if (nv <= 2048) go(IV{}, integral_constant<int, 512>{}, integral_constant<int, 4>{});
-  else go(IV{}, integral_constant<int, 512>{}, integral_constant<int, MAXV / 512>{});
-  return true;
+  using G16 = integral_constant<int, 16>;
+  using G64 = integral_constant<int, 64>;
+  using G256 = integral_constant<int, 256>;
+  using G512 = integral_constant<int, 512>;
+  using G1024 = integral_constant<int, 1024>;
+  if (cols <= 16) return go(I1{}, G16{}, I1{});
+  if (nv <= 16) return go(IV{}, G16{}, I1{});
+  if (nv <= 64) return go(IV{}, G64{}, I1{});
+  if (nv <= 128) return go(IV{}, G64{}, I2{});
+  if (nv <= 256) return go(IV{}, G64{}, I4{});
+  if (nv <= 512) return go(IV{}, G64{}, integral_constant<int, 8>{});
+  if constexpr (BWD) {
+    return nv <= 1024 ? go(IV{}, G1024{}, I1{}) : go(IV{}, G1024{}, I2{});
+  } else {
+    if (nv <= 1024) return go(IV{}, G256{}, I4{});
+    if (nv <= 2048) return go(IV{}, G512{}, I4{});
+    return go(IV{}, G512{}, integral_constant<int, MAXV / 512>{});
+  }
 }
 
 template <typename TI, typename TO, int VPT, bool LOG>
@@ -1116,7 +1131,10 @@ inline int64_t split_vecs(int64_t cols, int v) { return cols % v == 0 ? cols / v
 // Aligned backward rows of 513 to 2048 whole vectors stay on the unguarded
 // 1024-thread kernels (bf16 [8192, 10000] 78 us against 88 on k_row_bwd,
 // [4096, 16384] 62 against 65; float32 rows within 2 %).
-inline bool bwd_reg_rows(int64_t cols, int v) { return cols % v == 0 && cols / v > 512 && cols / v <= 2 * kRowBlock; }
+// Not past 2^22 rows, 2^32 threads.
+inline bool bwd_reg_rows(int64_t rows, int64_t cols, int v) {
+  return cols % v == 0 && cols / v > 512 && cols / v <= 2 * kRowBlock && rows < (int64_t(1) << 22);
+}
 
 template <bool LOG>
 int softmax_forward(const void* in, int32_t in_dtype, void* out, int32_t out_dtype, int64_t rows, int64_t cols,
@@ -1141,11 +1159,14 @@ int softmax_forward(const void* in, int32_t in_dtype, void* out, int32_t out_dty
             <<<(unsigned)std::min<int64_t>(rows, kLsmGrid), kRowBlock, 0, st>>>(pi, po, rows, cols);
         return launch_status();
       }
-      if (row_split<V, kSplitBlock * kFwdNV, false>(rows, cols, [&](auto vw, auto g, auto nv, unsigned blocks) {
-            k_row_fwd<TI, TO, vw.value, g.value, nv.value, LOG>
-                <<<blocks, row_block<g.value>(), 0, st>>>(pi, po, rows, (int)cols);
-          }))
-        return launch_status();
+      int rc;
+      if (row_split<V, kSplitBlock * kFwdNV, false>(
+              rows, cols, rc, [&](auto vw, auto g, auto nv, int64_t r0, int64_t nr, unsigned blocks) {
+                k_row_fwd<TI, TO, vw.value, g.value, nv.value, LOG>
+                    <<<blocks, row_block<g.value>(), 0, st>>>(pi + r0 * cols, po + r0 * cols, nr, (int)cols);
+                return launch_status();
+              }))
+        return rc;
       const int64_t nvec = (cols + V - 1) / V;
       const int K = split_parts(nvec, kSplitBlock * kFwdNV, in, nullptr, rows * cols * (int64_t)sizeof(TI), out,
                                 rows * cols * (int64_t)sizeof(TO));
@@ -1213,16 +1234,19 @@ int supa_amd_log_softmax_backward(const void* grad, const void* output, int32_t 
       TO* po = static_cast<TO*>(grad_in);
       const bool al = aligned(grad, 16) && aligned(output, 16) && aligned(grad_in, 16);
       const int64_t nvec = split_vecs(cols, V);
-      if (al && bwd_reg_rows(cols, V)) {
+      if (al && bwd_reg_rows(rows, cols, V)) {
         if (nvec <= kRowBlock) k_lsm_bwd_reg<TG, TO, 1><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         else k_lsm_bwd_reg<TG, TO, 2><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         return launch_status();
       }
-      if (row_split<V, kSplitBlock * kBwdNV, true>(rows, cols, [&](auto vw, auto g, auto nv, unsigned blocks) {
-            k_row_bwd<TG, TO, vw.value, g.value, nv.value, true>
-                <<<blocks, row_block<g.value>(), 0, st>>>(pg, py, po, rows, (int)cols);
-          }))
-        return launch_status();
+      int rc;
+      if (row_split<V, kSplitBlock * kBwdNV, true>(
+              rows, cols, rc, [&](auto vw, auto g, auto nv, int64_t r0, int64_t nr, unsigned blocks) {
+                k_row_bwd<TG, TO, vw.value, g.value, nv.value, true><<<blocks, row_block<g.value>(), 0, st>>>(
+                    pg + r0 * cols, py + r0 * cols, po + r0 * cols, nr, (int)cols);
+                return launch_status();
+              }))
+        return rc;
       const int K = al ? split_parts(nvec, kSplitBlock * kBwdNV, grad, output, rows * cols * (int64_t)sizeof(TG),
                                      grad_in, rows * cols * (int64_t)sizeof(TO))
                        : 0;
@@ -1273,16 +1297,19 @@ int supa_amd_softmax_backward(const void* grad, const void* output, int32_t gy_d
       const TG* pg = static_cast<const TG*>(grad);
       const TG* py = static_cast<const TG*>(output);
       TO* po = static_cast<TO*>(grad_in);
-      if (reg_ok && bwd_reg_rows(cols, V)) {
+      if (reg_ok && bwd_reg_rows(rows, cols, V)) {
         if (cols / V <= kRowBlock) k_sm_bwd_reg<TG, TO, 1><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         else k_sm_bwd_reg<TG, TO, 2><<<(unsigned)rows, kRowBlock, 0, st>>>(pg, py, po, cols);
         return launch_status();
       }
-      if (row_split<V, kSplitBlock * kBwdNV, true>(rows, cols, [&](auto vw, auto g, auto nv, unsigned blocks) {
-            k_row_bwd<TG, TO, vw.value, g.value, nv.value, false>
-                <<<blocks, row_block<g.value>(), 0, st>>>(pg, py, po, rows, (int)cols);
-          }))
-        return launch_status();
+      int rc;
+      if (row_split<V, kSplitBlock * kBwdNV, true>(
+              rows, cols, rc, [&](auto vw, auto g, auto nv, int64_t r0, int64_t nr, unsigned blocks) {
+                k_row_bwd<TG, TO, vw.value, g.value, nv.value, false><<<blocks, row_block<g.value>(), 0, st>>>(
+                    pg + r0 * cols, py + r0 * cols, po + r0 * cols, nr, (int)cols);
+                return launch_status();
+              }))
+        return rc;
       if (reg_ok) {
         const int64_t nvec = cols / V;
         const int vpt = (int)((nvec + kRowBlock - 1) / kRowBlock);

@@ -76,6 +76,7 @@ __device__ __forceinline__ void dim_store(TO* p, const float (&f)[VW], int skip)
 
 struct DimGeom {
   uint32_t npos;    // position vectors: outer * ceil(inner / VW)
+  uint32_t first;   // the launch's first one
   FastDiv ivec;     // vectors per plane
   uint32_t cols;
   int64_t inner;
@@ -91,7 +92,7 @@ struct DimPlace {
 template <int VW, int TXL>
 __device__ __forceinline__ DimPlace dim_place(const DimGeom& g) {
   const uint32_t tx = threadIdx.x & ((1u << TXL) - 1u);
-  const uint32_t p = blockIdx.x * (1u << TXL) + tx;
+  const uint32_t p = g.first + blockIdx.x * (1u << TXL) + tx;
   DimPlace r{0, 0, p < g.npos};
   uint32_t o, v;
   g.ivec.divmod(p, o, v);
@@ -331,45 +332,59 @@ inline bool dim_geom(DimGeom& g, int64_t outer, int64_t cols, int64_t inner, int
   const int64_t ivec = (inner + vw - 1) / vw;
   if (cols >= (int64_t(1) << 31) || ivec >= (int64_t(1) << 31) || outer * ivec >= (int64_t(1) << 31)) return false;
   g.npos = (uint32_t)(outer * ivec);
+  g.first = 0;
   g.ivec = FastDiv((uint32_t)ivec);
   g.cols = (uint32_t)cols;
   g.inner = inner;
   return true;
 }
 
-// Calls launch(TXL, NC, HOLD as integral constants, blocks) with the split of
-// the classes over class groups.
+// Calls launch(TXL, NC, HOLD as integral constants, workgroups) with the split
+// of the classes over class groups, once per slab of positions (g.first): HIP
+// takes fewer than 2^32 threads a launch.
 template <int NCMAX, typename F>
-void dim_split(const DimGeom& g, F&& launch) {
-  auto blocks = [&](int txl) { return (unsigned)(((uint64_t)g.npos + (1u << txl) - 1) >> txl); };
+int dim_split(DimGeom& g, F&& launch) {
   using std::integral_constant;
   constexpr int H = NCMAX / 2;
-  if (g.cols <= H) launch(integral_constant<int, 8>{}, integral_constant<int, H>{}, std::true_type{}, blocks(8));
-  else if (g.cols <= 4 * H) launch(integral_constant<int, 6>{}, integral_constant<int, H>{}, std::true_type{}, blocks(6));
-  else if (g.cols <= 16 * H) launch(integral_constant<int, 4>{}, integral_constant<int, H>{}, std::true_type{}, blocks(4));
-  else if (g.cols <= 16 * NCMAX)
-    launch(integral_constant<int, 4>{}, integral_constant<int, NCMAX>{}, std::true_type{}, blocks(4));
-  else launch(integral_constant<int, 4>{}, integral_constant<int, H>{}, std::false_type{}, blocks(4));
+  auto go = [&](auto txl, auto nc, auto hold) -> int {
+    constexpr uint64_t slab = (((uint64_t(1) << 32) - 1) / kDimBlock) << txl.value;
+    for (uint64_t p0 = 0; p0 < g.npos; p0 += slab) {
+      g.first = (uint32_t)p0;
+      const uint64_t n = std::min<uint64_t>(slab, g.npos - p0);
+      const int rc = launch(txl, nc, hold, (unsigned)((n + (1u << txl.value) - 1) >> txl.value));
+      if (rc) return rc;
+    }
+    return SUPA_AMD_OK;
+  };
+  using X8 = integral_constant<int, 8>;
+  using X6 = integral_constant<int, 6>;
+  using X4 = integral_constant<int, 4>;
+  using NH = integral_constant<int, H>;
+  if (g.cols <= H) return go(X8{}, NH{}, std::true_type{});
+  if (g.cols <= 4 * H) return go(X6{}, NH{}, std::true_type{});
+  if (g.cols <= 16 * H) return go(X4{}, NH{}, std::true_type{});
+  if (g.cols <= 16 * NCMAX) return go(X4{}, integral_constant<int, NCMAX>{}, std::true_type{});
+  return go(X4{}, NH{}, std::false_type{});
 }
 
 template <typename TI, typename TO, int VW, bool LOG>
 int dim_forward(const TI* in, TO* out, int64_t outer, int64_t cols, int64_t inner, hipStream_t st) {
   DimGeom g;
   if (!dim_geom(g, outer, cols, inner, VW)) return SUPA_AMD_ELAYOUT;
-  dim_split<16>(g, [&](auto txl, auto nc, auto hold, unsigned blocks) {
+  return dim_split<16>(g, [&](auto txl, auto nc, auto hold, unsigned blocks) {
     k_dim_fwd<TI, TO, VW, txl.value, nc.value, hold.value, LOG><<<blocks, kDimBlock, 0, st>>>(in, out, g);
+    return launch_status();
   });
-  return launch_status();
 }
 
 template <typename TG, typename TO, int VW, bool LOG>
 int dim_backward(const TG* grad, const TG* y, TO* gin, int64_t outer, int64_t cols, int64_t inner, hipStream_t st) {
   DimGeom g;
   if (!dim_geom(g, outer, cols, inner, VW)) return SUPA_AMD_ELAYOUT;
-  dim_split<16>(g, [&](auto txl, auto nc, auto hold, unsigned blocks) {
+  return dim_split<16>(g, [&](auto txl, auto nc, auto hold, unsigned blocks) {
     k_dim_bwd<TG, TO, VW, txl.value, nc.value, hold.value, LOG><<<blocks, kDimBlock, 0, st>>>(grad, y, gin, g);
+    return launch_status();
   });
-  return launch_status();
 }
 
 }  // namespace sa
