@@ -135,3 +135,18 @@ def test_planes_over_every_split(shape, no_fallback):
     wv, wi = torch.max(x, dim=1)
     eq(gv, wv)
     eq(gi, wi)
+
+
+def test_more_rows_than_one_launch(no_fallback):
+    """2^28 rows of 8: more threads than a launch holds."""
+    if torch.supa.mem_get_info()[0] < 40 << 30:
+        pytest.skip("takes 9 GiB of device memory")
+    small = torch.randn(65, 8, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to("supa")
+    x = torch.empty(1 << 22, 65, 8, dtype=torch.bfloat16, device="supa")
+    x.copy_(small)
+    v, i = x.view(-1, 8).max(1)
+    wv, wi = small.max(1)
+    del x
+    assert bool((v.view(-1, 65) == wv).all()) and bool((i.view(-1, 65) == wi).all())
+    del v, i
+    torch.supa.empty_cache()

@@ -131,3 +131,17 @@ def test_moments_at_the_edges_of_a_chunk(dtype, vecs, no_fallback):
             var, mean = torch.var_mean(t.to("supa"), dim=dims)
             torch.testing.assert_close(var.cpu().double(), t.double().var(dim=dims), rtol=RTOL[dtype], atol=0)
             torch.testing.assert_close(mean.cpu().double(), t.double().mean(dim=dims), rtol=RTOL[dtype], atol=0)
+
+
+def test_more_rows_than_one_launch(no_fallback):
+    """2^24 rows of a workgroup each: more threads than a launch holds."""
+    if torch.supa.mem_get_info()[0] < 120 << 30:
+        pytest.skip("takes 65 GiB of device memory")
+    small = torch.randn(256, 2064, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to("supa")
+    x = torch.empty((1 << 16) + 1, 256, 2064, dtype=torch.bfloat16, device="supa")
+    x.copy_(small)
+    var, mean = torch.var_mean(x.view(-1, 2064), dim=1)
+    wv, wm = torch.var_mean(small, dim=1)
+    del x
+    assert bool((var.view(-1, 256) == wv).all()) and bool((mean.view(-1, 256) == wm).all())
+    torch.supa.empty_cache()

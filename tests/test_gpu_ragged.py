@@ -197,6 +197,24 @@ def test_fused_cross_entropy_special_values(c, dtype, no_fallback, fused_ce):
             torch.testing.assert_close(d.grad.cpu().double(), r.grad, rtol=tol, atol=tol, equal_nan=True)
 
 
+@pytest.mark.parametrize("prob", [False, True])
+def test_cross_entropy_of_more_rows_than_one_launch(prob, no_fallback, fused_ce):
+    """2^26 rows (2^24 with probability targets): more threads than a launch holds."""
+    if torch.supa.mem_get_info()[0] < 20 << 30:
+        pytest.skip("takes 4 GiB of device memory")
+    n = 1 << (18 if prob else 20)
+    small = seeded((65, 4), 32).to("supa")
+    st = torch.softmax(seeded((65, 4), 33), 1).to("supa") if prob else (torch.arange(65) % 4).to("supa")
+    x = torch.empty(n, 65, 4, device="supa")
+    x.copy_(small)
+    t = torch.empty(n, *st.shape, dtype=st.dtype, device="supa")
+    t.copy_(st)
+    got = F.cross_entropy(x.view(-1, 4), t.flatten(0, 1), reduction="none")
+    assert bool((got.view(n, 65) == F.cross_entropy(small, st, reduction="none")).all())
+    del x, t, got
+    torch.supa.empty_cache()
+
+
 def test_fused_cross_entropy_mean_precision(no_fallback):
     """The mean over rows of one sign against 64 bits.  In a tree of n sums the
     last additions round at the size of the whole: 1 + 1/2 + 1/4 + ... and the

@@ -77,3 +77,19 @@ def test_other_layouts_and_types(no_fallback):
         w[2, 3, 4, 5] = special
         got, want = w.to("supa").sum(0).cpu(), w.sum(0)
         assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+
+
+@pytest.mark.parametrize("shape, dim", [((1 << 22, 64 + 1, 2), 2), ((1 << 23, 64, 17, 2), 2)])
+def test_more_results_than_one_launch(shape, dim, no_fallback):
+    """More threads than a launch holds: 2^28 rows, and 2^30 columns in planes of two."""
+    if torch.supa.mem_get_info()[0] < 80 << 30:
+        pytest.skip("takes 45 GiB of device memory")
+    small = seeded(shape[1:], 7, torch.bfloat16).to("supa")
+    x = torch.empty(shape, dtype=torch.bfloat16, device="supa")
+    x.copy_(small)
+    want = small.sum(dim - 1)
+    got = x.view(-1, *shape[2:]).sum(dim - 1).view(shape[0], *want.shape)
+    del x
+    assert bool((got == want).all())
+    del got
+    torch.supa.empty_cache()

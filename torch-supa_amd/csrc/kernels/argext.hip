@@ -136,12 +136,12 @@ constexpr int kExtUnroll = 4;
 
 template <bool MIN, typename T, int G>
 __global__ void __launch_bounds__(kExtBlock)
-k_argext_rows(const T* __restrict__ in, int64_t inner, int64_t chunk, FastDiv nchunks, uint32_t nseg,
+k_argext_rows(const T* __restrict__ in, int64_t inner, int64_t chunk, FastDiv nchunks, uint32_t first, uint32_t nseg,
               T* __restrict__ out_val, int64_t* __restrict__ out_idx) {
   using A = typename ExtReg<T>::type;
   constexpr int V = 16 / sizeof(T);
   const int lane = threadIdx.x % G;
-  uint32_t seg = blockIdx.x * (kExtBlock / G) + threadIdx.x / G;
+  uint32_t seg = first + blockIdx.x * (kExtBlock / G) + threadIdx.x / G;
   const bool valid = seg < nseg;
   if (!valid) seg = nseg - 1;  // the block's shuffles need every lane
   uint32_t row, c;
@@ -296,13 +296,21 @@ int launch_ext_rows(const T* in, int64_t outer, int64_t inner, int64_t chunk, in
   const uint32_t nseg = (uint32_t)(outer * nchunks);
   const int64_t vecs = std::min(chunk, inner) * (int64_t)sizeof(T) / 16;
   const FastDiv div((uint32_t)nchunks);
-  auto grid = [&](int g) { return (unsigned)(((int64_t)nseg * g + kExtBlock - 1) / kExtBlock); };
-  if (vecs <= (nseg >= (1u << 15) ? 128 : 64))
-    k_argext_rows<MIN, T, 16><<<grid(16), kExtBlock, 0, st>>>(in, inner, chunk, div, nseg, out_val, out_idx);
-  else if (vecs <= (nseg >= (1u << 13) ? 512 : 256))
-    k_argext_rows<MIN, T, 64><<<grid(64), kExtBlock, 0, st>>>(in, inner, chunk, div, nseg, out_val, out_idx);
-  else k_argext_rows<MIN, T, 256><<<grid(256), kExtBlock, 0, st>>>(in, inner, chunk, div, nseg, out_val, out_idx);
-  return launch_status();
+  auto go = [&](auto g) -> int {
+    constexpr int64_t per = kExtBlock / g.value;
+    constexpr int64_t slab = per * (((int64_t(1) << 32) - 1) / kExtBlock);  // HIP: fewer than 2^32 threads a launch
+    for (int64_t s0 = 0; s0 < nseg; s0 += slab) {
+      const int64_t n = std::min<int64_t>(slab, nseg - s0);
+      k_argext_rows<MIN, T, g.value><<<(unsigned)((n + per - 1) / per), kExtBlock, 0, st>>>(
+          in, inner, chunk, div, (uint32_t)s0, nseg, out_val, out_idx);
+      const int rc = launch_status();
+      if (rc) return rc;
+    }
+    return SUPA_AMD_OK;
+  };
+  if (vecs <= (nseg >= (1u << 15) ? 128 : 64)) return go(std::integral_constant<int, 16>{});
+  if (vecs <= (nseg >= (1u << 13) ? 512 : 256)) return go(std::integral_constant<int, 64>{});
+  return go(std::integral_constant<int, 256>{});
 }
 
 // TY: 4 or 16 threads along the reduced dim while the position vectors alone

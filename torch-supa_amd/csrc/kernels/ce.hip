@@ -66,6 +66,8 @@ __device__ __forceinline__ bool ce_kept(int64_t t, int64_t c, int64_t ignore_ind
 // a workgroup per row, 46 with a wavefront; from 257 vectors on a wavefront
 // would hold a second batch of loads while the next row's wait).
 constexpr int kCeWaveVecs = 64 * kCeUnroll;
+// Workgroups of a launch: HIP takes fewer than 2^32 threads.
+constexpr int64_t kCeSlab = ((int64_t(1) << 32) - 1) / kCeBlock;
 
 template <typename T, int G>
 __global__ void __launch_bounds__(kCeBlock)
@@ -509,14 +511,21 @@ int supa_amd_cross_entropy_forward(const void* logits, int32_t dtype, const int6
     if (n > 0) {
       const T* x = static_cast<const T*>(logits);
       T* on = reduction == SUPA_AMD_REDUCTION_NONE ? o : nullptr;
-      if ((c + CeVec<T>::V - 1) / CeVec<T>::V <= kCeWaveVecs)
-        k_ce_fwd<T, 64><<<(unsigned)((n + 3) / 4), kCeBlock, 0, st>>>(x, target, n, c, ignore_index, rows, lse, on,
-                                                                      error_flag);
-      else
-        k_ce_fwd<T, kCeBlock><<<(unsigned)n, kCeBlock, 0, st>>>(x, target, n, c, ignore_index, rows, lse, on,
-                                                                error_flag);
-      const int rc = launch_status();
-      if (rc) return rc;
+      const bool wave = (c + CeVec<T>::V - 1) / CeVec<T>::V <= kCeWaveVecs;
+      const int64_t per = wave ? kCeBlock / 64 : 1, slab = per * kCeSlab;
+      for (int64_t r0 = 0; r0 < n; r0 += slab) {
+        const int64_t nr = std::min(slab, n - r0);
+        const unsigned blocks = (unsigned)((nr + per - 1) / per);
+        T* const o0 = on ? on + r0 : nullptr;
+        if (wave)
+          k_ce_fwd<T, 64><<<blocks, kCeBlock, 0, st>>>(x + r0 * c, target + r0, nr, c, ignore_index, rows + r0, lse + r0,
+                                                       o0, error_flag);
+        else
+          k_ce_fwd<T, kCeBlock><<<blocks, kCeBlock, 0, st>>>(x + r0 * c, target + r0, nr, c, ignore_index, rows + r0,
+                                                             lse + r0, o0, error_flag);
+        const int rc = launch_status();
+        if (rc) return rc;
+      }
     }
     if (reduction == SUPA_AMD_REDUCTION_NONE) return SUPA_AMD_OK;
     return ce_final<T>(rows, target, n, c, ignore_index, reduction, o, count, st);
@@ -573,9 +582,12 @@ int supa_amd_cross_entropy_prob_forward(const void* logits, const void* target, 
       const T* x = static_cast<const T*>(logits);
       const T* t = static_cast<const T*>(target);
       T* on = reduction == SUPA_AMD_REDUCTION_NONE ? o : nullptr;
-      k_ce_prob_fwd<T><<<(unsigned)n, kCeBlock, 0, st>>>(x, t, c, rows, lse, tsum, on);
-      const int rc = launch_status();
-      if (rc) return rc;
+      for (int64_t r0 = 0; r0 < n; r0 += kCeSlab) {
+        k_ce_prob_fwd<T><<<(unsigned)std::min(kCeSlab, n - r0), kCeBlock, 0, st>>>(
+            x + r0 * c, t + r0 * c, c, rows + r0, lse + r0, tsum + r0, on ? on + r0 : nullptr);
+        const int rc = launch_status();
+        if (rc) return rc;
+      }
     }
     if (reduction == SUPA_AMD_REDUCTION_NONE) return SUPA_AMD_OK;
     return ce_final<T>(rows, nullptr, n, c, 0, reduction, o, nullptr, st);

@@ -197,11 +197,17 @@ int moments_launch(const T* in, T* out_var, T* out_mean, int64_t rows, int64_t s
                                                          out_mean);
     return launch_status();
   }
-  auto go = [&](auto G, auto NV) {
-    const unsigned blocks = (unsigned)((rows + 256 / G.value - 1) / (256 / G.value));
-    k_moments<T, A, VW, G.value, NV.value, true>
-        <<<blocks, kMomBlock, 0, st>>>(in, g, FastDiv(), (A)correction, take_sqrt, out_var, out_mean, nullptr);
-    return launch_status();
+  auto slabs = [&](int64_t per, auto&& launch) -> int {  // `per` rows a workgroup
+    const int64_t slab = per * (((int64_t(1) << 32) - 1) / kMomBlock);  // HIP: fewer than 2^32 threads a launch
+    for (int64_t r0 = 0; r0 < rows; r0 += slab) {
+      SegGeom gs = g;
+      gs.rows = std::min(slab, rows - r0);
+      launch((unsigned)((gs.rows + per - 1) / per), in + r0 * row_stride, gs, out_var + r0,
+             out_mean ? out_mean + r0 : nullptr);
+      const int rc = launch_status();
+      if (rc) return rc;
+    }
+    return SUPA_AMD_OK;
   };
   using std::integral_constant;
   using G16 = integral_constant<int, 16>;
@@ -211,6 +217,12 @@ int moments_launch(const T* in, T* out_var, T* out_mean, int64_t rows, int64_t s
   using N2 = integral_constant<int, 2>;
   using N4 = integral_constant<int, 4>;
   using N8 = integral_constant<int, 8>;
+  auto go = [&](auto G, auto NV) -> int {
+    return slabs(256 / G.value, [&](unsigned blocks, const T* x, const SegGeom& gs, T* v, T* m) {
+      k_moments<T, A, VW, G.value, NV.value, true>
+          <<<blocks, kMomBlock, 0, st>>>(x, gs, FastDiv(), (A)correction, take_sqrt, v, m, nullptr);
+    });
+  };
   // the fewest threads a row, and of those the fewest vectors a thread
   if (nvec <= 16) return go(G16{}, N1{});
   if (nvec <= 64) return go(G64{}, N1{});

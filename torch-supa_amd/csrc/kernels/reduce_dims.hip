@@ -35,6 +35,7 @@ constexpr int64_t kDimSumBlocks = 1024;  // workgroups to aim at when cutting ch
 // the columns no other vector covers.
 struct ColsGeom {
   uint32_t npos;    // position vectors: outer * ceil(inner / VW)
+  uint32_t first;   // the launch's first one
   FastDiv ivec;     // vectors per row
   int64_t red, inner;
   int64_t chunk;    // rows per chunk (blockIdx.y)
@@ -47,7 +48,7 @@ k_sum_cols(const T* __restrict__ in, OT* __restrict__ out, ColsGeom g, ACC scale
   constexpr int TX = 1 << TXL, TY = kDimSumBlock / TX, NW = kDimSumBlock / 64, U = 8;
   __shared__ ACC lds[TX <= 64 ? NW * TX * VW : 1];
   const uint32_t tx = threadIdx.x & (TX - 1), ty = threadIdx.x >> TXL;
-  const uint32_t p = blockIdx.x * TX + tx;
+  const uint32_t p = g.first + blockIdx.x * TX + tx;
   const bool valid = p < g.npos;
   uint32_t o, v;
   g.ivec.divmod(p, o, v);
@@ -121,13 +122,23 @@ inline int64_t cols_chunk(int64_t red, int64_t npos, int txl) {
   return (per + rows - 1) / rows * rows;
 }
 
+constexpr int64_t kDimSumSlab = ((int64_t(1) << 32) - 1) / kDimSumBlock;  // workgroups: HIP takes fewer than 2^32 threads
+
 template <typename T, typename OT, typename ACC, int VW>
-int cols_launch(const T* in, OT* out, const ColsGeom& g, int txl, ACC scale, hipStream_t st) {
-  const dim3 grid((unsigned)(((uint64_t)g.npos + (1u << txl) - 1) >> txl), (unsigned)((g.red + g.chunk - 1) / g.chunk));
-  if (txl == 8) k_sum_cols<T, OT, ACC, VW, 8><<<grid, kDimSumBlock, 0, st>>>(in, out, g, scale);
-  else if (txl == 6) k_sum_cols<T, OT, ACC, VW, 6><<<grid, kDimSumBlock, 0, st>>>(in, out, g, scale);
-  else k_sum_cols<T, OT, ACC, VW, 4><<<grid, kDimSumBlock, 0, st>>>(in, out, g, scale);
-  return launch_status();
+int cols_launch(const T* in, OT* out, ColsGeom g, int txl, ACC scale, hipStream_t st) {
+  const unsigned chunks = (unsigned)((g.red + g.chunk - 1) / g.chunk);
+  const int64_t slab = kDimSumSlab << txl;
+  for (int64_t p0 = 0; p0 < g.npos; p0 += slab) {
+    g.first = (uint32_t)p0;
+    const int64_t n = std::min<int64_t>(slab, g.npos - p0);
+    const dim3 grid((unsigned)((n + (1 << txl) - 1) >> txl), chunks);
+    if (txl == 8) k_sum_cols<T, OT, ACC, VW, 8><<<grid, kDimSumBlock, 0, st>>>(in, out, g, scale);
+    else if (txl == 6) k_sum_cols<T, OT, ACC, VW, 6><<<grid, kDimSumBlock, 0, st>>>(in, out, g, scale);
+    else k_sum_cols<T, OT, ACC, VW, 4><<<grid, kDimSumBlock, 0, st>>>(in, out, g, scale);
+    const int rc = launch_status();
+    if (rc) return rc;
+  }
+  return SUPA_AMD_OK;
 }
 
 // Geometry of a [outer, red, inner] sum in VW-wide vectors; false when its
@@ -135,7 +146,7 @@ int cols_launch(const T* in, OT* out, const ColsGeom& g, int txl, ACC scale, hip
 inline bool cols_geom(ColsGeom& g, int64_t outer, int64_t red, int64_t inner, int vw, int64_t chunk) {
   const int64_t ivec = (inner + vw - 1) / vw;
   if (ivec >= (int64_t(1) << 31) || outer * ivec >= (int64_t(1) << 31) || (red + chunk - 1) / chunk > 65535) return false;
-  g = ColsGeom{(uint32_t)(outer * ivec), FastDiv((uint32_t)ivec), red, inner, chunk, outer * inner};
+  g = ColsGeom{(uint32_t)(outer * ivec), 0, FastDiv((uint32_t)ivec), red, inner, chunk, outer * inner};
   return true;
 }
 
@@ -228,17 +239,25 @@ inline int64_t seg_chunks(int64_t rows, int64_t nvec) {
 
 template <typename T, typename OT, typename ACC, int VW>
 int segs_launch(const T* in, OT* out, const SegGeom& g, unsigned nch, ACC scale, hipStream_t st) {
+  auto go = [&](auto G) -> int {
+    constexpr int64_t per = kDimSumBlock / G.value, slab = per * kDimSumSlab;
+    for (int64_t r0 = 0; r0 < g.rows; r0 += slab) {
+      SegGeom gs = g;
+      gs.rows = std::min(slab, g.rows - r0);
+      const dim3 grid((unsigned)((gs.rows + per - 1) / per), nch);
+      k_sum_segs<T, OT, ACC, VW, G.value><<<grid, kDimSumBlock, 0, st>>>(in + r0 * g.row_stride, out + r0 * nch, gs, scale);
+      const int rc = launch_status();
+      if (rc) return rc;
+    }
+    return SUPA_AMD_OK;
+  };
+  using std::integral_constant;
   // a wavefront per row up to 512 vectors where the rows alone fill the chip
   // (bf16 [6007, 2047] 6.3 us, 11.5 with four)
   const bool wave = g.rows >= 1024 && g.nvec <= 512;
-  if (nch == 1 && g.nvec <= 32) {
-    k_sum_segs<T, OT, ACC, VW, 16><<<(unsigned)((g.rows + 15) / 16), kDimSumBlock, 0, st>>>(in, out, g, scale);
-  } else if (nch == 1 && wave) {
-    k_sum_segs<T, OT, ACC, VW, 64><<<(unsigned)((g.rows + 3) / 4), kDimSumBlock, 0, st>>>(in, out, g, scale);
-  } else {
-    k_sum_segs<T, OT, ACC, VW, 256><<<dim3((unsigned)g.rows, nch), kDimSumBlock, 0, st>>>(in, out, g, scale);
-  }
-  return launch_status();
+  if (nch == 1 && g.nvec <= 32) return go(integral_constant<int, 16>{});
+  if (nch == 1 && wave) return go(integral_constant<int, 64>{});
+  return go(integral_constant<int, 256>{});
 }
 
 inline int64_t segs_vecs(int64_t segs, int64_t len, int vw) { return segs * ((len + vw - 1) / vw); }
