@@ -17,9 +17,13 @@ def seeded(shape, seed, dtype=torch.float32):
 def check(x, dx, dims, keepdim=False):
     want = x.double().sum(dims, keepdim)
     n = x.numel() // max(want.numel(), 1)
-    # float32 sums in chains of at most n / 64 + 128 additions, then one rounding
+    # float32 sums, each element in at most n / 256 + 40 of the additions one
+    # after another: columns add trees of 8, eight of those, a thread's eights
+    # (n / 256 with four row groups), then the groups; rows eight of a vector,
+    # a thread's vectors (n / 1024), then the threads; a chunk's rows and the
+    # chunks likewise.  Then one rounding
     u = 2.0 ** -53 if x.dtype == torch.float64 else 2.0 ** -24
-    tol = x.double().abs().sum(dims, keepdim) * (n / 64 + 128) * u
+    tol = x.double().abs().sum(dims, keepdim) * (n / 256 + 40) * u
     got = dx.sum(dims, keepdim)
     assert got.shape == want.shape and got.dtype == x.dtype
     err = (got.cpu().double() - want).abs()
@@ -49,6 +53,22 @@ def test_three_dims(shape, dtype, no_fallback):
     p = dx.permute(2, 0, 1)  # dense in another order: kept dims in and out of their own order
     for dims in (0, 1, 2, (0, 2), (1, 2)):
         check(x.permute(2, 0, 1), p, dims)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [300, 4096, 9000])
+def test_precision_of_many_columns(rows, dtype, no_fallback):
+    """Columns that fill the chip alone, so that a thread adds a quarter of the
+    rows: against 64 bits.  The squared rounding errors of a sum of n equal
+    variances add up to about (n / 512 + 16) / 3 of 2^-48 with chains of n / 256
+    (one chain of n / 4 additions: n / 8 / 3)."""
+    x = seeded((rows, 128), 6, dtype)
+    want = x.double().sum(0)
+    wide = x.to("supa").unsqueeze(1).expand(rows, 1040, 128).reshape(rows, -1)
+    got = wide.sum(0, dtype=torch.float32).view(-1, 128)
+    assert bool((got == got[0]).all())
+    err = (got[0].cpu().double() - want).norm() / want.norm()
+    assert err <= ((rows / 512 + 16) / 3) ** 0.5 * 2.0 ** -24, float(err)
 
 
 def test_other_layouts_and_types(no_fallback):

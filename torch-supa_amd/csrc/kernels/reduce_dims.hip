@@ -70,10 +70,24 @@ k_sum_cols(const T* __restrict__ in, OT* __restrict__ out, ColsGeom g, ACC scale
       sum_raw_t<T, VW> w[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) w[u] = sum_load<T, VW>(src + (r + u * TY) * g.inner);
+      if constexpr (std::is_integral<ACC>::value) {
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int k = 0; k < VW; ++k) acc[k] += sum_elem<T, VW, ACC>(w[u], k);
+          for (int k = 0; k < VW; ++k) acc[k] += sum_elem<T, VW, ACC>(w[u], k);
+      } else {  // U rows by a tree, then the steps (cols_chunk says how many)
+#pragma unroll
+        for (int k = 0; k < VW; ++k) {
+          ACC t[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) t[u] = sum_elem<T, VW, ACC>(w[u], k);
+#pragma unroll
+          for (int h = 1; h < U; h *= 2)
+#pragma unroll
+            for (int u = 0; u < U; u += 2 * h) t[u] += t[u + h];
+          acc[k] += t[0];
+        }
+      }
     }
     for (; r < hi; r += TY) {
       const sum_raw_t<T, VW> w = sum_load<T, VW>(src + r * g.inner);
@@ -112,11 +126,18 @@ k_sum_cols(const T* __restrict__ in, OT* __restrict__ out, ColsGeom g, ACC scale
 inline int cols_txl(int64_t red, int64_t npos) { return red <= 16 ? 8 : (npos >= 32 ? 6 : 4); }
 
 // Rows per chunk: enough chunks for kDimSumBlocks workgroups, each of at least
-// 8 rows a thread; one chunk when the columns alone give that many.
+// 8 rows a thread, and no more than 64 rows a thread (or a 256th of the column,
+// as a workgroup per column would give each of its threads): where the columns
+// alone fill the chip a thread of a single chunk would add red / TY rows one
+// after another, and its rounding errors with them (float32 against 64 bits,
+// [8192, 128256]: 4.4e-7 in one chunk, 1.2e-7 so and with a workgroup per
+// column).  The partials are a 64th of the rows at most.
 inline int64_t cols_chunk(int64_t red, int64_t npos, int txl) {
   const int64_t blocks = (npos + (1 << txl) - 1) >> txl;
-  const int64_t rows = 8 * (kDimSumBlock >> txl);  // one unrolled step
-  const int64_t want = std::min<int64_t>((kDimSumBlocks + blocks - 1) / blocks, (red + rows - 1) / rows);
+  const int64_t ty = kDimSumBlock >> txl, rows = 8 * ty;  // one unrolled step
+  const int64_t fill = std::min<int64_t>((kDimSumBlocks + blocks - 1) / blocks, (red + rows - 1) / rows);
+  const int64_t most = ty * std::max<int64_t>(64, red / kDimSumBlock);
+  const int64_t want = std::max<int64_t>(fill, (red + most - 1) / most);
   if (want <= 1) return red;
   const int64_t per = (red + want - 1) / want;
   return (per + rows - 1) / rows * rows;
