@@ -96,6 +96,23 @@ def test_spatial_softmax_layouts_and_special_values(no_fallback):
                                rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("shape", [(1, 4096, 128, 128), (1, 1000, 64, 128)])
+def test_spatial_gradient_precision(shape, no_fallback):
+    """The sums over many streamed classes against 64 bits.  A sum of n equal
+    variances whose thread chains are n / 128 steps of 8 additions, then 16
+    groups, carries about (n / 256 + 16) / 3 squared roundings of 2^-24; one
+    chain of n / 16 additions, as before, n / 32 / 3 of them."""
+    n, reps = shape[1], shape[3]
+    g, y = (seeded(shape[:3], 9 + i) for i in range(2))
+    p = y.double()
+    want = p * (g.double() - (g.double() * p).sum(1, keepdim=True))
+    dg, dy = (t.repeat(1, 1, reps).to("supa") for t in (g, y))
+    got = SM_BWD(dg, dy, 1, torch.float32)
+    err = (got[:, :, :shape[2]].cpu().double() - want).norm() / want.norm()
+    assert err <= ((n / 256 + 16) / 3) ** 0.5 * 2.0 ** -24, float(err)
+    assert torch.equal(got[:, :, -shape[2]:].cpu(), got[:, :, :shape[2]].cpu())
+
+
 @pytest.mark.parametrize("log", [True, False])
 def test_more_positions_than_one_launch(log, no_fallback):
     """2^28 positions of 33 classes: more threads than a launch holds."""

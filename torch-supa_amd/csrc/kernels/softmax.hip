@@ -170,12 +170,15 @@ k_row_fwd(const TI* __restrict__ in, TO* __restrict__ out, int64_t rows, int col
     }
   const float mb = m == -__builtin_inff() ? 0.0f : m;  // all -inf: keep exp arguments finite
   if constexpr (VW > 1) opaque<NV>(x);
+  // a vector's sum, then the sum of the thread's vectors: chains of NV and VW
   float s = VW > 1 ? __builtin_amdgcn_exp2f((xt - mb) * kLog2e) : 0.0f;
 #pragma unroll
   for (int j = 0; j < NV; ++j)
     if (l + j * G < nvec) {
+      float t = NV == 1 ? s : 0.0f;
 #pragma unroll
-      for (int k = 0; k < VW; ++k) s += __builtin_amdgcn_exp2f((row_elem<TI, VW>(x[j], k) - mb) * kLog2e);
+      for (int k = 0; k < VW; ++k) t += __builtin_amdgcn_exp2f((row_elem<TI, VW>(x[j], k) - mb) * kLog2e);
+      s = NV == 1 ? t : s + t;
     }
   row_lse<G>(m, s);
   // log: (x - M) - log S;  softmax: e^(x - M) / S (an all -inf row gives
@@ -221,11 +224,13 @@ k_row_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restri
 #pragma unroll
   for (int j = 0; j < NV; ++j)
     if (l + j * G < nvec) {
+      float t = 0.0f;  // a vector's sum first, as in the forward
 #pragma unroll
       for (int k = 0; k < VW; ++k) {
-        if constexpr (LOG) s += row_elem<TG, VW>(g[j], k);
-        else s = fmaf(row_elem<TG, VW>(g[j], k), row_elem<TG, VW>(y[j], k), s);
+        if constexpr (LOG) t += row_elem<TG, VW>(g[j], k);
+        else t = fmaf(row_elem<TG, VW>(g[j], k), row_elem<TG, VW>(y[j], k), t);
       }
+      s = NV == 1 ? t : s + t;
     }
   s = row_sum<G>(LOG ? s + gt : fmaf(gt, yt, s));
   auto res = [&](float gk, float yk) {
@@ -912,9 +917,24 @@ k_lsm_fwd_split(const TI* __restrict__ in, TO* __restrict__ out, int64_t cols, i
   // each part's sum rescaled to it (K exponentials)
   float M = __uint_as_float((uint32_t)part_w[0]);
   for (int q = 1; q < K; ++q) M = fmaxf(M, __uint_as_float((uint32_t)part_w[q]));
+  auto part_sum_at = [&](int q) {
+    return lse_rescale(__uint_as_float((uint32_t)(part_w[q] >> 32)), __uint_as_float((uint32_t)part_w[q]), M);
+  };
   float S = 0.0f;
-  for (int q = 0; q < K; ++q)
-    S += lse_rescale(__uint_as_float((uint32_t)(part_w[q] >> 32)), __uint_as_float((uint32_t)part_w[q]), M);
+  if (K <= 8) {
+    for (int q = 0; q < K; ++q) S += part_sum_at(q);
+  } else {  // four sums side by side: fewer roundings at the size of the whole
+    float S1 = 0.0f, S2 = 0.0f, S3 = 0.0f;
+    int q = 0;
+    for (; q + 3 < K; q += 4) {
+      S += part_sum_at(q);
+      S1 += part_sum_at(q + 1);
+      S2 += part_sum_at(q + 2);
+      S3 += part_sum_at(q + 3);
+    }
+    for (; q < K; ++q) S += part_sum_at(q);
+    S = (S + S1) + (S2 + S3);
+  }
   const float logsum = LOG ? sa_logf(S) : 0.0f;
   const float inv = LOG ? 0.0f : 1.0f / S;
   const float Mb = M == -__builtin_inff() ? 0.0f : M;

@@ -213,12 +213,17 @@ k_dim_fwd(const TI* __restrict__ in, TO* __restrict__ out, DimGeom g) {
       mb[k] = M[k] == -__builtin_inff() ? 0.0f : M[k];
     }
     dim_opaque<TI, VW, NC>(x);
+    float t[VW];  // this step's NC classes, then the steps: no chain is as long as the class dim
+#pragma unroll
+    for (int k = 0; k < VW; ++k) t[k] = HOLD ? s[k] : 0.0f;
 #pragma unroll
     for (int j = 0; j < NC; ++j)
       if (at.valid && c0 + j * TY < g.cols) {
 #pragma unroll
-        for (int k = 0; k < VW; ++k) s[k] += __builtin_amdgcn_exp2f((dim_elem<TI, VW>(x[j], k) - mb[k]) * kLog2e);
+        for (int k = 0; k < VW; ++k) t[k] += __builtin_amdgcn_exp2f((dim_elem<TI, VW>(x[j], k) - mb[k]) * kLog2e);
       }
+#pragma unroll
+    for (int k = 0; k < VW; ++k) s[k] = HOLD ? t[k] : s[k] + t[k];
     if constexpr (HOLD) break;
   }
   dim_lse<VW, TXL>(m, s, lds);
@@ -281,15 +286,20 @@ k_dim_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restri
         if (HOLD || !LOG) yv[j] = dim_load<TG, VW, HOLD>(ys + (int64_t)c * g.inner);
       }
     }
+    float t[VW];  // as in the forward
+#pragma unroll
+    for (int k = 0; k < VW; ++k) t[k] = HOLD ? s[k] : 0.0f;
 #pragma unroll
     for (int j = 0; j < NC; ++j)
       if (at.valid && c0 + j * TY < g.cols) {
 #pragma unroll
         for (int k = 0; k < VW; ++k) {
-          if constexpr (LOG) s[k] += dim_elem<TG, VW>(gv[j], k);
-          else s[k] = fmaf(dim_elem<TG, VW>(gv[j], k), dim_elem<TG, VW>(yv[j], k), s[k]);
+          if constexpr (LOG) t[k] += dim_elem<TG, VW>(gv[j], k);
+          else t[k] = fmaf(dim_elem<TG, VW>(gv[j], k), dim_elem<TG, VW>(yv[j], k), t[k]);
         }
       }
+#pragma unroll
+    for (int k = 0; k < VW; ++k) s[k] = HOLD ? t[k] : s[k] + t[k];
     if constexpr (HOLD) break;
   }
   dim_sum<VW, TXL>(s, lds);
