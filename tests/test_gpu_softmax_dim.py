@@ -1,8 +1,18 @@
-# a 16-bit gradient is one rounding too, of a difference whose terms' sum moves
-# by `atol`: one unit in the last place, relative, on top of that
-ULP = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
-# the smallest gradients: float32's own floor, half a unit of a float16 subnormal
-FLOOR = {torch.float32: 1e-6, torch.bfloat16: 0.0, torch.float16: 2.0 ** -24}
+"""log_softmax and softmax over a dim that is not the last one (the spatial
+kernels): class counts around the edges of each split of the classes over
+class groups, planes of every remainder of the vector, special values, and
+the output written over the input."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import bf16_ulp_dist
+
+pytestmark = pytest.mark.gpu
+
+LSM_BWD = torch.ops.aten._log_softmax_backward_data
+SM_BWD = torch.ops.aten._softmax_backward_data
 
 
 def seeded(shape, seed, scale=1.0, dtype=torch.float32):

@@ -1,5 +1,19 @@
-# vectors a row: the last of each thread split, and one more
-VECS = [1, 2, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 2560, 2561, 5121]
+"""Row softmax, log_softmax and their gradients at the edges of the row
+kernels: the longest row of each thread split and one element more, rows of
+every remainder of the vector, rows whose base is not 16-byte aligned, the
+output over the input, special values in every position of a short row."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import bf16_ulp_dist
+
+pytestmark = pytest.mark.gpu
+
+LSM_BWD = torch.ops.aten._log_softmax_backward_data
+SM_BWD = torch.ops.aten._softmax_backward_data
+ULP = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
 
 
 def seeded(shape, seed, scale=1.0, dtype=torch.float32):
@@ -15,8 +29,8 @@ def shifted(t):
     return v
 
 
-# vectors a row: the last of each thread split, and one more
-VECS = [1, 2, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 2560, 2561, 5121]
+# the smallest gradients: float32's own floor, half a unit of a float16 subnormal
+FLOOR = {torch.float32: 1e-6, torch.bfloat16: 0.0, torch.float16: 2.0 ** -24}
 
 
 def check_forward(got, ref, dtype, atol):
