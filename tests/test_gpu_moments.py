@@ -133,6 +133,28 @@ def test_moments_at_the_edges_of_a_chunk(dtype, vecs, no_fallback):
             torch.testing.assert_close(mean.cpu().double(), t.double().mean(dim=dims), rtol=RTOL[dtype], atol=0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("n", [1, 2, 7, 100, 3000, 9001, 140001])
+def test_infinities_and_nan(dtype, n, no_fallback):
+    """The mean of a row with an infinity is that infinity (NaN with both, or a
+    NaN), its variance NaN, wherever it stands, also in rows cut in chunks."""
+    inf, rows = float("inf"), []
+    base = (torch.randn(n, generator=torch.Generator().manual_seed(n)) + 2).to(dtype)
+    for at in sorted({0, n // 2, n - 1}):
+        for v in (inf, -inf, float("nan")):
+            r = base.clone()
+            r[at] = v
+            rows.append(r)
+    both = base.clone()
+    both[0], both[-1] = inf, -inf
+    x = torch.stack(rows + [both, torch.full_like(base, inf), base])
+    for t, dims in ((x, 1), (x.view(1, -1, n), (0, 2))):
+        var, mean = torch.var_mean(t.to("supa"), dim=dims, correction=0)
+        assert torch.isnan(var[:-1].cpu()).all() and not torch.isnan(var[-1].cpu())
+        want = x.double().mean(1)
+        torch.testing.assert_close(mean.cpu().double(), want, rtol=RTOL[dtype], atol=0, equal_nan=True)
+
+
 def test_more_rows_than_one_launch(no_fallback):
     """2^24 rows of a workgroup each: more threads than a launch holds."""
     if torch.supa.mem_get_info()[0] < 120 << 30:

@@ -39,13 +39,21 @@ template <typename A> struct Welford {
   A n, mean, m2;
 };
 
+template <typename A> __device__ __forceinline__ bool mom_finite(A x) { return x - x == A(0); }
+
+// Means of +inf or -inf meet as they would in a sum (inf + finite is inf).
 template <typename A> __device__ __forceinline__ Welford<A> wf_merge(Welford<A> a, Welford<A> b) {
   if (a.n == A(0)) return b;
   if (b.n == A(0)) return a;
   const A n = a.n + b.n;
   const A d = b.mean - a.mean;
   const A nb_n = b.n / n;
-  return {n, a.mean + d * nb_n, a.m2 + b.m2 + d * d * a.n * nb_n};
+  return {n, mom_finite(d) ? a.mean + d * nb_n : a.mean + b.mean, a.m2 + b.m2 + d * d * a.n * nb_n};
+}
+// The value that chunk means are taken relative to: the row's first element.
+template <typename A, typename T> __device__ __forceinline__ A mom_shift(T first) {
+  const A k = (A)to_arith(first);
+  return mom_finite(k) ? k : A(0);
 }
 
 template <typename A> __device__ __forceinline__ Welford<A> wf_shfl(Welford<A> w, int off) {
@@ -143,15 +151,16 @@ k_moments(const T* __restrict__ in, SegGeom g, FastDiv nch, A correction, int ta
   }
   mom_sum<G, A>(sd, m2, lds);
   if (l == 0) {
-    const A corr = sd / count;
-    const A q = m2 - sd * corr;
+    const A c1 = sd / count;
+    const A q = m2 - sd * c1;
+    const A corr = mom_finite(mean) ? c1 : A(0);  // an infinite mean stands: its deviations are NaN
     Welford<A> w{count, mean + corr, q < A(0) ? A(0) : q};
     if constexpr (FINAL) {
       mom_write<A, T>(w, correction, take_sqrt, out_var + row, out_mean ? out_mean + row : nullptr);
     } else {
       A* p = part + 3 * (int64_t)blockIdx.x;
       p[0] = w.n;
-      p[1] = (mean - (A)to_arith(src[0])) + corr;
+      p[1] = (mean - mom_shift<A>(src[0])) + corr;
       p[2] = w.m2;
     }
   }
@@ -168,7 +177,7 @@ k_moments_final(const T* __restrict__ in, int64_t row_stride, const A* __restric
   for (int64_t i = threadIdx.x; i < nch; i += 64) w = wf_merge(w, Welford<A>{src[3 * i], src[3 * i + 1], src[3 * i + 2]});
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) w = wf_merge(w, wf_shfl(w, off));
-  w.mean += (A)to_arith(in[row * row_stride]);
+  w.mean += mom_shift<A>(in[row * row_stride]);
   if (threadIdx.x == 0)
     mom_write<A, T>(w, correction, take_sqrt, out_var + row,
                     out_mean ? out_mean + row : nullptr);
