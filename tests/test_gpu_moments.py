@@ -155,6 +155,18 @@ def test_infinities_and_nan(dtype, n, no_fallback):
         torch.testing.assert_close(mean.cpu().double(), want, rtol=RTOL[dtype], atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("shape", [(1, 5000000), (3, 1200007), (1030, 4099), (5, 8192), (2050, 70003), (2, 3, 40001)])
+def test_float64_rows_and_long_merges(shape, no_fallback):
+    """float64 rows by a wavefront, by a workgroup, cut in chunks; more chunks than a wavefront merges."""
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(3), dtype=torch.float64) * 0.01 + 1000
+    for dt in (torch.float64, torch.float32):
+        t = x.to(dt)
+        dims = (0, 2) if t.dim() == 3 else 1
+        var, mean = torch.var_mean(t.to("supa"), dim=dims)
+        torch.testing.assert_close(var.cpu().double(), t.double().var(dim=dims), rtol=1e-5, atol=0)
+        torch.testing.assert_close(mean.cpu().double(), t.double().mean(dim=dims), rtol=1e-6, atol=0)
+
+
 def test_more_rows_than_one_launch(no_fallback):
     """2^24 rows of a workgroup each: more threads than a launch holds."""
     if torch.supa.mem_get_info()[0] < 120 << 30:

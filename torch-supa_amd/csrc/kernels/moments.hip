@@ -166,17 +166,38 @@ k_moments(const T* __restrict__ in, SegGeom g, FastDiv nch, A correction, int ta
   }
 }
 
-// One wavefront merges a row's chunk triples.
-template <typename T, typename A>
-__global__ void __launch_bounds__(64)
+// BS threads merge a row's chunk triples, each kMomMerge of them loaded ahead
+// of its merges: a wavefront for up to 128, else 1024 threads (the variance of
+// 64 Mi float32 elements, 8192 triples, 83.6 us with a wavefront of 128 merges
+// a lane one after another).
+constexpr int kMomMerge = 4;
+template <typename T, typename A, int BS>
+__global__ void __launch_bounds__(BS)
 k_moments_final(const T* __restrict__ in, int64_t row_stride, const A* __restrict__ part, int64_t nch, A correction,
                 int take_sqrt, T* __restrict__ out_var, T* __restrict__ out_mean) {
   const int64_t row = blockIdx.x;
   const A* src = part + 3 * row * nch;
   Welford<A> w{A(0), A(0), A(0)};
-  for (int64_t i = threadIdx.x; i < nch; i += 64) w = wf_merge(w, Welford<A>{src[3 * i], src[3 * i + 1], src[3 * i + 2]});
+  for (int64_t i0 = threadIdx.x; i0 < nch; i0 += kMomMerge * BS) {
+    Welford<A> t[kMomMerge];
+#pragma unroll
+    for (int u = 0; u < kMomMerge; ++u) {
+      const int64_t i = i0 + u * BS;
+      t[u] = i < nch ? Welford<A>{src[3 * i], src[3 * i + 1], src[3 * i + 2]} : Welford<A>{A(0), A(0), A(0)};
+    }
+#pragma unroll
+    for (int u = 0; u < kMomMerge; ++u) w = wf_merge(w, t[u]);
+  }
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) w = wf_merge(w, wf_shfl(w, off));
+  if constexpr (BS > 64) {
+    __shared__ Welford<A> lds[BS / 64];
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
+    __syncthreads();
+    w = lds[threadIdx.x & (BS / 64 - 1)];
+#pragma unroll
+    for (int off = 1; off < BS / 64; off <<= 1) w = wf_merge(w, wf_shfl(w, off));
+  }
   w.mean += mom_shift<A>(in[row * row_stride]);
   if (threadIdx.x == 0)
     mom_write<A, T>(w, correction, take_sqrt, out_var + row,
@@ -202,8 +223,12 @@ int moments_launch(const T* in, T* out_var, T* out_mean, int64_t rows, int64_t s
                                                       nullptr, part);
     const int rc = launch_status();
     if (rc) return rc;
-    k_moments_final<T, A><<<(unsigned)rows, 64, 0, st>>>(in, row_stride, part, nch, (A)correction, take_sqrt, out_var,
-                                                         out_mean);
+    if (nch <= 128)
+      k_moments_final<T, A, 64><<<(unsigned)rows, 64, 0, st>>>(in, row_stride, part, nch, (A)correction, take_sqrt,
+                                                               out_var, out_mean);
+    else
+      k_moments_final<T, A, 1024><<<(unsigned)rows, 1024, 0, st>>>(in, row_stride, part, nch, (A)correction, take_sqrt,
+                                                                   out_var, out_mean);
     return launch_status();
   }
   auto slabs = [&](int64_t per, auto&& launch) -> int {  // `per` rows a workgroup
