@@ -34,6 +34,10 @@ namespace sa {
 constexpr int kMomBlock = 256;
 constexpr int kMomVecs = 8;                                        // most vectors a thread holds
 constexpr uint32_t kMomChunk = (uint32_t)kMomBlock * kMomVecs;     // most vectors a chunk holds
+// float64 rows stream through (k_moments_stream) and are cut when few and long.
+constexpr int64_t kMomStreamRow = 16384;   // vectors of the longest uncut row
+constexpr int64_t kMomStreamRows = 2048;   // rows from which none is cut
+constexpr int64_t kMomStreamChunk = 8192;  // vectors a chunk
 
 template <typename A> struct Welford {
   A n, mean, m2;
@@ -166,6 +170,99 @@ k_moments(const T* __restrict__ in, SegGeom g, FastDiv nch, A correction, int ta
   }
 }
 
+// The same in one pass, as k_moments where a row's vectors are too many
+// registers: each thread merges the triples of kMomStreamU vectors at a time
+// into its own.  float64, whose vectors hold two elements and whose deviations
+// take twice the registers: [8192, 4100] 54 us, 79.5 in register chunks;
+// [2048, 10000] 29, 43; 32 Mi elements in one row 49, 102.
+constexpr int kMomStreamU = 4;
+template <typename T, typename A, int VW, int G, bool FINAL>
+__global__ void __launch_bounds__(kMomBlock)
+k_moments_stream(const T* __restrict__ in, SegGeom g, FastDiv nch, A correction, int take_sqrt,
+                 T* __restrict__ out_var, T* __restrict__ out_mean, A* __restrict__ part) {
+  constexpr int U = kMomStreamU;
+  const int l = threadIdx.x & (G - 1);
+  uint32_t wrow = blockIdx.x, c = 0;
+  if constexpr (!FINAL) nch.divmod(blockIdx.x, wrow, c);
+  const int64_t row = G < 256 ? (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G : (int64_t)wrow;
+  if (row >= g.rows) return;
+  const T* src = in + row * g.row_stride;
+  const int64_t lo = (int64_t)c * g.chunk;
+  const int64_t hi = g.nvec - lo < g.chunk ? g.nvec : lo + g.chunk;
+  const A K = mom_shift<A>(src[0]);
+  Welford<A> w{A(0), A(0), A(0)};
+  // U vectors' triple from their elements less K (zeros where not the row's)
+  auto merge = [&](const A (&x)[U * VW], const bool (&own)[U * VW], int n) {
+    A s = A(0);
+#pragma unroll
+    for (int k = 0; k < U * VW; ++k) s += x[k];
+    const A mean = s / (A)n;
+    A m2 = A(0);
+#pragma unroll
+    for (int k = 0; k < U * VW; ++k) {
+      const A d = own[k] ? x[k] - mean : A(0);
+      m2 = fma(d, d, m2);
+    }
+    w = wf_merge(w, Welford<A>{(A)n, mean, m2});
+  };
+  const int64_t whole = g.runs > 1 ? 0 : min(hi, g.len / VW);
+  int64_t i0 = lo + l;
+  for (; i0 + (U - 1) * G < whole; i0 += U * G) {
+    sum_raw_t<T, VW> q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) q[u] = sum_load<T, VW, false>(src + (i0 + u * G) * VW);
+    A x[U * VW];
+    bool own[U * VW];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < VW; ++k) {
+        x[u * VW + k] = sum_elem<T, VW, A>(q[u], k) - K;
+        own[u * VW + k] = true;
+      }
+    merge(x, own, U * VW);
+  }
+  for (; i0 < hi; i0 += U * G) {
+    A x[U * VW];
+    bool own[U * VW];
+    int n = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      sum_raw_t<T, VW> q;
+      uint32_t valid = 0;
+      if (i0 + u * G < hi) q = seg_load<T, VW, false>(src, g, i0 + u * G, valid);
+#pragma unroll
+      for (int k = 0; k < VW; ++k) {
+        own[u * VW + k] = valid >> k & 1u;
+        x[u * VW + k] = own[u * VW + k] ? sum_elem<T, VW, A>(q, k) - K : A(0);
+      }
+      n += __popc(valid);
+    }
+    merge(x, own, n);
+  }
+#pragma unroll
+  for (int off = 1; off < (G < 64 ? G : 64); off <<= 1) w = wf_merge(w, wf_shfl(w, off));
+  if constexpr (G > 64) {
+    __shared__ Welford<A> lds[G / 64];
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
+    __syncthreads();
+    w = lds[0];
+#pragma unroll
+    for (int v = 1; v < G / 64; ++v) w = wf_merge(w, lds[v]);
+  }
+  if (l == 0) {
+    if constexpr (FINAL) {
+      w.mean += K;
+      mom_write<A, T>(w, correction, take_sqrt, out_var + row, out_mean ? out_mean + row : nullptr);
+    } else {
+      A* p = part + 3 * (int64_t)blockIdx.x;
+      p[0] = w.n;
+      p[1] = w.mean;
+      p[2] = w.m2;
+    }
+  }
+}
+
 // BS threads merge a row's chunk triples, each kMomMerge of them loaded ahead
 // of its merges: a wavefront for up to 128, else 1024 threads (the variance of
 // 64 Mi float32 elements, 8192 triples, 83.6 us with a wavefront of 128 merges
@@ -205,22 +302,30 @@ k_moments_final(const T* __restrict__ in, int64_t row_stride, const A* __restric
 }
 
 inline int64_t mom_vecs(int64_t segs, int64_t len, int vw) { return segs * ((len + vw - 1) / vw); }
-inline int64_t mom_chunks(int64_t nvec) { return (nvec + kMomChunk - 1) / kMomChunk; }
+inline int64_t mom_chunks(int64_t rows, int64_t nvec, int esize) {
+  if (esize < 8) return (nvec + kMomChunk - 1) / kMomChunk;
+  return nvec > kMomStreamRow && rows < kMomStreamRows ? (nvec + kMomStreamChunk - 1) / kMomStreamChunk : 1;
+}
 
 template <typename T>
 int moments_launch(const T* in, T* out_var, T* out_mean, int64_t rows, int64_t segs, int64_t len, int64_t row_stride,
                    int64_t seg_stride, double correction, int take_sqrt, void* ws, hipStream_t st) {
   using A = opmath_t<T>;
   constexpr int VW = 16 / (int)sizeof(T);
-  const int64_t nvec = mom_vecs(segs, len, VW), nch = mom_chunks(nvec);
+  const int64_t nvec = mom_vecs(segs, len, VW), nch = mom_chunks(rows, nvec, (int)sizeof(T));
   const int64_t chunk = (nvec + nch - 1) / nch;
   const SegGeom g{rows, row_stride, seg_stride, segs, len, FastDiv(segs > 1 ? (uint32_t)((len + VW - 1) / VW) : 1u), nvec,
                   (uint32_t)chunk};
   if (nch > 1) {
     A* part = static_cast<A*>(ws);
-    k_moments<T, A, VW, 256, kMomVecs, false>
-        <<<(unsigned)(rows * nch), kMomBlock, 0, st>>>(in, g, FastDiv((uint32_t)nch), (A)correction, take_sqrt, nullptr,
-                                                      nullptr, part);
+    const unsigned blocks = (unsigned)(rows * nch);
+    const FastDiv div((uint32_t)nch);
+    if constexpr (sizeof(T) == 8)
+      k_moments_stream<T, A, VW, 256, false>
+          <<<blocks, kMomBlock, 0, st>>>(in, g, div, (A)correction, take_sqrt, nullptr, nullptr, part);
+    else
+      k_moments<T, A, VW, 256, kMomVecs, false>
+          <<<blocks, kMomBlock, 0, st>>>(in, g, div, (A)correction, take_sqrt, nullptr, nullptr, part);
     const int rc = launch_status();
     if (rc) return rc;
     if (nch <= 128)
@@ -262,9 +367,19 @@ int moments_launch(const T* in, T* out_var, T* out_mean, int64_t rows, int64_t s
   if (nvec <= 64) return go(G64{}, N1{});
   if (nvec <= 128) return go(G64{}, N2{});
   if (nvec <= 256) return go(G64{}, N4{});
-  if (nvec <= 512) return go(G256{}, N2{});
-  if (nvec <= 1024) return go(G256{}, N4{});
-  return go(G256{}, N8{});
+  if constexpr (sizeof(T) == 8) {
+    auto stream = [&](auto G) -> int {
+      return slabs(256 / G.value, [&](unsigned blocks, const T* x, const SegGeom& gs, T* v, T* m) {
+        k_moments_stream<T, A, VW, G.value, true>
+            <<<blocks, kMomBlock, 0, st>>>(x, gs, FastDiv(), (A)correction, take_sqrt, v, m, nullptr);
+      });
+    };
+    return nvec <= 2048 && rows >= 1024 ? stream(G64{}) : stream(G256{});
+  } else {
+    if (nvec <= 512) return go(G256{}, N2{});
+    if (nvec <= 1024) return go(G256{}, N4{});
+    return go(G256{}, N8{});
+  }
 }
 
 }  // namespace sa
@@ -277,7 +392,7 @@ int64_t supa_amd_moments_segments_workspace_bytes(int64_t rows, int64_t segs, in
   if (rows < 0 || segs <= 0 || len <= 0) return SUPA_AMD_EINVAL;
   if (dtype != SUPA_AMD_F32 && dtype != SUPA_AMD_BF16 && dtype != SUPA_AMD_F16 && dtype != SUPA_AMD_F64)
     return SUPA_AMD_EDTYPE;
-  const int64_t nch = mom_chunks(mom_vecs(segs, len, 16 / dtype_size(dtype)));
+  const int64_t nch = mom_chunks(rows, mom_vecs(segs, len, 16 / dtype_size(dtype)), dtype_size(dtype));
   return nch == 1 ? 0 : rows * nch * 3 * (dtype == SUPA_AMD_F64 ? 8 : 4);
 }
 
@@ -293,7 +408,7 @@ int supa_amd_moments_segments(const void* in, int32_t dtype, int64_t rows, int64
   const int64_t need = supa_amd_moments_segments_workspace_bytes(rows, segs, len, dtype);
   if (need < 0) return (int)need;
   const int64_t nvec = mom_vecs(segs, len, 16 / dtype_size(dtype));
-  if (rows * mom_chunks(nvec) >= (int64_t(1) << 31) || (segs > 1 && nvec >= (int64_t(1) << 31))) return SUPA_AMD_ELAYOUT;
+  if (rows * mom_chunks(rows, nvec, dtype_size(dtype)) >= (int64_t(1) << 31) || (segs > 1 && nvec >= (int64_t(1) << 31))) return SUPA_AMD_ELAYOUT;
   if (need > 0 && (!workspace || ws_bytes < need)) return SUPA_AMD_EWORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto go = [&](auto* tag) -> int {
