@@ -79,6 +79,35 @@ def test_rows_at_the_edges(vecs, dtype, no_fallback):
         compare(x, g, dtype, shifted)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("vecs, rows", [(128, 1535), (129, 1535), (129, 1536), (256, 1535), (256, 1536), (257, 1023),
+                                        (257, 1024), (512, 3071), (512, 3072), (513, 599), (513, 600), (1024, 600),
+                                        (1025, 599), (1025, 600), (2048, 600), (2049, 599), (2049, 600), (2560, 600)])
+def test_rows_by_their_number(rows, vecs, dtype, no_fallback):
+    """The thread splits that depend on the number of rows, on both sides of
+    each line: every row as the same row is among few."""
+    v = 16 // torch.empty(0, dtype=dtype).element_size()
+    for cols in (vecs * v, vecs * v - 1):
+        x, g = seeded((5, cols), cols, 2.0, dtype), seeded((5, cols), cols + 1, 1.0, dtype)
+        dx, dg = (t.to("supa").expand(-(-rows // 5), 5, cols).reshape(-1, cols)[:rows] for t in (x, g))
+        for log, fwd, bwd, ofwd, obwd in ((True, torch.log_softmax, LSM_BWD, O.log_softmax, O.log_softmax_backward),
+                                          (False, torch.softmax, SM_BWD, O.softmax, O.softmax_backward)):
+            last = slice(rows // 5 * 5 - 5, rows // 5 * 5)
+            y = fwd(dx, 1)
+            gi = bwd(dg, y, 1, dtype)
+            for at in (slice(0, 5), last):
+                yc = y[at].cpu()
+                check_forward(yc, ofwd(x.float().numpy()), dtype, cols * 2.0 ** -24 if log else 0.0)
+                yd = yc.double().numpy()
+                p, t = (np.exp(yd), g.double().numpy()) if log else (yd, g.double().numpy() * yd)
+                atol = 2 * (cols / 16 + 16) * 2.0 ** -24 * np.abs(t).sum(1, keepdims=True) * p
+                check(gi[at], obwd(g.float().numpy(), yc.float().numpy()), dtype, atol)
+            if cols % v == 0:  # rows of one alignment add in one order: as the rows repeat, so do the results
+                for r in (y, gi):
+                    same = bool((r[5:] == r[:-5]).all())
+                    assert same
+
+
 def test_more_rows_than_one_launch(no_fallback):
     """2^28 rows of 8: more threads than a launch holds."""
     if torch.supa.mem_get_info()[0] < 30 << 30:

@@ -261,6 +261,10 @@ k_row_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restri
 // forward 256 threads by 4 and 512 by 4 or 5, backward 1024 by 1 or 2 (bf16
 // [8192, 8192] forward 45 us against 56 with 1024 threads, backward 64 us
 // against 66 with 256).
+// Rows too few to fill the chip that way (256 CUs) take more threads each, so
+// that a row waits for one or two loads a thread: bf16 [512, 4096] backward
+// 11.3 us by wavefronts, 4.6 so, and forward 8.0, 5.0; [256, 8192] forward 5.5
+// with 256 threads, 4.3 so.
 // Launches stay below HIP's 2^32 threads: more rows go in several.
 template <int V, int MAXV, bool BWD, typename F>
 bool row_split(int64_t rows, int64_t cols, int& rc, F&& launch) {
@@ -290,14 +294,16 @@ bool row_split(int64_t rows, int64_t cols, int& rc, F&& launch) {
   if (nv <= 16) return go(IV{}, G16{}, I1{});
   if (nv <= 64) return go(IV{}, G64{}, I1{});
   if (nv <= 128) return go(IV{}, G64{}, I2{});
-  if (nv <= 256) return go(IV{}, G64{}, I4{});
-  if (nv <= 512) return go(IV{}, G64{}, integral_constant<int, 8>{});
+  if (nv <= 256) return rows < 1536 ? go(IV{}, G256{}, I1{}) : go(IV{}, G64{}, I4{});
+  if (nv <= 512) return rows < (BWD ? 3072 : 1024) ? go(IV{}, G256{}, I2{}) : go(IV{}, G64{}, integral_constant<int, 8>{});
   if constexpr (BWD) {
     return nv <= 1024 ? go(IV{}, G1024{}, I1{}) : go(IV{}, G1024{}, I2{});
   } else {
-    if (nv <= 1024) return go(IV{}, G256{}, I4{});
-    if (nv <= 2048) return go(IV{}, G512{}, I4{});
-    return go(IV{}, G512{}, integral_constant<int, MAXV / 512>{});
+    const bool few = rows < 600;
+    if (nv <= 1024) return few ? go(IV{}, G1024{}, I1{}) : go(IV{}, G256{}, I4{});
+    if (nv <= 2048) return few ? go(IV{}, G1024{}, I2{}) : go(IV{}, G512{}, I4{});
+    static_assert(MAXV <= 3 * 1024, "a forward row fits three vectors of 1024 threads");
+    return few ? go(IV{}, G1024{}, integral_constant<int, 3>{}) : go(IV{}, G512{}, integral_constant<int, MAXV / 512>{});
   }
 }
 
