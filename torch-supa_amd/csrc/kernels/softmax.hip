@@ -1179,11 +1179,12 @@ int softmax_forward(const void* in, int32_t in_dtype, void* out, int32_t out_dty
       TO* po = static_cast<TO*>(out);
       // aligned float32 rows of 1025 to 2048 vectors: the persistent kernel
       // ([8192, 8192] 92 us, k_row_fwd 94)
-      if (sizeof(TI) == 4 && cols % V == 0 && cols / V > kRowBlock && cols / V <= 2 * kRowBlock && aligned(in, 16) &&
-          aligned(out, 16)) {
-        k_lsm_fwd_reg<TI, TO, 2, LOG>
-            <<<(unsigned)std::min<int64_t>(rows, kLsmGrid), kRowBlock, 0, st>>>(pi, po, rows, cols);
-        return launch_status();
+      if constexpr (sizeof(TI) == 4) {
+        if (cols % V == 0 && cols / V > kRowBlock && cols / V <= 2 * kRowBlock && aligned(in, 16) && aligned(out, 16)) {
+          k_lsm_fwd_reg<TI, TO, 2, LOG>
+              <<<(unsigned)std::min<int64_t>(rows, kLsmGrid), kRowBlock, 0, st>>>(pi, po, rows, cols);
+          return launch_status();
+        }
       }
       int rc;
       if (row_split<V, kSplitBlock * kFwdNV, false>(
