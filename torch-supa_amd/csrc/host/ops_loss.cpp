@@ -440,12 +440,17 @@ at::Tensor& binary_cross_entropy_backward_out(const at::Tensor& grad, const at::
 //
 // outer and inner sizes around dim d, and whether the spatial kernels take
 // (outer, cols, inner): more than one inner element, 32-bit positions, and,
-// for more classes than a workgroup holds (kSpatialHeld), enough positions
-// for kSpatialBlocks workgroups of kSpatialVecs 16-byte vectors.  Measured on
-// MI355X, forward + backward, spatial kernels / copies and row kernels:
-// float32 [2, 1000, 4096] (128 workgroups) 95 / 148 us, bf16 (64) 107 / 108
-// us, float32 [2, 5000, 1024] (32) 568 / 135 us.
-constexpr int64_t kSpatialHeld = 256, kSpatialBlocks = 128, kSpatialVecs = 16;
+// for more classes than a workgroup holds (kSpatialHeld), enough positions for
+// spatial_blocks(cols) workgroups of kSpatialVecs 16-byte vectors: each walks
+// the classes twice at its own pace, the copies and row kernels at the chip's.
+// Measured on MI355X, us, spatial kernels / copies and row kernels, float32
+// forward and softmax gradient: 1000 classes and 128 workgroups 31 / 43 and 53
+// / 65; 4096 classes and 128 workgroups 188 / 159 and 269 / 241, 192 workgroups
+// 212 / 206 and 335 / 301, 256 workgroups 199 / 350 and 354 / 538; 16384 classes
+// and 192 workgroups 1132 / 952 and 1565 / 1471, 256 workgroups 1304 / 1215 and
+// 1730 / 1828.
+constexpr int64_t kSpatialHeld = 256, kSpatialVecs = 16;
+inline int64_t spatial_blocks(int64_t cols) { return cols <= 2048 ? 128 : (cols <= 8192 ? 256 : 320); }
 struct DimSplit {
   int64_t outer = 1, cols = 1, inner = 1;
   bool spatial = false;
@@ -459,7 +464,7 @@ DimSplit split_dim(const at::Tensor& t, int64_t d) {
   const int64_t vec = 16 / (int64_t)t.element_size();
   const int64_t blocks = s.outer * ((s.inner + vec - 1) / vec) / kSpatialVecs;
   s.spatial = s.inner > 1 && s.outer * s.inner < lim && s.cols < lim &&
-              (s.cols <= kSpatialHeld || blocks >= kSpatialBlocks);
+              (s.cols <= kSpatialHeld || blocks >= spatial_blocks(s.cols));
   return s;
 }
 at::Tensor& softmax_into(bool log, const at::Tensor& self, int64_t dim, bool half_to_float, at::Tensor& out,
