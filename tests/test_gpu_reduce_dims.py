@@ -35,7 +35,7 @@ def check(x, dx, dims, keepdim=False):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
 @pytest.mark.parametrize("shape", [(1, 9), (2, 7), (16, 64), (17, 257), (33, 1023), (4099, 130), (8192, 40), (100003, 3),
-                                   (70001, 17), (3, 70001)])
+                                   (70001, 17), (3, 70001), (3, 32769), (4100, 2051)])
 def test_columns_and_rows(shape, dtype, no_fallback):
     x = seeded(shape, 1, dtype)
     for dx, cx in ((x.to("supa"), x), (x.to("supa").t(), x.t())):

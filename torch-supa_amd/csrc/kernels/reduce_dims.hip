@@ -211,7 +211,13 @@ int cols_run(const T* in, OT* out, int64_t outer, int64_t red, int64_t inner, co
 // numbered across the runs; G threads share a row: 16 lanes or a wavefront
 // for short rows, a workgroup of 256 for long ones, and chunks of `chunk`
 // vectors in blockIdx.y for few long ones.
-template <typename T, typename OT, typename ACC, int VW, int G>
+//
+// STREAM: nontemporal loads, for inputs past 64 MiB; smaller ones were often
+// written just before, are still in a cache and take plain loads (float32
+// [2000, 4096] read over and over 3.8 us, 6.5 with the hint; [1400, 8000] 7.4,
+// 8.5; [8000, 12000] 66 us, 58 with it; a normalisation of [8192, 4096], whose
+// row sums read tensors that left the caches, 811 us, 803 with it).
+template <typename T, typename OT, typename ACC, int VW, int G, bool STREAM>
 __global__ void __launch_bounds__(kDimSumBlock)
 k_sum_segs(const T* __restrict__ in, OT* __restrict__ out, SegGeom g, ACC scale) {
   constexpr int U = 4;
@@ -223,20 +229,32 @@ k_sum_segs(const T* __restrict__ in, OT* __restrict__ out, SegGeom g, ACC scale)
   const uint32_t nvec = (uint32_t)g.nvec;
   const uint32_t hi = nvec - lo < g.chunk ? nvec : lo + g.chunk;
   ACC acc = ACC(0);
-  for (uint32_t i0 = lo + l; i0 < hi; i0 += U * G) {
+  auto add = [&](const sum_raw_t<T, VW>& w) {
+    ACC t = sum_elem<T, VW, ACC>(w, 0);
+#pragma unroll
+    for (int k = 1; k < VW; ++k) t += sum_elem<T, VW, ACC>(w, k);
+    acc += t;
+  };
+  uint32_t i0 = lo + l;
+  if constexpr (G > 16) {  // rows of one run: steps of whole vectors without a look at each
+    const uint32_t whole = g.runs > 1 ? 0u : (uint32_t)min((int64_t)hi, g.len / VW);
+    for (; i0 + (U - 1) * G < whole; i0 += U * G) {
+      sum_raw_t<T, VW> w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = sum_load<T, VW, STREAM>(src + (int64_t)(i0 + u * G) * VW);
+#pragma unroll
+      for (int u = 0; u < U; ++u) add(w[u]);
+    }
+  }
+  for (; i0 < hi; i0 += U * G) {
     sum_raw_t<T, VW> w[U];
     uint32_t valid;  // elements past a run's end are zeros
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i0 + u * G < hi) w[u] = seg_load<T, VW>(src, g, i0 + u * G, valid);
+      if (i0 + u * G < hi) w[u] = seg_load<T, VW, STREAM>(src, g, i0 + u * G, valid);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i0 + u * G < hi) {
-        ACC t = sum_elem<T, VW, ACC>(w[u], 0);
-#pragma unroll
-        for (int k = 1; k < VW; ++k) t += sum_elem<T, VW, ACC>(w[u], k);
-        acc += t;
-      }
+      if (i0 + u * G < hi) add(w[u]);
   }
 #pragma unroll
   for (int off = (G < 64 ? G : 64) / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
@@ -252,21 +270,29 @@ k_sum_segs(const T* __restrict__ in, OT* __restrict__ out, SegGeom g, ACC scale)
 }
 
 // Chunks per row: rows too few for kDimSumBlocks workgroups are cut in chunks
-// of at least 8 vectors a thread.
+// of at least 8 vectors a thread, from 32 on (the second launch costs 2 us:
+// float32 [700, 16384], 16 vectors a thread, 7.1 us in one launch, 11.1 in two;
+// [1, 16384] 4.3, 6.7).
 inline int64_t seg_chunks(int64_t rows, int64_t nvec) {
-  const int64_t most = nvec / (8 * kDimSumBlock);
-  return std::max<int64_t>(1, std::min<int64_t>(most, (kDimSumBlocks + rows - 1) / rows));
+  const int64_t most = nvec >= 32 * kDimSumBlock ? nvec / (8 * kDimSumBlock) : 1;
+  return std::max<int64_t>(1, std::min<int64_t>(most, kDimSumBlocks / rows));
 }
+
+constexpr int64_t kSegStreamBytes = int64_t(64) << 20;
 
 template <typename T, typename OT, typename ACC, int VW>
 int segs_launch(const T* in, OT* out, const SegGeom& g, unsigned nch, ACC scale, hipStream_t st) {
+  const bool stream = VW > 1 && g.rows * g.nvec * 16 > kSegStreamBytes;
   auto go = [&](auto G) -> int {
     constexpr int64_t per = kDimSumBlock / G.value, slab = per * kDimSumSlab;
     for (int64_t r0 = 0; r0 < g.rows; r0 += slab) {
       SegGeom gs = g;
       gs.rows = std::min(slab, g.rows - r0);
+      const T* x = in + r0 * g.row_stride;
+      OT* y = out + r0 * nch;
       const dim3 grid((unsigned)((gs.rows + per - 1) / per), nch);
-      k_sum_segs<T, OT, ACC, VW, G.value><<<grid, kDimSumBlock, 0, st>>>(in + r0 * g.row_stride, out + r0 * nch, gs, scale);
+      if (stream) k_sum_segs<T, OT, ACC, VW, G.value, VW != 1><<<grid, kDimSumBlock, 0, st>>>(x, y, gs, scale);
+      else k_sum_segs<T, OT, ACC, VW, G.value, false><<<grid, kDimSumBlock, 0, st>>>(x, y, gs, scale);
       const int rc = launch_status();
       if (rc) return rc;
     }
@@ -275,7 +301,7 @@ int segs_launch(const T* in, OT* out, const SegGeom& g, unsigned nch, ACC scale,
   using std::integral_constant;
   // a wavefront per row up to 512 vectors where the rows alone fill the chip
   // (bf16 [6007, 2047] 6.3 us, 11.5 with four)
-  const bool wave = g.rows >= 1024 && g.nvec <= 512;
+  const bool wave = g.rows >= 4096 && g.nvec <= 512;
   if (nch == 1 && g.nvec <= 32) return go(integral_constant<int, 16>{});
   if (nch == 1 && wave) return go(integral_constant<int, 64>{});
   return go(integral_constant<int, 256>{});

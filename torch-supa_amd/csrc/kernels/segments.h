@@ -22,9 +22,9 @@ template <typename T> struct SumRaw<T, 1> {
 };
 template <typename T, int VW> using sum_raw_t = typename SumRaw<T, VW>::type;
 
-template <typename T, int VW> __device__ __forceinline__ sum_raw_t<T, VW> sum_load(const T* p) {
+template <typename T, int VW, bool STREAM = true> __device__ __forceinline__ sum_raw_t<T, VW> sum_load(const T* p) {
   if constexpr (VW == 1) return *p;
-  else return ld_any_stream(p);
+  else return STREAM ? ld_any_stream(p) : ld_any(p);
 }
 template <typename T, int VW, typename ACC>
 __device__ __forceinline__ ACC sum_elem(const sum_raw_t<T, VW>& w, int k) {
@@ -48,7 +48,7 @@ struct SegGeom {
 // Vector i of a row (across its runs).  A run's last short vector comes back
 // with zeros in place of the elements that are not its own; bit k of `valid`
 // is set for element k that is.
-template <typename T, int VW>
+template <typename T, int VW, bool STREAM = true>
 __device__ __forceinline__ sum_raw_t<T, VW> seg_load(const T* row, const SegGeom& g, int64_t i, uint32_t& valid) {
   valid = (1u << VW) - 1u;
   const T* p = row + i * VW;
@@ -62,7 +62,7 @@ __device__ __forceinline__ sum_raw_t<T, VW> seg_load(const T* row, const SegGeom
   if constexpr (VW == 1) {
     return *p;
   } else {
-    if (left >= VW) return ld_any_stream(p);
+    if (left >= VW) return sum_load<T, VW, STREAM>(p);
     T w[VW];
     uint4 q;
     if (g.len >= VW) {  // the run's last vector, zeros for what the one before holds
