@@ -197,6 +197,17 @@ def test_fused_cross_entropy_special_values(c, dtype, no_fallback, fused_ce):
             torch.testing.assert_close(d.grad.cpu().double(), r.grad, rtol=tol, atol=tol, equal_nan=True)
 
 
+def test_losses_of_short_odd_runs(no_fallback):
+    """Runs of a few vectors with a broadcast weight, from one workgroup to all of them."""
+    for shape in ((1, 9), (3, 100), (700, 13), (8192, 100), (40000, 33)):
+        for dtype in (torch.float32, torch.bfloat16):
+            x, t = seeded(shape, 29, dtype), (seeded(shape, 30) > 0).to(dtype)
+            w = (seeded(shape[1:], 31).abs() + 0.5).to(dtype)
+            got = F.binary_cross_entropy_with_logits(x.to("supa"), t.to("supa"), pos_weight=w.to("supa"))
+            want = F.binary_cross_entropy_with_logits(x.double(), t.double(), pos_weight=w.double())
+            torch.testing.assert_close(got.cpu().double(), want, rtol=1e-5 if dtype == torch.float32 else 1e-2, atol=0)
+
+
 @pytest.mark.parametrize("prob", [False, True])
 def test_cross_entropy_of_more_rows_than_one_launch(prob, no_fallback, fused_ce):
     """2^26 rows (2^24 with probability targets): more threads than a launch holds."""
