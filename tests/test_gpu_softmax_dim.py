@@ -106,6 +106,23 @@ def test_spatial_softmax_layouts_and_special_values(no_fallback):
                                rtol=1e-5, atol=1e-6)
 
 
+def test_spatial_softmax_over_a_shifted_view(no_fallback):
+    """An output that overlaps the input out of step is written after the input is read."""
+    n, shape = 2 * 19 * 515, (2, 19, 515)
+    x, g = seeded(shape, 7, 2.0), seeded(shape, 8)
+    want = torch.softmax(x.to("supa"), 1)
+    gwant = SM_BWD(g.to("supa"), want, 1, torch.float32)
+    for off in (1, 515):
+        buf = torch.empty(n + off, device="supa")
+        src, dst = buf[:n].view(shape), buf[off:].view(shape)
+        src.copy_(x.to("supa"))
+        torch.ops.aten._softmax.out(src, 1, False, out=dst)
+        assert torch.equal(dst.cpu(), want.cpu())
+        src.copy_(g.to("supa"))
+        SM_BWD.out(src, want, 1, torch.float32, grad_input=dst)
+        assert torch.equal(dst.cpu(), gwant.cpu())
+
+
 @pytest.mark.parametrize("shape", [(1, 4096, 128, 128), (1, 1000, 64, 128)])
 def test_spatial_gradient_precision(shape, no_fallback):
     """The sums over many streamed classes against 64 bits.  A sum of n equal

@@ -467,6 +467,12 @@ DimSplit split_dim(const at::Tensor& t, int64_t d) {
               (s.cols <= kSpatialHeld || blocks >= spatial_blocks(s.cols));
   return s;
 }
+// Whether the spatial kernels may write `out` while they read `in`: no memory in
+// common, or element for element the same (a shifted view would be overwritten
+// ahead of its reads).
+bool in_place_or_apart(const at::Tensor& out, const at::Tensor& in) {
+  return !out.is_alias_of(in) || (out.data_ptr() == in.data_ptr() && out.scalar_type() == in.scalar_type());
+}
 at::Tensor& softmax_into(bool log, const at::Tensor& self, int64_t dim, bool half_to_float, at::Tensor& out,
                          const char* name) {
   TORCH_CHECK(is_float_dtype(self.scalar_type()), name, ": expected a floating-point input, got ", self.scalar_type());
@@ -490,7 +496,9 @@ at::Tensor& softmax_into(bool log, const at::Tensor& self, int64_t dim, bool hal
   const DimSplit sp = split_dim(self, d);
   if (sp.spatial && !self.movedim(d, -1).is_contiguous()) {
     at::Tensor x = self.contiguous();
-    at::Tensor res = out.is_contiguous() ? out : empty_supa(self.sizes(), odt, self.device().index());
+    at::Tensor res = out.is_contiguous() && in_place_or_apart(out, x)
+                         ? out
+                         : empty_supa(self.sizes(), odt, self.device().index());
     check_status(supa_amd_softmax_dim_forward(log ? 1 : 0, x.data_ptr(), dtype_code(x.scalar_type()), res.data_ptr(),
                                               dtype_code(odt), sp.outer, sp.cols, sp.inner,
                                               current_stream(self.device().index())),
@@ -542,7 +550,7 @@ at::Tensor& softmax_bwd_into(bool log, const at::Tensor& grad, const at::Tensor&
     at::Tensor g = to_dtype(grad.contiguous(), gdt);
     at::Tensor y = to_dtype(output.contiguous(), gdt);
     const c10::ScalarType kdt = gi.scalar_type() == gdt ? gdt : at::kFloat;
-    at::Tensor res = gi.is_contiguous() && gi.scalar_type() == kdt
+    at::Tensor res = gi.is_contiguous() && gi.scalar_type() == kdt && in_place_or_apart(gi, g) && in_place_or_apart(gi, y)
                          ? gi
                          : empty_supa(grad.sizes(), kdt, grad.device().index());
     check_status(supa_amd_softmax_dim_backward(log ? 1 : 0, g.data_ptr(), y.data_ptr(), dtype_code(gdt),
