@@ -197,6 +197,27 @@ def test_fused_cross_entropy_special_values(c, dtype, no_fallback, fused_ce):
             torch.testing.assert_close(d.grad.cpu().double(), r.grad, rtol=tol, atol=tol, equal_nan=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("n", [65535, 65536, 70001])
+def test_nll_loss_of_many_rows(n, dtype, no_fallback):
+    """Both sides of the line between one launch and two."""
+    lp = -seeded((n, 5), 26).abs().to(dtype)
+    t = torch.randint(0, 5, (n,), generator=torch.Generator().manual_seed(27))
+    t[::11] = -100
+    w = (seeded((5,), 28).abs() + 0.5).to(dtype)
+    for red in ("mean", "sum"):
+        for weight in (None, w):
+            got = F.nll_loss(lp.to("supa"), t.to("supa"), None if weight is None else weight.to("supa"), reduction=red)
+            want = F.nll_loss(lp.double(), t, None if weight is None else weight.double(), reduction=red)
+            # chains of at most n / 1024 + 64 float32 additions of one sign, then one rounding
+            tol = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float64: 0.0}[dtype]
+            tol += 2 * (n / 1024 + 64) * 2.0 ** (-53 if dtype == torch.float64 else -24)
+            torch.testing.assert_close(got.cpu().double(), want, rtol=tol, atol=0)
+    t[-1] = 5
+    with pytest.raises(IndexError):
+        F.nll_loss(lp.to("supa"), t.to("supa")).cpu()
+
+
 def test_losses_of_short_odd_runs(no_fallback):
     """Runs of a few vectors with a broadcast weight, from one workgroup to all of them."""
     for shape in ((1, 9), (3, 100), (700, 13), (8192, 100), (40000, 33)):
