@@ -66,7 +66,7 @@ ExtResult argext(const at::Tensor& self, std::vector<int64_t> dims, bool keepdim
   for (int64_t d : dims) perm.push_back(d);
   const auto dev = self.device().index();
   // one dim between or before kept ones: read where it lies
-  if (dims.size() == 1 && inner > 1 && self.numel() > 0) {
+  if (dims.size() == 1 && inner > 1 && self.numel() > 0 && self.stride(dims[0]) != 1) {
     const DimPlan p = dim_plan(self, red);
     const int64_t vec = 16 / (int64_t)self.element_size();
     if (p.kind == DimPlan::kCols && p.inner >= vec && p.red < (int64_t(1) << 31) &&
