@@ -229,6 +229,22 @@ def test_losses_of_short_odd_runs(no_fallback):
             torch.testing.assert_close(got.cpu().double(), want, rtol=1e-5 if dtype == torch.float32 else 1e-2, atol=0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_fused_cross_entropy_gradient_at_any_alignment(dtype, no_fallback, fused_ce):
+    """Rows of whole vectors that start at a boundary and off it: the same bits."""
+    for n, c in ((1, 8), (37, 64), (5, 1000), (9, 4104)):
+        flat = seeded((n * c + 8,), 37, dtype).to("supa")
+        t = (torch.arange(n) * 7 % c).to("supa")
+        for off in (0, 1, 3, 8):
+            x = flat[off:off + n * c].view(n, c)
+            grads = []
+            for logits in (x, x.clone()):
+                logits = logits.detach().requires_grad_()
+                F.cross_entropy(logits, t).backward()
+                grads.append(logits.grad)
+            assert torch.equal(grads[0].cpu(), grads[1].cpu()), (n, c, off)
+
+
 @pytest.mark.parametrize("prob", [False, True])
 def test_cross_entropy_of_more_rows_than_one_launch(prob, no_fallback, fused_ce):
     """2^26 rows (2^24 with probability targets): more threads than a launch holds."""

@@ -257,12 +257,14 @@ int ce_final(float* rows, const int64_t* target, int64_t n, int64_t c, int64_t i
 // go element by element.
 //
 // grad[i, :] over a 2-d grid: blockIdx.y = row in the slab, x = column blocks
-// of kCeBwdBlock vectors.  A whole vector's logits load goes out unconditionally, before the row's target,
-// and the scale and lse that depend on it, have arrived (an ignored row then
-// reads logits it does not need); waiting for the target first held the
-// kernel at 75 % of the HBM roofline on c3's bf16 rows, against 85 % with the
-// load first.
-template <typename T>
+// of kCeBwdBlock vectors.  WHOLE: rows of whole aligned vectors.  A vector's
+// logits load then goes out unconditionally, before the row's target, and the
+// scale and lse that depend on it, have arrived (an ignored row then reads
+// logits it does not need); waiting for the target first, as the kernel does
+// that has partial vectors to tell from whole ones, held it at 75 % of the HBM
+// roofline on c3's bf16 rows, against 85 % with the load first (forward and
+// backward 1002 us and 921; float32 1837 and 1804).
+template <typename T, bool WHOLE>
 __global__ void __launch_bounds__(kCeBwdBlock)
 k_ce_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const int64_t* __restrict__ target,
          const float* __restrict__ lse, const float* __restrict__ count, int64_t c, int64_t ignore_index,
@@ -271,10 +273,10 @@ k_ce_bwd(const T* __restrict__ grad_out, const T* __restrict__ x, const int64_t*
   const int64_t row = blockIdx.y;
   const T* xr = x + row * c;
   T* dst = gx + row * c;
-  const int64_t col0 = ((int64_t)blockIdx.x * kCeBwdBlock + threadIdx.x) * V - grid_off<T, V>(dst, c);
+  const int64_t col0 = ((int64_t)blockIdx.x * kCeBwdBlock + threadIdx.x) * V - (WHOLE ? 0 : grid_off<T, V>(dst, c));
   if (col0 >= c) return;
   Vec<T, V> w;
-  const bool whole = col0 >= 0 && col0 + V <= c;
+  const bool whole = WHOLE || (col0 >= 0 && col0 + V <= c);
   if (whole) w = ld_vec_any<true, T, V>(xr + col0);
   const int64_t t = target[row];
   const bool kept = ce_kept(t, c, ignore_index);
@@ -550,13 +552,18 @@ int supa_amd_cross_entropy_backward(const void* grad_out, const void* logits, in
     const T* g = static_cast<const T*>(grad_out);
     const T* x = static_cast<const T*>(logits);
     T* gx = static_cast<T*>(grad_logits);
+    const bool whole = c % V == 0 && aligned(x, 16) && aligned(gx, 16);
     const unsigned gx_blocks = (unsigned)((grid_vecs<T, V>(gx, c) + kCeBwdBlock - 1) / kCeBwdBlock);
     for (int64_t r0 = 0; r0 < n; r0 += 65535) {
       const int64_t rows = std::min<int64_t>(65535, n - r0);
       const T* gs = reduction == SUPA_AMD_REDUCTION_NONE ? g + r0 : g;
       const dim3 grid(gx_blocks, (unsigned)rows);
-      k_ce_bwd<T><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, target + r0, lse + r0, count, c, ignore_index,
-                                                reduction, gx + r0 * c);
+      if (whole)
+        k_ce_bwd<T, true><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, target + r0, lse + r0, count, c, ignore_index,
+                                                        reduction, gx + r0 * c);
+      else
+        k_ce_bwd<T, false><<<grid, kCeBwdBlock, 0, st>>>(gs, x + r0 * c, target + r0, lse + r0, count, c, ignore_index,
+                                                         reduction, gx + r0 * c);
       const int rc = launch_status();
       if (rc) return rc;
     }
