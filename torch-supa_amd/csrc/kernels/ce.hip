@@ -383,37 +383,24 @@ k_ce_prob_fwd(const T* __restrict__ x, const T* __restrict__ tgt, int64_t c, flo
 #pragma unroll
         for (int k = 0; k < V; ++k) mb = fmaxf(mb, ce_elem<T>(wx[u], k));
       }
-    const float M = fmaxf(st.m, mb);
-    if (M != -__builtin_inff()) {
-      if (st.m != -__builtin_inff()) {
-        st.s *= __builtin_amdgcn_exp2f((st.m - M) * kCeLog2e);
-        st.B = fmaf(st.T, st.m - M, st.B);
-      }
-      st.m = M;
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (v0 + (int64_t)u * kCeBlock < nvec) {
-#pragma unroll
-          for (int k = 0; k < V; ++k) {
-            const float xv = ce_elem<T>(wx[u], k), tv = ce_elem<T>(wt[u], k);
-            st.s += __builtin_amdgcn_exp2f((xv - M) * kCeLog2e);
-            st.T += tv;
-            st.B = fmaf(tv, xv - M, st.B);
-          }
-        }
-    } else {  // every value so far -inf, or NaN: s stays 0, or NaN; B = sum t x
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (v0 + (int64_t)u * kCeBlock < nvec) {
-#pragma unroll
-          for (int k = 0; k < V; ++k) {
-            const float xv = ce_elem<T>(wx[u], k), tv = ce_elem<T>(wt[u], k);
-            st.s += __builtin_amdgcn_exp2f(xv);
-            st.T += tv;
-            st.B = fmaf(tv, xv, st.B);
-          }
-        }
+    // every value so far -inf, or NaN: s stays 0, or NaN; B = sum t x
+    const float M = fmaxf(st.m, mb), base = M == -__builtin_inff() ? 0.0f : M;
+    if (st.m != -__builtin_inff()) {
+      st.s *= __builtin_amdgcn_exp2f((st.m - M) * kCeLog2e);
+      st.B = fmaf(st.T, st.m - M, st.B);
     }
+    st.m = M;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (v0 + (int64_t)u * kCeBlock < nvec) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          const float xv = ce_elem<T>(wx[u], k), tv = ce_elem<T>(wt[u], k);
+          st.s += __builtin_amdgcn_exp2f((xv - base) * kCeLog2e);
+          st.T += tv;
+          st.B = fmaf(tv, xv - base, st.B);
+        }
+      }
   }
   // the elements after the whole vectors
   for (int64_t j = nvec * V + threadIdx.x; j < c; j += kCeBlock)
