@@ -229,6 +229,30 @@ def test_losses_of_short_odd_runs(no_fallback):
             torch.testing.assert_close(got.cpu().double(), want, rtol=1e-5 if dtype == torch.float32 else 1e-2, atol=0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_losses_of_whole_runs_beside_a_weight(dtype, no_fallback):
+    """Whole aligned vectors beside an operand that is read again, below and above
+    the size from which the others stream.  The mean of equal rows is that of one;
+    bounds: n / 2^24 additions of one sign for float32, half a step for bfloat16."""
+    for rows, cols in ((3, 8), (64, 264), (1000, 4096), (40, 1 << 20), (72, 1 << 20)):
+        x, t = seeded((cols + 8,), 34, dtype), (seeded((cols,), 35) > 0).to(dtype)
+        w = (seeded((cols,), 36).abs() + 0.5).to(dtype)
+        xs = torch.empty(rows, cols + 8, dtype=dtype, device="supa")
+        ts = torch.empty(rows, cols, dtype=dtype, device="supa")
+        xs.copy_(x.to("supa"))
+        ts.copy_(t.to("supa"))
+        rtol = 1e-5 if dtype == torch.float32 else 2.0 ** -8
+        for view in (xs[:, 8:], xs[:, 8:].contiguous()):
+            got = F.binary_cross_entropy_with_logits(view, ts, pos_weight=w.to("supa"))
+            want = F.binary_cross_entropy_with_logits(x[8:].double(), t.double(), pos_weight=w.double())
+            torch.testing.assert_close(got.cpu().double(), want, rtol=rtol, atol=0)
+            got = F.mse_loss(view, w.to("supa").expand_as(view))
+            want = F.mse_loss(x[8:].double(), w.double())
+            torch.testing.assert_close(got.cpu().double(), want, rtol=rtol, atol=0)
+        del xs, ts, view
+    torch.supa.empty_cache()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_fused_cross_entropy_gradient_at_any_alignment(dtype, no_fallback, fused_ce):
     """Rows of whole vectors that start at a boundary and off it: the same bits."""

@@ -25,9 +25,18 @@ namespace sa {
 
 constexpr int kRedBlocks = 1024;   // stage-1 grid (capped by the work)
 constexpr int kRedBlock = 256;     // stage-1 workgroup
+// Beside an operand that is read again, the others stream past the caches (a
+// nontemporal hint) from this many bytes on, what the last-level cache holds:
+// BCE with a weight per column of float32 [32, 1048576], 256 MiB in fresh
+// tensors each call, 43 us, 47 without the hint; bf16 [4096, 8192], 128 MiB
+// that the caches hold, 32 us without it, 41 with it, and 41 either way in
+// fresh tensors.
+constexpr int64_t kRedStreamBytes = int64_t(256) << 20;
 constexpr int kCounterBytes = 256; // reserved head of the workspace (keeps partials 256-byte aligned)
 
-enum RedLayout { R_CONTIG = 0, R_VECND = 1, R_STRIDED = 2 };
+// R_VECND: runs of whole aligned vectors; R_VECND_ANY: runs of any length from
+// one vector on, at element alignment.
+enum RedLayout { R_CONTIG = 0, R_VECND = 1, R_STRIDED = 2, R_VECND_ANY = 3 };
 
 template <int BS, typename ACC>
 __device__ __forceinline__ ACC block_sum(ACC v, ACC* lds) {
@@ -90,16 +99,21 @@ __device__ __forceinline__ ACC accumulate(const Op& op, const TArgs<1 + sizeof..
       }(std::make_integer_sequence<int, N>{});
       acc += (ACC)op(y);
     }
-  } else if constexpr (LAYOUT == R_VECND) {
-    const uint32_t nvec = g.div[0].d * (uint32_t)(n / g.size[0]);
+  } else if constexpr (LAYOUT == R_VECND || LAYOUT == R_VECND_ANY) {
+    constexpr bool WHOLE = LAYOUT == R_VECND;
+    const uint32_t nvec = WHOLE ? (uint32_t)(n / VEC) : g.div[0].d * (uint32_t)(n / g.size[0]);
     for (uint32_t v = (uint32_t)tid; v < nvec; v += (uint32_t)nthreads) {
       uint32_t q, r;
-      g.div[0].divmod(v, q, r);  // vectors of a run
-      r *= VEC;
       uint32_t skip = 0;  // a run's last vector ends at its end; the elements another one holds do not count
-      if (r + VEC > g.size[0]) {
-        skip = r + VEC - g.size[0];
-        r = g.size[0] - VEC;
+      if constexpr (WHOLE) {
+        g.div[0].divmod(v * VEC, q, r);
+      } else {
+        g.div[0].divmod(v, q, r);  // vectors of a run
+        r *= VEC;
+        if (r + VEC > g.size[0]) {
+          skip = r + VEC - g.size[0];
+          r = g.size[0] - VEC;
+        }
       }
       int64_t off[1 + N];
 #pragma unroll
@@ -121,7 +135,13 @@ __device__ __forceinline__ ACC accumulate(const Op& op, const TArgs<1 + sizeof..
 #pragma unroll
              for (int k = 0; k < VEC; ++k) x[k][I] = s;
            } else {
-             const Vec<St, VEC> w = ld_vec_any<!BC, St, VEC>(p);
+             // runs that are not whole vectors share cache lines: no hint where some operand is read again
+             Vec<St, VEC> w;
+             if constexpr (WHOLE)
+               w = (BC && a.mode[1 + I]) ? *reinterpret_cast<const Vec<St, VEC>*>(p)
+                                         : ld_stream(reinterpret_cast<const Vec<St, VEC>*>(p));
+             else
+               w = ld_vec_any<!BC, St, VEC>(p);
 #pragma unroll
              for (int k = 0; k < VEC; ++k) x[k][I] = load_cvt<C, CT>(w.v[k]);
            }
@@ -222,26 +242,41 @@ int launch_reduce(const Op& op, const supa_amd_ew_desc& d, const int* tin, doubl
   if (contig) layout = R_CONTIG;
   if (layout != R_CONTIG) {
     if (n >= (int64_t(1) << 31)) return SUPA_AMD_ELAYOUT;
-    // runs of any length (from one vector on) at any alignment
     bool vnd = VEC > 1 && d.ndim >= 1 && d.sizes[0] >= VEC;
-    for (int i = 0; i < N && vnd; ++i) vnd = a.st[1 + i][0] == 0 || a.st[1 + i][0] == 1;
-    layout = vnd ? R_VECND : R_STRIDED;
+    bool whole = d.sizes[0] % VEC == 0;
+    for (int i = 0; i < N && vnd; ++i) {
+      const int64_t s0 = a.st[1 + i][0];
+      vnd = s0 == 0 || s0 == 1;
+      if (s0 == 0) continue;
+      whole = whole && aligned(a.p[1 + i], VEC * sizes_of[i]);
+      for (int j = 1; j < d.ndim; ++j) whole = whole && a.st[1 + i][j] % VEC == 0;
+    }
+    // Whole vectors keep a kernel without the look at a run's end and with the
+    // hint per operand.
+    layout = !vnd ? R_STRIDED : whole ? R_VECND : R_VECND_ANY;
     if (vnd) {
       // operands broadcast along an outer dim are re-read: keep them cached
+      bool any = false;
+      int64_t once = 0;
       for (int i = 0; i < N; ++i) {
         a.mode[1 + i] = 0;
         for (int j = 1; j < d.ndim; ++j)
           if (a.st[1 + i][j] == 0 && d.sizes[j] > 1) a.mode[1 + i] = 1;
+        const bool again = a.mode[1 + i] != 0 || a.st[1 + i][0] == 0;
+        any = any || again;
+        if (!again) once += n * sizes_of[i];
       }
+      if (any && once < kRedStreamBytes)
+        for (int i = 0; i < N; ++i) a.mode[1 + i] = 1;
     }
   }
   NdGeom g = make_geom(d);
-  if (layout == R_VECND) g.div[0] = FastDiv((uint32_t)((d.sizes[0] + VEC - 1) / VEC));
+  if (layout == R_VECND_ANY) g.div[0] = FastDiv((uint32_t)((d.sizes[0] + VEC - 1) / VEC));
   // Four vectors (or elements) a thread; one of a run's vectors, so that small
   // inputs keep the chip busy (bf16 [8192, 100] with a weight per column: 10.4
   // us with four, 8.5 one element at a time).
   const int64_t units = layout == R_STRIDED ? n : std::max<int64_t>(n / VEC, 1);
-  const int64_t per = layout == R_VECND ? kRedBlock : 4 * kRedBlock;
+  const int64_t per = layout == R_VECND || layout == R_VECND_ANY ? kRedBlock : 4 * kRedBlock;
   const int64_t want = (units + per - 1) / per;
   const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, kRedBlocks));
   bool bc = false;
@@ -255,6 +290,10 @@ int launch_reduce(const Op& op, const supa_amd_ew_desc& d, const int* tin, doubl
     case R_VECND:
       if (bc) k_reduce_partial<kRedBlock, R_VECND, VEC, true, Op, C, CT, ACC, S...><<<blocks, kRedBlock, 0, st>>>(op, a, g, n, partial);
       else k_reduce_partial<kRedBlock, R_VECND, VEC, false, Op, C, CT, ACC, S...><<<blocks, kRedBlock, 0, st>>>(op, a, g, n, partial);
+      break;
+    case R_VECND_ANY:
+      if (bc) k_reduce_partial<kRedBlock, R_VECND_ANY, VEC, true, Op, C, CT, ACC, S...><<<blocks, kRedBlock, 0, st>>>(op, a, g, n, partial);
+      else k_reduce_partial<kRedBlock, R_VECND_ANY, VEC, false, Op, C, CT, ACC, S...><<<blocks, kRedBlock, 0, st>>>(op, a, g, n, partial);
       break;
     default:
       k_reduce_partial<kRedBlock, R_STRIDED, 1, false, Op, C, CT, ACC, S...><<<blocks, kRedBlock, 0, st>>>(op, a, g, n, partial);
