@@ -18,11 +18,11 @@
 // covers, so every position is written once, by a thread that read it first
 // (the output may be the input).
 //
-// Measured on MI355X, float32 [8, 19, 512, 512] (159 MB a tensor): forward 55
-// us (5.8 TB/s), backward 80 us (6.0 TB/s), where copying the planes to rows,
-// one 256-thread workgroup per 19-element row, and copying back took 2855 and
-// 2442 us; bf16 35 and 42 us (1752 and 1181); planes of 262143 elements 65
-// and 93 us; float32 [4, 150, 256, 256] 62 and 96 us (808 and 994).
+// Measured on MI355X, float32 [8, 19, 512, 512] (159 MB a tensor): forward 57
+// us (5.6 TB/s), backward 80 us (6.0 TB/s), where copying the planes to rows,
+// one 256-thread workgroup per 19-element row, and copying back took 2870 and
+// 2440 us; bf16 37 and 42 us (1755 and 1190); planes of 262143 elements 65
+// and 93 us; float32 [4, 150, 256, 256] 62 and 94 us (818 and 985).
 //
 // Replaces _log_softmax.out (NF:3752), _log_softmax_backward_data.out
 // (NF:3763), _softmax.out and _softmax_backward_data.out over inner dims
@@ -105,45 +105,41 @@ __device__ __forceinline__ DimPlace dim_place(const DimGeom& g) {
   return r;
 }
 
-// (max, sum) pairs per position combined over the TY class groups; every
-// thread of a position ends with the same values.
+// The maximum, or the sum, per position over the TY class groups; every thread
+// of a position ends with the same values.
 template <int VW, int TXL>
-__device__ __forceinline__ void dim_lse(float (&m)[VW], float (&s)[VW], float* lds) {
+__device__ __forceinline__ void dim_max(float (&m)[VW], float* lds) {
   constexpr int TX = 1 << TXL, NW = kDimBlock / 64;
 #pragma unroll
   for (int off = TX; off < 64; off <<= 1) {
 #pragma unroll
-    for (int k = 0; k < VW; ++k) {
-      const float m2 = __shfl_xor(m[k], off, 64), s2 = __shfl_xor(s[k], off, 64);
-      const float M = fmaxf(m[k], m2);
-      s[k] = lse_rescale(s[k], m[k], M) + lse_rescale(s2, m2, M);
-      m[k] = M;
-    }
+    for (int k = 0; k < VW; ++k) m[k] = fmaxf(m[k], __shfl_xor(m[k], off, 64));
   }
   if constexpr (TX <= 64) {  // the wavefronts hold different classes of the same positions
     const int wave = threadIdx.x >> 6, tx = threadIdx.x & (TX - 1);
-    float* lm = lds;
-    float* ls = lds + NW * TX * VW;
     if ((threadIdx.x & 63) < TX) {
 #pragma unroll
-      for (int k = 0; k < VW; ++k) {
-        lm[(wave * VW + k) * TX + tx] = m[k];
-        ls[(wave * VW + k) * TX + tx] = s[k];
-      }
+      for (int k = 0; k < VW; ++k) lds[(wave * VW + k) * TX + tx] = m[k];
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < VW; ++k) {
-      float M = lm[k * TX + tx];
+      float M = lds[k * TX + tx];
 #pragma unroll
-      for (int w = 1; w < NW; ++w) M = fmaxf(M, lm[(w * VW + k) * TX + tx]);
-      float S = 0.0f;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) S += lse_rescale(ls[(w * VW + k) * TX + tx], lm[(w * VW + k) * TX + tx], M);
+      for (int w = 1; w < NW; ++w) M = fmaxf(M, lds[(w * VW + k) * TX + tx]);
       m[k] = M;
-      s[k] = S;
     }
   }
+}
+
+// t[0] + ... + t[N - 1] by a tree.
+template <int N>
+__device__ __forceinline__ float dim_tree(float (&t)[N]) {
+#pragma unroll
+  for (int h = 1; h < N; h *= 2)
+#pragma unroll
+    for (int i = 0; i + h < N; i += 2 * h) t[i] += t[i + h];
+  return t[0];
 }
 
 template <int VW, int TXL>
@@ -163,10 +159,10 @@ __device__ __forceinline__ void dim_sum(float (&s)[VW], float* lds) {
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < VW; ++k) {
-      float S = lds[k * TX + tx];
+      float w[NW];
 #pragma unroll
-      for (int w = 1; w < NW; ++w) S += lds[(w * VW + k) * TX + tx];
-      s[k] = S;
+      for (int i = 0; i < NW; ++i) w[i] = lds[(i * VW + k) * TX + tx];
+      s[k] = dim_tree<NW>(w);
     }
   }
 }
@@ -174,11 +170,16 @@ __device__ __forceinline__ void dim_sum(float (&s)[VW], float* lds) {
 // HOLD: the thread's classes (at most NC) stay in registers between the
 // statistics and the output; otherwise they stream through in groups of NC,
 // twice (plain loads first, so that the second pass may find them cached).
+// The maximum of all groups comes before the exponentials that are held, and
+// before the one rescale of those that stream: each rescale costs the sum two
+// roundings.
 template <typename TI, typename TO, int VW, int TXL, int NC, bool HOLD, bool LOG>
 __global__ void __launch_bounds__(kDimBlock)
 k_dim_fwd(const TI* __restrict__ in, TO* __restrict__ out, DimGeom g) {
   constexpr int TX = 1 << TXL, TY = kDimBlock / TX;
-  __shared__ float lds[TX <= 64 ? 2 * (kDimBlock / 64) * TX * VW : 1];
+  constexpr int GRP = VW <= 4 ? 4 : 2;  // classes added by a tree; of eight positions four cost registers
+  constexpr int LDS_SUM = TX <= 64 ? (kDimBlock / 64) * TX * VW : 0;  // the sums' place, then the maxima's
+  __shared__ float lds[TX <= 64 ? 2 * LDS_SUM : 1];
   const DimPlace at = dim_place<VW, TXL>(g);
   const uint32_t ty = threadIdx.x >> TXL;
   const TI* src = in + at.base;
@@ -205,6 +206,7 @@ k_dim_fwd(const TI* __restrict__ in, TO* __restrict__ out, DimGeom g) {
 #pragma unroll
         for (int k = 0; k < VW; ++k) M[k] = fmaxf(M[k], dim_elem<TI, VW>(x[j], k));
       }
+    if constexpr (HOLD) dim_max<VW, TXL>(M, lds + LDS_SUM);
     float mb[VW];  // all -inf: keep exp arguments finite
 #pragma unroll
     for (int k = 0; k < VW; ++k) {
@@ -213,20 +215,39 @@ k_dim_fwd(const TI* __restrict__ in, TO* __restrict__ out, DimGeom g) {
       mb[k] = M[k] == -__builtin_inff() ? 0.0f : M[k];
     }
     dim_opaque<TI, VW, NC>(x);
-    float t[VW];  // this step's NC classes, then the steps: no chain is as long as the class dim
+    float t[VW];  // this step's NC classes by fours or twos, then the steps: no chain is as long as the class dim
 #pragma unroll
-    for (int k = 0; k < VW; ++k) t[k] = HOLD ? s[k] : 0.0f;
+    for (int k = 0; k < VW; ++k) t[k] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NC; ++j)
+    for (int j = 0; j < NC; j += GRP)
       if (at.valid && c0 + j * TY < g.cols) {
 #pragma unroll
-        for (int k = 0; k < VW; ++k) t[k] += __builtin_amdgcn_exp2f((dim_elem<TI, VW>(x[j], k) - mb[k]) * kLog2e);
+        for (int k = 0; k < VW; ++k) {
+          float e[GRP];
+#pragma unroll
+          for (int i = 0; i < GRP; ++i)
+            e[i] = c0 + (j + i) * TY < g.cols
+                       ? __builtin_amdgcn_exp2f((dim_elem<TI, VW>(x[j + i], k) - mb[k]) * kLog2e)
+                       : 0.0f;
+          t[k] += dim_tree<GRP>(e);
+        }
       }
 #pragma unroll
-    for (int k = 0; k < VW; ++k) s[k] = HOLD ? t[k] : s[k] + t[k];
+    for (int k = 0; k < VW; ++k) s[k] += t[k];
     if constexpr (HOLD) break;
   }
-  dim_lse<VW, TXL>(m, s, lds);
+  if constexpr (!HOLD) {
+    float M[VW];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) M[k] = m[k];
+    dim_max<VW, TXL>(M, lds + LDS_SUM);
+#pragma unroll
+    for (int k = 0; k < VW; ++k) {
+      s[k] = lse_rescale(s[k], m[k], M[k]);
+      m[k] = M[k];
+    }
+  }
+  dim_sum<VW, TXL>(s, lds);
   if constexpr (HOLD) dim_opaque<TI, VW, NC>(x);
   // log: (x - M) - log S;  softmax: e^(x - M) / S (an all -inf column gives
   // 0 * inf = NaN, a NaN anywhere a NaN sum)
@@ -267,6 +288,7 @@ template <typename TG, typename TO, int VW, int TXL, int NC, bool HOLD, bool LOG
 __global__ void __launch_bounds__(kDimBlock)
 k_dim_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restrict__ gin, DimGeom g) {
   constexpr int TX = 1 << TXL, TY = kDimBlock / TX;
+  constexpr int GRP = LOG && VW <= 4 ? 4 : 2;  // as in the forward; products by two, the second fused
   __shared__ float lds[TX <= 64 ? (kDimBlock / 64) * TX * VW : 1];
   const DimPlace at = dim_place<VW, TXL>(g);
   const uint32_t ty = threadIdx.x >> TXL;
@@ -288,18 +310,28 @@ k_dim_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restri
     }
     float t[VW];  // as in the forward
 #pragma unroll
-    for (int k = 0; k < VW; ++k) t[k] = HOLD ? s[k] : 0.0f;
+    for (int k = 0; k < VW; ++k) t[k] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NC; ++j)
+    for (int j = 0; j < NC; j += GRP)
       if (at.valid && c0 + j * TY < g.cols) {
 #pragma unroll
         for (int k = 0; k < VW; ++k) {
-          if constexpr (LOG) t[k] += dim_elem<TG, VW>(gv[j], k);
-          else t[k] = fmaf(dim_elem<TG, VW>(gv[j], k), dim_elem<TG, VW>(yv[j], k), t[k]);
+          float e[GRP];
+#pragma unroll
+          for (int i = 0; i < GRP; ++i) {
+            e[i] = 0.0f;
+            if (c0 + (j + i) * TY < g.cols) {
+              const float gk = dim_elem<TG, VW>(gv[j + i], k);
+              if constexpr (LOG) e[i] = gk;
+              else e[i] = fmaf(gk, dim_elem<TG, VW>(yv[j + i], k), i > 0 ? e[i - 1] : 0.0f);
+              if constexpr (!LOG) if (i > 0) e[i - 1] = 0.0f;
+            }
+          }
+          t[k] += dim_tree<GRP>(e);
         }
       }
 #pragma unroll
-    for (int k = 0; k < VW; ++k) s[k] = HOLD ? t[k] : s[k] + t[k];
+    for (int k = 0; k < VW; ++k) s[k] += t[k];
     if constexpr (HOLD) break;
   }
   dim_sum<VW, TXL>(s, lds);
