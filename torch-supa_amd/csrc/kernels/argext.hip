@@ -16,8 +16,8 @@
 // two launches: the first writes one pair per chunk, the second (k_argext)
 // reduces each row's chunk pairs, reading their indices from `in_idx`.
 // Measured on MI355X, us, before (a workgroup and scalar loads for every row)
-// -> now, bf16: [131072, 50] 197 -> 9.6, [16384, 1000] 40 -> 8.8,
-// [4096, 50257] 226 -> 88; float32 [8192, 8192] 50.5 -> 40.5 (6.6 TB/s, HBM
+// -> now, bf16: [131072, 50] 196 -> 9.8, [16384, 1000] 40 -> 9.2,
+// [4096, 50257] 227 -> 89; float32 [8192, 8192] 50.5 -> 41 (6.5 TB/s, HBM
 // bound; bf16 65.6 -> 25, 5.4 TB/s, bound by the compares: six instructions an
 // element).
 //
@@ -25,8 +25,8 @@
 // reduced dim, TY threads apart where positions alone would leave the chip
 // idle; the planes are read once where a transposing copy and a workgroup per
 // position came before: classes of float32
-// [32, 19, 256, 256] 3424 us -> 29 (6.1 TB/s), of bf16 [4, 21, 513, 513]
-// 1589 -> 17.
+// [32, 19, 256, 256] 3415 us -> 30 (5.4 TB/s), of bf16 [4, 21, 513, 513]
+// 1583 -> 17.
 //
 // Replaces amax.out NF:3926, amin.out NF:4115, max.dim_max NF:3894,
 // min.dim_min NF:4091, argmax.out NF:839, argmin.out NF:852, max.unary_out

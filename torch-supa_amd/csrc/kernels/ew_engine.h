@@ -479,10 +479,10 @@ k_vecnd(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {
 // end at the run's end and stores only the elements no other vector covers
 // (so an output may still be an input).  Every access is at element
 // alignment.  Runs of odd length took one element per thread (k_strided)
-// before: [6007, 2047] + a row in float32 43.4 us, 17.0 now, in bf16 43.4, 9.6;
-// [5843, 8821] slices of odd rows in bf16: silu 173 us, 41 now, a product 173, 52.
+// before: [6007, 2047] + a row in float32 43.6 us, 17 now, in bf16 43.5, 11;
+// [5843, 8821] slices of odd rows in bf16: silu 174 us, 44 now, a product 174, 52.
 // Loads take no streaming hint: a run's ends share cache lines with its
-// neighbours (bf16 [32768, 4095] + a row 103 us, 119 with the hint).
+// neighbours (bf16 [32768, 4095] + a row 96 us, 119 with the hint).
 template <int VEC, typename OFF, typename Op, typename C, typename CT, typename OT, typename... S>
 __global__ void __launch_bounds__(kStreamBlock)
 k_vecnd_any(Op op, TArgs<1 + sizeof...(S)> a, NdGeom g, uint32_t nvec) {

@@ -19,10 +19,11 @@
 // SharedReduceOps.h) does.
 //
 // Measured on MI355X, us, before (Welford triples per thread, one element a
-// load; planes copied to rows first) -> now: float32 [8192, 4096] 28.0 -> 20.5
-// (6.5 TB/s, HBM bound), bf16 25.0 -> 13.6; [65536, 512] 40.7 -> 22.7, bf16
-// 40.2 -> 20.7; [2048, 65536] 141 -> 83; dims (0, 2) of [32, 64, 12544]
-// 73.7 -> 18.7; [64, 512, 49] 26 -> 5.
+// load; planes copied to rows first) -> now: float32 [8192, 4096] 28.2 -> 21.5
+// (6.2 TB/s, HBM bound), bf16 25.2 -> 14.7; [65536, 512] 40.8 -> 23.8, bf16
+// 40.4 -> 21; [2048, 65536] 143 -> 85; dims (0, 2) of [32, 64, 12544]
+// 74 -> 20; [64, 512, 49] 26 -> 5.8; all of 64 Mi elements 61 -> 47, bf16 55 ->
+// 27.  float64 rows stream instead (k_moments_stream).
 //
 // Replaces var.correction_out NF:6629, std.correction_out NF:6088,
 // var_mean.correction NF:6668, std_mean.correction NF:6063 (upstream
@@ -173,8 +174,8 @@ k_moments(const T* __restrict__ in, SegGeom g, FastDiv nch, A correction, int ta
 // The same in one pass, as k_moments where a row's vectors are too many
 // registers: each thread merges the triples of kMomStreamU vectors at a time
 // into its own.  float64, whose vectors hold two elements and whose deviations
-// take twice the registers: [8192, 4100] 54 us, 79.5 in register chunks;
-// [2048, 10000] 29, 43; 32 Mi elements in one row 49, 102.
+// take twice the registers: [8192, 4100] 45 us, 80 in register chunks;
+// [2048, 10000] 30, 44; [512, 8192] 5.8, 13; 32 Mi elements in one row 50, 104.
 constexpr int kMomStreamU = 4;
 template <typename T, typename A, int VW, int G, bool FINAL>
 __global__ void __launch_bounds__(kMomBlock)
@@ -265,7 +266,7 @@ k_moments_stream(const T* __restrict__ in, SegGeom g, FastDiv nch, A correction,
 
 // BS threads merge a row's chunk triples, each kMomMerge of them loaded ahead
 // of its merges: a wavefront for up to 128, else 1024 threads (the variance of
-// 64 Mi float32 elements, 8192 triples, 83.6 us with a wavefront of 128 merges
+// 64 Mi float32 elements, 8192 triples, 47 us, 84.5 with a wavefront of 128 merges
 // a lane one after another).
 constexpr int kMomMerge = 4;
 template <typename T, typename A, int BS>

@@ -153,8 +153,8 @@ k_nll_bwd(const T* __restrict__ grad_out, const int64_t* __restrict__ target, co
   T* dst = gin + row * c;
   // the row's vectors start o elements before it (unaligned.h's grid); a row's
   // first and last partial vectors go element by element (bf16 [4096, 50257]:
-  // 74 us, with the 16-byte grid 90, at element alignment 94, one element a
-  // thread 334)
+  // 75 us, with the 16-byte grid 90, at element alignment 94, one element a
+  // thread 340)
   const int o = grid_off<T, VEC>(dst, c);
 #pragma unroll
   for (int u = 0; u < kNllUnroll; ++u) {
@@ -176,8 +176,8 @@ k_nll_bwd(const T* __restrict__ grad_out, const int64_t* __restrict__ target, co
 // Rows of fewer than kNllFlat elements: vector v of the flat [n c] range, its
 // first element's row by magic division; the rows it touches are walked, a
 // row's target element written where it falls.  A 256-thread workgroup per
-// row left most threads idle there (bf16 [262144, 19] 122 us, 5.2 now;
-// [8192, 1000] 18.7 and 5.2).
+// row left most threads idle there (bf16 [262144, 19] 124 us, 8.8 now;
+// [8192, 1000] 19.3 and 9.1, a call's host time).
 constexpr int64_t kNllFlat = 2048;
 
 template <typename T, int VEC>

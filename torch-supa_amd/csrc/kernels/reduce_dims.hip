@@ -14,10 +14,10 @@
 //
 // Measured on MI355X, us, before (a copy where the reduced dims are not last,
 // then a 256-thread workgroup of scalar loads per row) -> after: sum over dim 0
-// of bf16 [8192, 4096] 57 -> 15, float32 76 -> 29, float32 [8192, 12288] 256 ->
-// 64 (6.3 TB/s), bf16 [131072, 256] 207 -> 18; over dims 0 and 2 of float32
-// [32, 64, 12544] 178 -> 18 (5.7 TB/s); over the rows of bf16 [8192, 4096] 23
-// -> 11 (6.2 TB/s), [16, 1048576] 405 -> 9, [1048576, 10] 418 -> 44.
+// of bf16 [8192, 4096] 58 -> 16, float32 76 -> 27, float32 [8192, 12288] 250 ->
+// 67 (6.0 TB/s), bf16 [131072, 256] 208 -> 17; over dims 0 and 2 of float32
+// [32, 64, 12544] 180 -> 20 (5.2 TB/s); over the rows of bf16 [8192, 4096] 23
+// -> 12 (5.7 TB/s), [16, 1048576] 408 -> 6.7, [1048576, 10] 420 -> 44.
 //
 // Replaces sum_stub / mean_stub over dims
 // (.../kernels/reduce/ReduceSumKernel.cu:102-113, ReduceMomentKernel.cu:37-55).
@@ -271,8 +271,8 @@ k_sum_segs(const T* __restrict__ in, OT* __restrict__ out, SegGeom g, ACC scale)
 
 // Chunks per row: rows too few for kDimSumBlocks workgroups are cut in chunks
 // of at least 8 vectors a thread, from 32 on (the second launch costs 2 us:
-// float32 [700, 16384], 16 vectors a thread, 7.1 us in one launch, 11.1 in two;
-// [1, 16384] 4.3, 6.7).
+// float32 [700, 16384], 16 vectors a thread, 6.3 us in one launch, 10.8 in two;
+// [1, 16384] 3.9, 6.7).
 inline int64_t seg_chunks(int64_t rows, int64_t nvec) {
   const int64_t most = nvec >= 32 * kDimSumBlock ? nvec / (8 * kDimSumBlock) : 1;
   return std::max<int64_t>(1, std::min<int64_t>(most, kDimSumBlocks / rows));
@@ -300,7 +300,7 @@ int segs_launch(const T* in, OT* out, const SegGeom& g, unsigned nch, ACC scale,
   };
   using std::integral_constant;
   // a wavefront per row up to 512 vectors where the rows alone fill the chip
-  // (bf16 [6007, 2047] 6.3 us, 11.5 with four)
+  // (bf16 [6007, 2047] 5.5 us, 11.5 with four)
   const bool wave = g.rows >= 4096 && g.nvec <= 512;
   if (nch == 1 && g.nvec <= 32) return go(integral_constant<int, 16>{});
   if (nch == 1 && wave) return go(integral_constant<int, 64>{});

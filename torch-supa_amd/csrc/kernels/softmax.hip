@@ -81,11 +81,11 @@ constexpr int kLsmGrid = 512;  // 2 workgroups per CU on MI355X's 256 CUs
 // A 1024-thread workgroup per row, as longer rows take, left most of its
 // threads without a vector here; rows of odd length took a 256-thread
 // workgroup of scalar loads and three passes.  Measured on MI355X, us before
-// -> after, forward / backward: bf16 [1048576, 10] 830 -> 40 / 449 -> 39,
-// [262144, 64] 1136 -> 20 / 674 -> 22, [65536, 1024] 292 -> 42 (6.3 TB/s) /
-// 201 -> 64 (6.3 TB/s), [32768, 1659] 105 -> 40 / 139 -> 60, [16384, 4096]
-// 89 -> 45 / 79 -> 68, [8192, 10000] 67 -> 56; float32 [65536, 1000] 289 ->
-// 96 / 268 -> 149.
+// -> after, forward / backward: bf16 [1048576, 10] 830 -> 40 / 452 -> 40,
+// [262144, 64] 1136 -> 20 / 685 -> 22, [65536, 1024] 292 -> 43 (6.2 TB/s) /
+// 204 -> 65 (6.2 TB/s), [32768, 1659] 106 -> 41 / 140 -> 61, [16384, 4096]
+// 89 -> 46 / 76 -> 70, [8192, 10000] 68 -> 57; float32 [65536, 1000] 290 ->
+// 95 / 268 -> 145.
 template <int G> constexpr int row_block() { return G <= 64 ? 256 : G; }
 
 // This thread's row and place in it; false past the last row.
@@ -263,7 +263,7 @@ k_row_bwd(const TG* __restrict__ grad, const TG* __restrict__ outp, TO* __restri
 // against 66 with 256).
 // Rows too few to fill the chip that way (256 CUs) take more threads each, so
 // that a row waits for one or two loads a thread: bf16 [512, 4096] backward
-// 11.3 us by wavefronts, 4.6 so, and forward 8.0, 5.0; [256, 8192] forward 5.5
+// 11.3 us by wavefronts, 5.1 so, and forward 8.1, 4.6; [256, 8192] forward 5.5
 // with 256 threads, 4.3 so.
 // Launches stay below HIP's 2^32 threads: more rows go in several.
 template <int V, int MAXV, bool BWD, typename F>
@@ -733,7 +733,7 @@ __device__ __forceinline__ float split_rest(const T* row, int64_t cols, int nvec
 // with zeros in the places outside.  bf16 [4096, 50257]: 233 us, on the
 // 16-byte grid 239, at element alignment 306 (the forward, 16-byte
 // grid and element alignment, 160 and 151 us;
-// aligned rows of 50304 193 and 133 us; streaming the rows twice by scalars,
+// aligned rows of 50304 200 and 135 us; streaming the rows twice by scalars,
 // as rows of odd length did before, 501 and 551 us).
 struct SplitRow {
   int o;         // elements between the line boundary and the row
