@@ -25,7 +25,7 @@
 // reduced dim, TY threads apart where positions alone would leave the chip
 // idle; the planes are read once where a transposing copy and a workgroup per
 // position came before: classes of float32
-// [32, 19, 256, 256] 3415 us -> 30 (5.4 TB/s), of bf16 [4, 21, 513, 513]
+// [32, 19, 256, 256] 3415 us -> 30 (5.9 TB/s), of bf16 [4, 21, 513, 513]
 // 1583 -> 17.
 //
 // Replaces amax.out NF:3926, amin.out NF:4115, max.dim_max NF:3894,
