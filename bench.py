@@ -597,7 +597,7 @@ def derive_traffic(fetch_csv, write_csv):
           f"Two counter runs of the bench's probe mode ({PROBE_REPS}x `abs.out` over 2^28 f32 as the calibration -- "
           f"exactly 1 GiB read and 1 GiB written per dispatch -- then {PROBE_REPS}x `gelu.out(approximate='tanh')` "
           "over the c2 f32 tensor [64,2048,4096]):", "", "```",
-          "cd /tmp && export TMPDIR=/tmp && cd $GRAFT_REPO_ROOT",
+          "cd /tmp && export TMPDIR=/tmp && cd REPOSITORY",
           "timeout -s KILL 120 rocprofv3 --pmc FETCH_SIZE --output-format csv -d {} -o {} -- python3 bench.py --probe"
           .format(*_run_args(fetch_csv, "_counter_collection.csv")),
           "timeout -s KILL 120 rocprofv3 --pmc WRITE_SIZE --output-format csv -d {} -o {} -- python3 bench.py --probe"
@@ -678,8 +678,8 @@ def render_kernel_stats(stats_csv, bench_log):
 
     by_name = {short(r["Name"]): r for r in rows}
     out = ["# Kernel statistics, every bench config (MI355X, gfx950)", "",
-           "Commands (repo root on the GPU box; the second runs on any machine):", "", "```",
-           "cd /tmp && export TMPDIR=/tmp && cd $GRAFT_REPO_ROOT",
+           "Commands (repo root on the machine with the GPU; the second runs on any machine):", "", "```",
+           "cd /tmp && export TMPDIR=/tmp && cd REPOSITORY",
            "rocprofv3 --kernel-trace --stats --output-format csv -d {} -o {} -- \\".format(
                *_run_args(stats_csv, "_kernel_stats.csv")),
            f"    python3 bench.py --no-cpu --steps 10 > {bench_log}",
@@ -932,8 +932,8 @@ def derive_counters(csvs, cfg, stats_csv=None):
     # the summary table
     lines = [f"# {cfg}: per-kernel counters (rocprofv3 on MI355X)", "", PROBE_NOTES.get(cfg, cfg) + ".", "",
              "Each dominant aten call runs 3 times after 3 calibration dispatches (`abs.out` over 2^28 f32: "
-             "1 GiB read, 1 GiB written).  Commands (from the repository root, on the GPU box):", "", "```",
-             "cd /tmp && export TMPDIR=/tmp && cd $GRAFT_REPO_ROOT",
+             "1 GiB read, 1 GiB written).  Commands (from the repository root, on the machine with the GPU):", "", "```",
+             "cd /tmp && export TMPDIR=/tmp && cd REPOSITORY",
              *cmds,
              "```", "",
              f"FETCH_SIZE scale {scale.get('FETCH_SIZE', 0):.5f}, WRITE_SIZE scale {scale.get('WRITE_SIZE', 0):.5f} "
