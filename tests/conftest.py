@@ -25,7 +25,7 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def supa():
-    """The supa backend on a GPU box; fails loudly when the build is missing."""
+    """The supa backend on a machine with a GPU; fails loudly when the build is missing."""
     import torch
     import torch_supa  # noqa: F401
 
